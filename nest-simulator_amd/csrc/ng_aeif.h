@@ -17,30 +17,70 @@
 namespace nestgpu
 {
 
+// Parameters of one neuron. FAST: the divisors lie within [1e-200, 1e200] (AEIF_FAST of the
+// parameter set), and their reciprocals are refined once per update for ng_div.
+template < bool FAST >
 struct AeifPar
 {
-  double V_peak, V_reset, g_L, C_m, E_ex, E_in, E_L, Delta_T, tau_w, a, b, V_th, tau_ex, tau_in, I_e, tol;
+  double V_peak, V_reset, g_L, C_m, E_ex, E_in, E_L, Delta_T, tau_w, a, V_th, tau_ex, tau_in, I_e, tol;
+  double gD;  // g_L Delta_T, the left factors of the spike current
+  double r_C_m, r_Delta_T, r_tau_w, r_tau_ex, r_tau_in;
+
+  // a / b: exactly, by the reciprocal where FAST
+  __device__ static double
+  div( double x, double b, double y )
+  {
+    return FAST ? ng_div( x, b, y ) : x / b;
+  }
 };
 
-__host__ __device__ inline void
-aeif_dynamics( const AeifPar& P, bool refractory, const double* y, double* f )
+// g_L Delta_T exp( ( V - V_th ) / Delta_T ) of the effective potential V
+template < bool FAST >
+__device__ inline double
+aeif_spike_current( const AeifPar< FAST >& P, double V )
 {
-  const double V = refractory ? P.V_reset : ( P.V_peak < y[ 0 ] ? P.V_peak : y[ 0 ] );  // std::min
+  const double e = P.gD * ng_exp( P.div( V - P.V_th, P.Delta_T, P.r_Delta_T ) );
+  return P.Delta_T == 0. ? 0. : e;
+}
+
+template < bool FAST >
+__device__ inline double
+aeif_V( const AeifPar< FAST >& P, bool refractory, double y0 )
+{
+  return refractory ? P.V_reset : ( P.V_peak < y0 ? P.V_peak : y0 );  // std::min
+}
+
+// the right-hand side at effective potential V (aeif_V of y[ 0 ]), its spike current given
+template < bool FAST >
+__device__ inline void
+aeif_dynamics( const AeifPar< FAST >& P, bool refractory, double V, double I_spike, const double* y, double* f )
+{
   const double g_ex = y[ 1 ];
   const double g_in = y[ 2 ];
   const double w = y[ 3 ];
   const double I_syn_exc = g_ex * ( V - P.E_ex );
   const double I_syn_inh = g_in * ( V - P.E_in );
-  const double I_spike = P.Delta_T == 0. ? 0. : ( P.g_L * P.Delta_T * ng_exp( ( V - P.V_th ) / P.Delta_T ) );
+  const double dV = V - P.E_L;
   // currents_ carries no CurrentEvents on this path: I_stim_ == 0.0
-  f[ 0 ] = refractory ? 0. : ( -P.g_L * ( V - P.E_L ) + I_spike - I_syn_exc - I_syn_inh - w + P.I_e + 0.0 ) / P.C_m;
-  f[ 1 ] = -g_ex / P.tau_ex;
-  f[ 2 ] = -g_in / P.tau_in;
-  f[ 3 ] = ( P.a * ( V - P.E_L ) - w ) / P.tau_w;
+  const double I = -P.g_L * dV + I_spike - I_syn_exc - I_syn_inh - w + P.I_e + 0.0;
+  f[ 0 ] = refractory ? 0. : P.div( I, P.C_m, P.r_C_m );
+  f[ 1 ] = P.div( -g_ex, P.tau_ex, P.r_tau_ex );
+  f[ 2 ] = P.div( -g_in, P.tau_in, P.r_tau_in );
+  f[ 3 ] = P.div( P.a * dV - w, P.tau_w, P.r_tau_w );
 }
 
-__host__ __device__ inline void
-aeif_rkf45_step( const AeifPar& P, bool refr, double* y, double h, const double* k1, double* yerr, double* dydt_out )
+template < bool FAST >
+__device__ inline void
+aeif_rhs( const AeifPar< FAST >& P, bool refractory, const double* y, double* f )
+{
+  const double V = aeif_V( P, refractory, y[ 0 ] );
+  aeif_dynamics( P, refractory, V, aeif_spike_current( P, V ), y, f );
+}
+
+template < bool FAST >
+__device__ inline void
+aeif_rkf45_step( const AeifPar< FAST >& P, bool refr, double* y, double h, const double* k1, double* yerr,
+  double* dydt_out )
 {
   const double b21 = 1.0 / 4.0;
   const double b31 = 3.0 / 32.0, b32 = 9.0 / 32.0;
@@ -55,23 +95,23 @@ aeif_rkf45_step( const AeifPar& P, bool refr, double* y, double h, const double*
 #pragma unroll
   for ( int i = 0; i < 4; ++i )
     yt[ i ] = y[ i ] + b21 * h * k1[ i ];
-  aeif_dynamics( P, refr, yt, k2 );
+  aeif_rhs( P, refr, yt, k2 );
 #pragma unroll
   for ( int i = 0; i < 4; ++i )
     yt[ i ] = y[ i ] + h * ( b31 * k1[ i ] + b32 * k2[ i ] );
-  aeif_dynamics( P, refr, yt, k3 );
+  aeif_rhs( P, refr, yt, k3 );
 #pragma unroll
   for ( int i = 0; i < 4; ++i )
     yt[ i ] = y[ i ] + h * ( b41 * k1[ i ] + b42 * k2[ i ] + b43 * k3[ i ] );
-  aeif_dynamics( P, refr, yt, k4 );
+  aeif_rhs( P, refr, yt, k4 );
 #pragma unroll
   for ( int i = 0; i < 4; ++i )
     yt[ i ] = y[ i ] + h * ( b51 * k1[ i ] + b52 * k2[ i ] + b53 * k3[ i ] + b54 * k4[ i ] );
-  aeif_dynamics( P, refr, yt, k5 );
+  aeif_rhs( P, refr, yt, k5 );
 #pragma unroll
   for ( int i = 0; i < 4; ++i )
     yt[ i ] = y[ i ] + h * ( b61 * k1[ i ] + b62 * k2[ i ] + b63 * k3[ i ] + b64 * k4[ i ] + b65 * k5[ i ] );
-  aeif_dynamics( P, refr, yt, k6 );
+  aeif_rhs( P, refr, yt, k6 );
 #pragma unroll
   for ( int i = 0; i < 4; ++i )
   {
@@ -84,11 +124,13 @@ aeif_rkf45_step( const AeifPar& P, bool refr, double* y, double h, const double*
     const double ei = ec1 * k1[ i ] + ec3 * k3[ i ] + ec4 * k4[ i ] + ec5 * k5[ i ] + ec6 * k6[ i ];
     yerr[ i ] = h * ei;
   }
-  aeif_dynamics( P, refr, y, dydt_out );
+  aeif_rhs( P, refr, y, dydt_out );
 }
 
-// returns -1 (decrease), 0 (keep), +1 (increase)
-__host__ __device__ inline int
+// y' error control of a step of size h with right-hand side yp at its end: -1 (decrease),
+// 0 (keep) or +1 (increase), and the next step size in *h. The two rules differ in exponent and
+// bounds only, so one power serves a wave whose lanes take either.
+__device__ inline int
 aeif_yp_hadjust( double tol, const double* yerr, const double* yp, double* h )
 {
   const double S = 0.9;
@@ -101,30 +143,25 @@ aeif_yp_hadjust( double tol, const double* yerr, const double* yp, double* h )
     const double r = fabs( yerr[ i ] ) / fabs( D0 );
     rmax = r > rmax ? r : rmax;
   }
-  if ( rmax > 1.1 )
+  const bool shrink = rmax > 1.1, grow = rmax < 0.5;
+  if ( not( shrink or grow ) )
+    return 0;
+  double r = S / ng_pow( rmax, shrink ? 1.0 / 5.0 : 1.0 / ( 5.0 + 1.0 ) );
+  if ( shrink )
+    r = r < 0.2 ? 0.2 : r;
+  else
   {
-    double r = S / ng_pow( rmax, 1.0 / 5.0 );
-    if ( r < 0.2 )
-      r = 0.2;
-    *h = r * h_old;
-    return -1;
+    r = r > 5.0 ? 5.0 : r;
+    r = r < 1.0 ? 1.0 : r;
   }
-  else if ( rmax < 0.5 )
-  {
-    double r = S / ng_pow( rmax, 1.0 / ( 5.0 + 1.0 ) );
-    if ( r > 5.0 )
-      r = 5.0;
-    if ( r < 1.0 )
-      r = 1.0;
-    *h = r * h_old;
-    return 1;
-  }
-  return 0;
+  *h = r * h_old;
+  return shrink ? -1 : 1;
 }
 
 // One accepted adaptive step from *t towards t1 (gsl_odeiv_evolve_apply semantics).
-__host__ __device__ inline void
-aeif_evolve( const AeifPar& P, bool refr, double* t, double t1, double* h, double* y )
+template < bool FAST >
+__device__ inline void
+aeif_evolve( const AeifPar< FAST >& P, bool refr, double* t, double t1, double* h, double* y )
 {
   const double t0 = *t;
   double h0 = *h;
@@ -133,7 +170,7 @@ aeif_evolve( const AeifPar& P, bool refr, double* t, double t1, double* h, doubl
 #pragma unroll
   for ( int i = 0; i < 4; ++i )
     y0[ i ] = y[ i ];
-  aeif_dynamics( P, refr, y, dydt_in );
+  aeif_rhs( P, refr, y, dydt_in );
   // A rejected attempt shrinks h0 by a factor of at most 0.9 * 1.1^(-1/5) < 0.89 and stops
   // once t + h0 rounds to t, so fewer than 400 attempts can occur; the bound only makes the
   // loop's exit evident.

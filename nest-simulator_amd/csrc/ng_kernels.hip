@@ -62,6 +62,9 @@ template < class T >
 using gptr = __attribute__( ( address_space( 1 ) ) ) T*;
 template < class T >
 using gref = __attribute__( ( address_space( 1 ) ) ) T&;
+// memory that no kernel writes while this one runs: uniform addresses load into scalar registers
+template < class T >
+using cptr = __attribute__( ( address_space( 4 ) ) ) T*;
 template < class T >
 using lptr = __attribute__( ( address_space( 3 ) ) ) T*;
 template < class T >
@@ -69,6 +72,17 @@ __device__ inline gptr< T >
 glob( T* p )
 {
   return ( gptr< T > )p;
+}
+
+// x of the first active lane, in scalar registers
+__device__ inline double
+wave_uniform( double x )
+{
+  uint64_t b = __builtin_bit_cast( uint64_t, x );
+  const uint32_t lo = __builtin_amdgcn_readfirstlane( static_cast< uint32_t >( b ) );
+  const uint32_t hi = __builtin_amdgcn_readfirstlane( static_cast< uint32_t >( b >> 32 ) );
+  b = ( static_cast< uint64_t >( hi ) << 32 ) | lo;
+  return __builtin_bit_cast( double, b );
 }
 
 // device-scope relaxed atomics on HBM counters (what atomicAdd / atomicOr do, without FLAT)

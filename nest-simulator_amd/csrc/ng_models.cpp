@@ -594,6 +594,12 @@ public:
       p.V_th, p.tau_ex, p.tau_in, p.I_e, p.tol, p.Delta_T > 0. ? p.V_peak : p.V_th, h };
     for ( int q = 0; q < 18; ++q )
       ps.p[ q ] = vals[ q ];
+    // whether divisions by the constants may go through their reciprocals (ng_div)
+    auto in_range = []( double x ) { return x >= 1e-200 and x <= 1e200; };
+    ps.p[ 18 ] = ( p.Delta_T == 0.0 or in_range( p.Delta_T ) ) and in_range( p.c_m ) and in_range( p.tau_w )
+        and in_range( p.tau_ex ) and in_range( p.tau_in )
+      ? 1.0
+      : 0.0;
   }
   void
   device_state( const NeuronParams&, const NeuronState& s, double h, double out[ 5 ] ) const override

@@ -210,8 +210,23 @@ struct DeviceNode< M_AEIF_COND_EXP >
   update( const NetDev& d, gref< const ParamSet > ps, uint32_t dev, uint32_t local, const Cells< WIN >& C,
     const SlicePhase& ph, uint64_t* bits, uint32_t mcol, int next_sample )
   {
+    // A wave whose neurons share one parameter set (a population with common parameters) reads
+    // it into scalar registers and divides by its constants through their reciprocals; other
+    // waves keep per-lane parameters and plain divisions.
+    const uint32_t pi = glob( d.pidx )[ dev ];
+    const uint32_t p0 = __builtin_amdgcn_readfirstlane( pi );
+    if ( __ballot( pi != p0 ) == 0 and glob( d.psets )[ p0 ].p[ 18 ] != 0.0 )
+      integrate< WIN, true >( d, ( (cptr< const ParamSet >)d.psets )[ p0 ], dev, local, C, ph, bits, mcol, next_sample );
+    else
+      integrate< WIN, false >( d, ps, dev, local, C, ph, bits, mcol, next_sample );
+  }
+  template < bool WIN, bool FAST, class PS >
+  __device__ __forceinline__ static void
+  integrate( const NetDev& d, PS& ps, uint32_t dev, uint32_t local, const Cells< WIN >& C,
+    const SlicePhase& ph, uint64_t* bits, uint32_t mcol, int next_sample )
+  {
     // models/aeif_cond_exp.cpp:443-523
-    AeifPar A;
+    AeifPar< FAST > A;
     A.V_peak = ps.p[ 0 ];
     A.V_reset = ps.p[ 1 ];
     A.g_L = ps.p[ 2 ];
@@ -222,12 +237,21 @@ struct DeviceNode< M_AEIF_COND_EXP >
     A.Delta_T = ps.p[ 7 ];
     A.tau_w = ps.p[ 8 ];
     A.a = ps.p[ 9 ];
-    A.b = ps.p[ 10 ];
     A.V_th = ps.p[ 11 ];
     A.tau_ex = ps.p[ 12 ];
     A.tau_in = ps.p[ 13 ];
     A.I_e = ps.p[ 14 ];
     A.tol = ps.p[ 15 ];
+    A.gD = A.g_L * A.Delta_T;
+    if ( FAST )
+    {
+      A.r_C_m = wave_uniform( ng_recip( A.C_m ) );
+      A.r_Delta_T = wave_uniform( ng_recip( A.Delta_T ) );
+      A.r_tau_w = wave_uniform( ng_recip( A.tau_w ) );
+      A.r_tau_ex = wave_uniform( ng_recip( A.tau_ex ) );
+      A.r_tau_in = wave_uniform( ng_recip( A.tau_in ) );
+    }
+    const double b_adapt = ps.p[ 10 ];
     const double V_peak_eff = ps.p[ 16 ];
     const double hstep = ps.p[ 17 ];
     double y[ 4 ] = { glob( d.v[ 0 ] )[ dev ], glob( d.v[ 1 ] )[ dev ], glob( d.v[ 2 ] )[ dev ],
@@ -265,7 +289,7 @@ struct DeviceNode< M_AEIF_COND_EXP >
         else if ( y[ 0 ] >= V_peak_eff )
         {
           y[ 0 ] = A.V_reset;
-          y[ 3 ] += A.b;
+          y[ 3 ] += b_adapt;
           r = ps.refractory_counts > 0 ? ps.refractory_counts + 1 : 0;
           const uint64_t bit = 1ull << ( lag & 63 );
           uint64_t had = 0;
