@@ -1,4 +1,4 @@
-// ng_aeif.h -- per-neuron adaptive Runge-Kutta-Fehlberg 4(5) for aeif_cond_exp.
+// ng_aeif.h -- adaptive Runge-Kutta-Fehlberg 4(5) for aeif_cond_exp, four lanes per neuron.
 //
 // Stands in for the GSL stepper NEST uses (models/aeif_cond_exp.cpp:386,395,463:
 // gsl_odeiv_step_rkf45, gsl_odeiv_control_yp_new(tol, tol), gsl_odeiv_evolve_apply).
@@ -10,6 +10,15 @@
 //   * evolve: one accepted step towards t1 per call, clipped to t1, retried from the saved
 //     state when the controller shrinks h and the shrink moves t by at least one ulp.
 // The right-hand side follows aeif_cond_exp_dynamics (models/aeif_cond_exp.cpp:79-124).
+//
+// Lane c of a neuron's quad of lanes holds component c of the state (V_m, g_ex, g_in, w). The
+// stage sums, the error and the final division of each component's derivative are then the
+// same instructions in all four lanes, done once instead of four times; the spike current is
+// computed in all four; components meet through quad permutes. A neuron's steps are a serial
+// chain and the slowest neuron of a network (up to 166 attempted steps in a slice of 15 steps,
+// where the mean is 16) decides how long a slice takes, so the chain's length is what counts:
+// an attempt takes about 700 instructions per lane instead of 1,300, and its registers fit
+// without spilling.
 #pragma once
 
 #include "ng_math.h"
@@ -17,16 +26,42 @@
 namespace nestgpu
 {
 
-// Parameters of one neuron. FAST: the divisors lie within [1e-200, 1e200] (AEIF_FAST of the
-// parameter set), and their reciprocals are refined once per update for ng_div.
-template < bool FAST >
-struct AeifPar
+// x of lane J of the lane's quad / of the lane with quad index c ^ X
+template < int CTRL >
+__device__ __forceinline__ double
+quad_perm( double x )
 {
-  double V_peak, V_reset, g_L, C_m, E_ex, E_in, E_L, Delta_T, tau_w, a, V_th, tau_ex, tau_in, I_e, tol;
-  double gD;  // g_L Delta_T, the left factors of the spike current
-  double r_C_m, r_Delta_T, r_tau_w, r_tau_ex, r_tau_in;
+  const uint64_t b = __builtin_bit_cast( uint64_t, x );
+  const uint32_t lo = static_cast< uint32_t >(
+    __builtin_amdgcn_update_dpp( 0, static_cast< int >( b ), CTRL, 0xf, 0xf, true ) );
+  const uint32_t hi = static_cast< uint32_t >(
+    __builtin_amdgcn_update_dpp( 0, static_cast< int >( b >> 32 ), CTRL, 0xf, 0xf, true ) );
+  return __builtin_bit_cast( double, ( static_cast< uint64_t >( hi ) << 32 ) | lo );
+}
+template < int J >
+__device__ __forceinline__ double
+quad_bcast( double x )
+{
+  return quad_perm< J * 0x55 >( x );
+}
+template < int J >
+__device__ __forceinline__ uint32_t
+quad_bcast( uint32_t x )
+{
+  return static_cast< uint32_t >(
+    __builtin_amdgcn_update_dpp( 0, static_cast< int >( x ), J * 0x55, 0xf, 0xf, true ) );
+}
 
-  // a / b: exactly, by the reciprocal where FAST
+// Parameters in one lane. E, m, den: the lane's reversal potential (E_L, E_ex, E_in, E_L),
+// its multiplier of V - E (-g_L and a in lanes 0 and 3; lanes 1 and 2 use their conductance)
+// and its divisor (C_m, tau_ex, tau_in, tau_w); r_*: refined reciprocals (ng_recip). FAST:
+// every divisor of the network lies within [1e-200, 1e200]; otherwise divisions are plain.
+template < bool FAST >
+struct AeifLane
+{
+  int c;
+  double V_peak, V_reset, V_th, Delta_T, gD, I_e, tol;
+  double E, m, den, r_den, r_Delta_T;
   __device__ static double
   div( double x, double b, double y )
   {
@@ -36,51 +71,55 @@ struct AeifPar
 
 // g_L Delta_T exp( ( V - V_th ) / Delta_T ) of the effective potential V
 template < bool FAST >
-__device__ inline double
-aeif_spike_current( const AeifPar< FAST >& P, double V )
+__device__ __forceinline__ double
+aeif_spike_current( const AeifLane< FAST >& P, double V )
 {
   const double e = P.gD * ng_exp( P.div( V - P.V_th, P.Delta_T, P.r_Delta_T ) );
   return P.Delta_T == 0. ? 0. : e;
 }
 
 template < bool FAST >
-__device__ inline double
-aeif_V( const AeifPar< FAST >& P, bool refractory, double y0 )
+__device__ __forceinline__ double
+aeif_V( const AeifLane< FAST >& P, bool refractory, double V )
 {
-  return refractory ? P.V_reset : ( P.V_peak < y0 ? P.V_peak : y0 );  // std::min
+  return refractory ? P.V_reset : ( P.V_peak < V ? P.V_peak : V );  // std::min
 }
 
-// the right-hand side at effective potential V (aeif_V of y[ 0 ]), its spike current given
+// The lane's component of the right-hand side at effective potential V with spike current
+// I_spike; y: the lane's component of the state
 template < bool FAST >
-__device__ inline void
-aeif_dynamics( const AeifPar< FAST >& P, bool refractory, double V, double I_spike, const double* y, double* f )
+__device__ __forceinline__ double
+aeif_dynamics( const AeifLane< FAST >& P, bool refractory, double V, double I_spike, double y )
 {
-  const double g_ex = y[ 1 ];
-  const double g_in = y[ 2 ];
-  const double w = y[ 3 ];
-  const double I_syn_exc = g_ex * ( V - P.E_ex );
-  const double I_syn_inh = g_in * ( V - P.E_in );
-  const double dV = V - P.E_L;
+  const double p = ( P.c == 1 or P.c == 2 ? y : P.m ) * ( V - P.E );
+  const double I_syn_exc = quad_bcast< 1 >( p );
+  const double I_syn_inh = quad_bcast< 2 >( p );
+  const double w = quad_bcast< 3 >( y );
   // currents_ carries no CurrentEvents on this path: I_stim_ == 0.0
-  const double I = -P.g_L * dV + I_spike - I_syn_exc - I_syn_inh - w + P.I_e + 0.0;
-  f[ 0 ] = refractory ? 0. : P.div( I, P.C_m, P.r_C_m );
-  f[ 1 ] = P.div( -g_ex, P.tau_ex, P.r_tau_ex );
-  f[ 2 ] = P.div( -g_in, P.tau_in, P.r_tau_in );
-  f[ 3 ] = P.div( P.a * dV - w, P.tau_w, P.r_tau_w );
+  double I = p + I_spike - I_syn_exc - I_syn_inh - w + P.I_e + 0.0;
+  // only lane 0 uses it: without this the compiler moves the sum and the spike current into a
+  // branch of that lane, whose masks and jumps lengthen the chain of every stage
+  asm( "" : "+v"( I ) );
+  const double num = P.c == 0 ? I : P.c == 3 ? p - y : -y;
+  const double f = P.div( num, P.den, P.r_den );
+  return refractory and P.c == 0 ? 0. : f;
 }
 
+// the same at state component y, evaluating the spike current; it is returned in I_spike
 template < bool FAST >
-__device__ inline void
-aeif_rhs( const AeifPar< FAST >& P, bool refractory, const double* y, double* f )
+__device__ __forceinline__ double
+aeif_rhs( const AeifLane< FAST >& P, bool refractory, double y, double& I_spike )
 {
-  const double V = aeif_V( P, refractory, y[ 0 ] );
-  aeif_dynamics( P, refractory, V, aeif_spike_current( P, V ), y, f );
+  const double V = aeif_V( P, refractory, quad_bcast< 0 >( y ) );
+  I_spike = aeif_spike_current( P, V );
+  return aeif_dynamics( P, refractory, V, I_spike, y );
 }
 
+// One attempted step of size h from component y with derivative k1: the lane's component at
+// its end, the error of the embedded 4th-order solution and the derivative at the end.
 template < bool FAST >
-__device__ inline void
-aeif_rkf45_step( const AeifPar< FAST >& P, bool refr, double* y, double h, const double* k1, double* yerr,
-  double* dydt_out )
+__device__ __forceinline__ double
+aeif_rkf45_step( const AeifLane< FAST >& P, bool refr, double y, double h, double k1, double& yerr, double& yp, double& I_spike )
 {
   const double b21 = 1.0 / 4.0;
   const double b31 = 3.0 / 32.0, b32 = 9.0 / 32.0;
@@ -91,58 +130,32 @@ aeif_rkf45_step( const AeifPar< FAST >& P, bool refr, double* y, double h, const
   const double c1 = 902880.0 / 7618050.0, c3 = 3953664.0 / 7618050.0, c4 = 3855735.0 / 7618050.0,
                c5 = -1371249.0 / 7618050.0, c6 = 277020.0 / 7618050.0;
   const double ec1 = 1.0 / 360.0, ec3 = -128.0 / 4275.0, ec4 = -2197.0 / 75240.0, ec5 = 1.0 / 50.0, ec6 = 2.0 / 55.0;
-  double k2[ 4 ], k3[ 4 ], k4[ 4 ], k5[ 4 ], k6[ 4 ], yt[ 4 ];
-#pragma unroll
-  for ( int i = 0; i < 4; ++i )
-    yt[ i ] = y[ i ] + b21 * h * k1[ i ];
-  aeif_rhs( P, refr, yt, k2 );
-#pragma unroll
-  for ( int i = 0; i < 4; ++i )
-    yt[ i ] = y[ i ] + h * ( b31 * k1[ i ] + b32 * k2[ i ] );
-  aeif_rhs( P, refr, yt, k3 );
-#pragma unroll
-  for ( int i = 0; i < 4; ++i )
-    yt[ i ] = y[ i ] + h * ( b41 * k1[ i ] + b42 * k2[ i ] + b43 * k3[ i ] );
-  aeif_rhs( P, refr, yt, k4 );
-#pragma unroll
-  for ( int i = 0; i < 4; ++i )
-    yt[ i ] = y[ i ] + h * ( b51 * k1[ i ] + b52 * k2[ i ] + b53 * k3[ i ] + b54 * k4[ i ] );
-  aeif_rhs( P, refr, yt, k5 );
-#pragma unroll
-  for ( int i = 0; i < 4; ++i )
-    yt[ i ] = y[ i ] + h * ( b61 * k1[ i ] + b62 * k2[ i ] + b63 * k3[ i ] + b64 * k4[ i ] + b65 * k5[ i ] );
-  aeif_rhs( P, refr, yt, k6 );
-#pragma unroll
-  for ( int i = 0; i < 4; ++i )
-  {
-    const double di = c1 * k1[ i ] + c3 * k3[ i ] + c4 * k4[ i ] + c5 * k5[ i ] + c6 * k6[ i ];
-    y[ i ] = y[ i ] + h * di;
-  }
-#pragma unroll
-  for ( int i = 0; i < 4; ++i )
-  {
-    const double ei = ec1 * k1[ i ] + ec3 * k3[ i ] + ec4 * k4[ i ] + ec5 * k5[ i ] + ec6 * k6[ i ];
-    yerr[ i ] = h * ei;
-  }
-  aeif_rhs( P, refr, y, dydt_out );
+  double I;
+  const double k2 = aeif_rhs( P, refr, y + b21 * h * k1, I );
+  const double k3 = aeif_rhs( P, refr, y + h * ( b31 * k1 + b32 * k2 ), I );
+  const double k4 = aeif_rhs( P, refr, y + h * ( b41 * k1 + b42 * k2 + b43 * k3 ), I );
+  const double k5 = aeif_rhs( P, refr, y + h * ( b51 * k1 + b52 * k2 + b53 * k3 + b54 * k4 ), I );
+  const double k6 = aeif_rhs( P, refr, y + h * ( b61 * k1 + b62 * k2 + b63 * k3 + b64 * k4 + b65 * k5 ), I );
+  const double y1 = y + h * ( c1 * k1 + c3 * k3 + c4 * k4 + c5 * k5 + c6 * k6 );
+  yerr = h * ( ec1 * k1 + ec3 * k3 + ec4 * k4 + ec5 * k5 + ec6 * k6 );
+  yp = aeif_rhs( P, refr, y1, I_spike );
+  return y1;
 }
 
-// y' error control of a step of size h with right-hand side yp at its end: -1 (decrease),
-// 0 (keep) or +1 (increase), and the next step size in *h. The two rules differ in exponent and
-// bounds only, so one power serves a wave whose lanes take either.
-__device__ inline int
-aeif_yp_hadjust( double tol, const double* yerr, const double* yp, double* h )
+// y' error control of a step of size h with derivative yp at its end: -1 (decrease), 0 (keep)
+// or +1 (increase), and the next step size in *h. The two rules differ in exponent and bounds
+// only, so one power serves a wave whose lanes take either.
+__device__ __forceinline__ int
+aeif_yp_hadjust( double tol, double yerr, double yp, double* h )
 {
   const double S = 0.9;
   const double h_old = *h;
-  double rmax = 2.2250738585072014e-308;  // DBL_MIN
-#pragma unroll
-  for ( int i = 0; i < 4; ++i )
-  {
-    const double D0 = tol * ( 0.0 * fabs( 0.0 ) + 1.0 * fabs( h_old * yp[ i ] ) ) + tol;
-    const double r = fabs( yerr[ i ] ) / fabs( D0 );
-    rmax = r > rmax ? r : rmax;
-  }
+  const double D0 = tol * ( 0.0 * fabs( 0.0 ) + 1.0 * fabs( h_old * yp ) ) + tol;
+  double rmax = fabs( yerr ) / fabs( D0 );
+  // the largest over the components and DBL_MIN; a NaN is passed over, as r > rmax does
+  rmax = fmax( rmax, quad_perm< 0xB1 >( rmax ) );
+  rmax = fmax( rmax, quad_perm< 0x4E >( rmax ) );
+  rmax = fmax( 2.2250738585072014e-308, rmax );
   const bool shrink = rmax > 1.1, grow = rmax < 0.5;
   if ( not( shrink or grow ) )
     return 0;
@@ -156,52 +169,6 @@ aeif_yp_hadjust( double tol, const double* yerr, const double* yp, double* h )
   }
   *h = r * h_old;
   return shrink ? -1 : 1;
-}
-
-// One accepted adaptive step from *t towards t1 (gsl_odeiv_evolve_apply semantics).
-template < bool FAST >
-__device__ inline void
-aeif_evolve( const AeifPar< FAST >& P, bool refr, double* t, double t1, double* h, double* y )
-{
-  const double t0 = *t;
-  double h0 = *h;
-  const double dt = t1 - t0;
-  double y0[ 4 ], dydt_in[ 4 ], yerr[ 4 ], dydt_out[ 4 ];
-#pragma unroll
-  for ( int i = 0; i < 4; ++i )
-    y0[ i ] = y[ i ];
-  aeif_rhs( P, refr, y, dydt_in );
-  // A rejected attempt shrinks h0 by a factor of at most 0.9 * 1.1^(-1/5) < 0.89 and stops
-  // once t + h0 rounds to t, so fewer than 400 attempts can occur; the bound only makes the
-  // loop's exit evident.
-  for ( int attempt = 0; attempt < 10000; ++attempt )
-  {
-    bool final_step = false;
-    if ( h0 > dt )
-    {
-      h0 = dt;
-      final_step = true;
-    }
-    aeif_rkf45_step( P, refr, y, h0, dydt_in, yerr, dydt_out );
-    *t = final_step ? t1 : t0 + h0;
-    const double h_old = h0;
-    const int st = aeif_yp_hadjust( P.tol, yerr, dydt_out, &h0 );
-    if ( st < 0 )
-    {
-      const double t_curr = *t;
-      const double t_next = ( *t ) + h0;
-      if ( fabs( h0 ) < fabs( h_old ) and t_next != t_curr )
-      {
-#pragma unroll
-        for ( int i = 0; i < 4; ++i )
-          y[ i ] = y0[ i ];
-        continue;
-      }
-      h0 = h_old;
-    }
-    break;
-  }
-  *h = h0;
 }
 
 }  // namespace nestgpu

@@ -126,6 +126,7 @@ struct NetDev
   int32_t min_delay, max_delay, L;  // steps; ring length L = min + max
   int32_t n_vp;
   int32_t uniform_model;  // model id when all neurons share one, else -1
+  int32_t plain_div;      // 1: some aeif_cond_exp neuron's divisors rule out ng_div
   uint32_t spk_cap;       // per-block spike list capacity (tb * min_delay)
   int32_t nch;            // ring-buffer channels per slot: 1 (iaf_psc_delta only) or 2
   int32_t win;            // 1: ring slots [wa, wa + wn) of the slice are staged in LDS

@@ -140,8 +140,13 @@ Engine::build_layout( const BuildSpec& b, bool keep_state, bool relayout )
   net_.ws = b.ws;
   net_.log_enabled = b.log_enabled ? 1 : 0;
   mask_ = 0;
+  net_.plain_div = 0;
   for ( const auto& ps : b.psets )
+  {
     mask_ |= 1 << ps.model;
+    if ( ps.model == M_AEIF_COND_EXP and ps.p[ 18 ] == 0.0 )
+      net_.plain_div = 1;
+  }
   if ( not b.stdp_prm.empty() )
     mask_ |= MASK_STDP;  // the launch needs the stdp_synapse instantiation of the slice kernel
   // ---- store and inputs (replaced on every build)

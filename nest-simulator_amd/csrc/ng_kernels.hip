@@ -62,9 +62,6 @@ template < class T >
 using gptr = __attribute__( ( address_space( 1 ) ) ) T*;
 template < class T >
 using gref = __attribute__( ( address_space( 1 ) ) ) T&;
-// memory that no kernel writes while this one runs: uniform addresses load into scalar registers
-template < class T >
-using cptr = __attribute__( ( address_space( 4 ) ) ) T*;
 template < class T >
 using lptr = __attribute__( ( address_space( 3 ) ) ) T*;
 template < class T >
@@ -72,17 +69,6 @@ __device__ inline gptr< T >
 glob( T* p )
 {
   return ( gptr< T > )p;
-}
-
-// x of the first active lane, in scalar registers
-__device__ inline double
-wave_uniform( double x )
-{
-  uint64_t b = __builtin_bit_cast( uint64_t, x );
-  const uint32_t lo = __builtin_amdgcn_readfirstlane( static_cast< uint32_t >( b ) );
-  const uint32_t hi = __builtin_amdgcn_readfirstlane( static_cast< uint32_t >( b >> 32 ) );
-  b = ( static_cast< uint64_t >( hi ) << 32 ) | lo;
-  return __builtin_bit_cast( double, b );
 }
 
 // device-scope relaxed atomics on HBM counters (what atomicAdd / atomicOr do, without FLAT)
@@ -133,18 +119,27 @@ struct SliceLds
 {
   using T = Tile< WIN >;
   double win[ T::WINDOW ];  // ring-buffer window [slot - origin][channel][tb]
-  double bw[ T::R ];        // event values, bucketed by target
   unsigned long long log_base;
-  uint32_t pref[ T::PMAX + 1 ];  // prefix of per-block spike counts
-  uint32_t c_g0[ T::CH ];        // first synapse of each chunk spike's run
-  uint32_t c_off[ T::CH + 1 ];   // exclusive prefix of run lengths
-  uint32_t bk[ T::R ];           // event keys (slot-channel << 11 | round index), bucketed by target
-  uint16_t perm[ T::R ];         // bucket position of the event at each sorted position
-  uint32_t bcnt[ 2 ][ T::BS ];   // events per target, alternating between rounds
-  uint32_t bst[ T::BS + 1 ];     // bucket starts
   uint32_t sh[ T::BS / 64 ];
   uint32_t cnt_base;
-  uint8_t c_lag[ T::CH ];
+  uint32_t pool_next;  // next neuron of the block-wide update
+  union
+  {
+    struct  // delivery
+    {
+      double bw[ T::R ];             // event values, bucketed by target
+      uint32_t pref[ T::PMAX + 1 ];  // prefix of per-block spike counts
+      uint32_t c_g0[ T::CH ];        // first synapse of each chunk spike's run
+      uint32_t c_off[ T::CH + 1 ];   // exclusive prefix of run lengths
+      uint32_t bk[ T::R ];           // event keys (slot-channel << 11 | round index), bucketed by target
+      uint16_t perm[ T::R ];         // bucket position of the event at each sorted position
+      uint32_t bcnt[ 2 ][ T::BS ];   // events per target, alternating between rounds
+      uint32_t bst[ T::BS + 1 ];     // bucket starts
+      uint8_t c_lag[ T::CH ];
+    };
+    // update: spike bits of the neurons a block-wide update integrates, 64 lags per word
+    unsigned long long spk_bits[ MAX_TB * 4 ];
+  };
 };
 
 // XCD-aware block mapping: workgroups are dispatched round-robin over 8 XCDs; give each
@@ -438,6 +433,19 @@ store_sample( const NetDev& d, uint32_t col, int64_t stamp, double f0, double f1
   p[ 1 ] = f1;
   p[ 2 ] = f2;
   p[ 3 ] = f3;
+}
+
+// One of the four fields of such a sample.
+__device__ inline void
+store_sample_field( const NetDev& d, uint32_t col, int64_t stamp, int field, double f )
+{
+  const int64_t row = ( stamp - d.mm_off ) / d.mm_int - d.mm_row0;
+  if ( row < 0 or row >= static_cast< int64_t >( d.mm_rows ) )
+  {
+    g_or( &d.counters[ 0 ], ERR_SAMPLES );
+    return;
+  }
+  glob( d.mm_buf )[ ( static_cast< size_t >( row ) * d.mm_cols + col ) * 4 + field ] = f;
 }
 
 }  // namespace nestgpu
@@ -1077,6 +1085,8 @@ __global__ void __launch_bounds__( Tile< WIN >::BS, ( MASK & WIDE_MODELS ) ? 1 :
     if ( d.rx and t < nb and rxc )
       glob( d.rx )[ dev0 + t ] += rxc;
   }
+  if ( t == 0 )
+    S.pool_next = BS / 4;
   __syncthreads();  // window staged and delivered
   if ( ptime and t == 0 )
     tp1 = wall_clock64();
@@ -1114,6 +1124,26 @@ __global__ void __launch_bounds__( Tile< WIN >::BS, ( MASK & WIDE_MODELS ) ? 1 :
 #undef NG_UPDATE
     if ( G == 0 )
       drive_adds( d, ps, m, dev, local, C, ph.origin, ph.from, 1, ph.to );
+  }
+  if constexpr ( ( MASK & BLOCK_MODELS ) != 0 )
+  {
+    // the neurons of the model that the workgroup updates together
+    using Node = DeviceNode< M_AEIF_COND_EXP >;
+    constexpr bool SINGLE = single_model< MASK >() >= 0;
+    const lptr< uint32_t > next = ( lptr< uint32_t > )&S.pool_next;
+    const lptr< unsigned long long > spk = ( lptr< unsigned long long > )S.spk_bits;
+    if ( d.plain_div )
+      Node::template update_block< WIN, SINGLE, false >( d, dev0, nb, C, ph, next, spk );
+    else
+      Node::template update_block< WIN, SINGLE, true >( d, dev0, nb, C, ph, next, spk );
+    __syncthreads();
+    if ( local < nb and ( single_model< MASK >() >= 0 or glob( d.model )[ dev ] == M_AEIF_COND_EXP ) )
+    {
+      const uint32_t nw = ( static_cast< uint32_t >( d.min_delay ) + 63u ) >> 6;
+#pragma unroll
+      for ( uint32_t w = 0; w < 4; ++w )
+        bits[ w ] = w < nw ? S.spk_bits[ local * nw + w ] : 0ull;
+    }
   }
   if ( STDP and d.stdp and local < nb )
     stdp_spikes( d, dev, ph.origin, static_cast< uint32_t >( ph.parity ), bits );

@@ -53,7 +53,7 @@ ng_exp( double x )
   // out-of-range arguments are selected at the end (NaN propagates through the sums)
   const bool over = x > 709.782712893383973096, under = x < -745.13321910194110842;
   const double kd = floor( x * invln2 + 0.5 );
-  const int k = over or under or x != x ? 0 : static_cast< int >( kd );
+  const int k = static_cast< int >( fmax( fmin( kd, 5000.0 ), -5000.0 ) );
   const double hi = x - kd * ln2hi;
   const double lo = kd * ln2lo;
   const double rr = hi - lo;
@@ -61,7 +61,8 @@ ng_exp( double x )
   const double c = rr - t * ( P1 + t * ( P2 + t * ( P3 + t * ( P4 + t * P5 ) ) ) );
   // 2 - c lies in [1.6, 2.4] for every argument in range
   const double y = 1.0 - ( ( lo - ng_div( rr * c, 2.0 - c, ng_recip( 2.0 - c ) ) ) - hi );
-  return over ? INFINITY : under ? 0.0 : ldexp( y, k );
+  const double r = under ? 0.0 : ldexp( y, k );
+  return over ? INFINITY : r;
 }
 
 __host__ __device__ inline double

@@ -23,7 +23,8 @@ struct DeviceNode;
 // The device model ids, in the order ModelManager registers them: a model with a DeviceNode
 // specialization joins the slice kernel by its entry here. WIDE marks models whose launches
 // run one workgroup per CU with up to 256 VGPRs; the others are held to 128 VGPRs, so that
-// two workgroups share a CU, spilling what does not fit.
+// two workgroups share a CU, spilling what does not fit. BLOCK marks models whose neurons are
+// updated by all threads of the workgroup together (update_block) instead of one thread each.
 #define NG_DEVICE_MODELS( X ) X( M_IAF_PSC_DELTA ) X( M_IAF_PSC_EXP ) X( M_AEIF_COND_EXP ) X( M_IAF_PSC_ALPHA )
 constexpr int N_DEVICE_MODELS = 4;
 constexpr int ALL_MODELS = ( 1 << N_DEVICE_MODELS ) - 1;
@@ -41,6 +42,7 @@ template <>
 struct DeviceNode< M_IAF_PSC_DELTA >
 {
   static constexpr bool WIDE = false;
+  static constexpr bool BLOCK = false;
   // iaf_psc_delta::handle( SpikeEvent& ) (iaf_psc_delta.cpp:332-341): one channel, the weight
   __device__ __forceinline__ static void
   receive( double w, uint32_t& ch, double& v )
@@ -116,6 +118,7 @@ template <>
 struct DeviceNode< M_IAF_PSC_EXP >
 {
   static constexpr bool WIDE = false;
+  static constexpr bool BLOCK = false;
   // iaf_psc_exp::handle( SpikeEvent& ) (iaf_psc_exp.cpp:351-362): positive weights to the
   // excitatory channel (1), others to the inhibitory one (0), signed
   __device__ __forceinline__ static void
@@ -185,10 +188,8 @@ struct DeviceNode< M_IAF_PSC_EXP >
 template <>
 struct DeviceNode< M_AEIF_COND_EXP >
 {
-  // The RKF45 stepper's state and coefficients want about 220 VGPRs. Held to 128 it spills
-  // about 95 of them to scratch, and two workgroups per CU still run the batched sweep (half
-  // its instances aeif_cond_exp) 37 % faster than one workgroup without spills.
   static constexpr bool WIDE = false;
+  static constexpr bool BLOCK = true;
   // aeif_cond_exp::handle( SpikeEvent& ) (aeif_cond_exp.cpp:526-541): positive weights to the
   // excitatory conductance (0), others negated to the inhibitory one (1)
   __device__ __forceinline__ static void
@@ -205,127 +206,191 @@ struct DeviceNode< M_AEIF_COND_EXP >
       v = -w;
     }
   }
-  template < bool WIN >
+  // Updates the block's aeif_cond_exp neurons with every thread of the workgroup, four lanes
+  // per neuron (ng_aeif.h). Neurons need very different numbers of steps (a slice of 15 steps
+  // takes 16 attempted steps on average and up to 166), so a quad that finishes its neuron
+  // takes the next one of the block from the counter *next (which starts at the number of
+  // quads) instead of waiting for the slowest lane of its wave. spk: spike bits of every
+  // neuron, [local][words of 64 lags]. Which quad integrates a neuron does not change its
+  // operations. Measured on the MI355X: 6,000 neurons, slices of 15 steps, 32 per block: AEIF_T1;
+  // the mixed sweep of 48 networks, 512 per block: AEIF_T2.
+  template < bool WIN, bool SINGLE, bool FAST >
   __device__ __forceinline__ static void
-  update( const NetDev& d, gref< const ParamSet > ps, uint32_t dev, uint32_t local, const Cells< WIN >& C,
-    const SlicePhase& ph, uint64_t* bits, uint32_t mcol, int next_sample )
-  {
-    // A wave whose neurons share one parameter set (a population with common parameters) reads
-    // it into scalar registers and divides by its constants through their reciprocals; other
-    // waves keep per-lane parameters and plain divisions.
-    const uint32_t pi = glob( d.pidx )[ dev ];
-    const uint32_t p0 = __builtin_amdgcn_readfirstlane( pi );
-    if ( __ballot( pi != p0 ) == 0 and glob( d.psets )[ p0 ].p[ 18 ] != 0.0 )
-      integrate< WIN, true >( d, ( (cptr< const ParamSet >)d.psets )[ p0 ], dev, local, C, ph, bits, mcol, next_sample );
-    else
-      integrate< WIN, false >( d, ps, dev, local, C, ph, bits, mcol, next_sample );
-  }
-  template < bool WIN, bool FAST, class PS >
-  __device__ __forceinline__ static void
-  integrate( const NetDev& d, PS& ps, uint32_t dev, uint32_t local, const Cells< WIN >& C,
-    const SlicePhase& ph, uint64_t* bits, uint32_t mcol, int next_sample )
+  update_block( const NetDev& d, uint32_t dev0, uint32_t nb, const Cells< WIN >& C, const SlicePhase& ph,
+    lptr< uint32_t > next, lptr< unsigned long long > spk )
   {
     // models/aeif_cond_exp.cpp:443-523
-    AeifPar< FAST > A;
-    A.V_peak = ps.p[ 0 ];
-    A.V_reset = ps.p[ 1 ];
-    A.g_L = ps.p[ 2 ];
-    A.C_m = ps.p[ 3 ];
-    A.E_ex = ps.p[ 4 ];
-    A.E_in = ps.p[ 5 ];
-    A.E_L = ps.p[ 6 ];
-    A.Delta_T = ps.p[ 7 ];
-    A.tau_w = ps.p[ 8 ];
-    A.a = ps.p[ 9 ];
-    A.V_th = ps.p[ 11 ];
-    A.tau_ex = ps.p[ 12 ];
-    A.tau_in = ps.p[ 13 ];
-    A.I_e = ps.p[ 14 ];
-    A.tol = ps.p[ 15 ];
-    A.gD = A.g_L * A.Delta_T;
-    if ( FAST )
+    const int c = static_cast< int >( threadIdx.x & 3u );
+    const uint32_t nw = ( static_cast< uint32_t >( d.min_delay ) + 63u ) >> 6;
+    const bool channel = c == 1 or c == 2;
+    const uint32_t ch = static_cast< uint32_t >( c - 1 );
+    gptr< double > const vc = glob( c == 0 ? d.v[ 0 ] : c == 1 ? d.v[ 1 ] : c == 2 ? d.v[ 2 ] : d.v[ 3 ] );
+    AeifLane< FAST > A;
+    A.c = c;
+    uint32_t pset = NONE;  // parameter set in A
+    double b_adapt = 0, V_peak_eff = 0, hstep = 0, I_reset = 0;
+    int32_t refractory_counts = 0;
+    double y = 0, h = 0, tt = 0, in = 0, I_spk = 0;
+    int32_t r = 0;
+    int lag = ph.to, guard = 0, next_sample = ph.to;
+    uint32_t mcol = NONE;
+    unsigned long long bits = 0;  // spikes in lags [64 c, 64 c + 64)
+    uint32_t local = threadIdx.x >> 2, dev = 0;
+    auto take = [ & ]
     {
-      A.r_C_m = wave_uniform( ng_recip( A.C_m ) );
-      A.r_Delta_T = wave_uniform( ng_recip( A.Delta_T ) );
-      A.r_tau_w = wave_uniform( ng_recip( A.tau_w ) );
-      A.r_tau_ex = wave_uniform( ng_recip( A.tau_ex ) );
-      A.r_tau_in = wave_uniform( ng_recip( A.tau_in ) );
-    }
-    const double b_adapt = ps.p[ 10 ];
-    const double V_peak_eff = ps.p[ 16 ];
-    const double hstep = ps.p[ 17 ];
-    double y[ 4 ] = { glob( d.v[ 0 ] )[ dev ], glob( d.v[ 1 ] )[ dev ], glob( d.v[ 2 ] )[ dev ],
-      glob( d.v[ 3 ] )[ dev ] };
-    double hint = glob( d.v[ 4 ] )[ dev ];
-    int32_t r = glob( d.r )[ dev ];
-    // One loop over (lag, accepted step): each iteration makes one adaptive step of the
-    // lane's neuron, or, once the neuron has reached the end of its lag, closes the lag.
-    // Lanes advance through their own lags independently, so a wave costs its slowest
-    // neuron's total number of steps, not the sum over lags of the slowest per lag. Each
-    // neuron's sequence of operations is that of the lag loop with an inner step loop.
-    // More than AEIF_MAX_STEPS accepted steps within one time step stop the lane's lag and
-    // raise ERR_AEIF_STEPS, which fails the run (the oracle stops with the same limit).
-    int lag = ph.from;
-    double tt = 0.0;
-    int guard = 0;
-    while ( lag < ph.to )
+      uint32_t n = 0;
+      if ( c == 0 )
+        n = __hip_atomic_fetch_add( next, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP );
+      local = quad_bcast< 0 >( n );
+    };
+    bool have = false;
+    // Every iteration is one attempted step of the quad's neuron, preceded by the exchange of
+    // a finished neuron for the next one. More than AEIF_MAX_STEPS accepted steps within one
+    // time step stop the neuron's lag and raise ERR_AEIF_STEPS, which fails the run (the
+    // oracle stops with the same limit); a rejected attempt shrinks h by a factor of at most
+    // 0.9 * 1.1^(-1/5) < 0.89 and is accepted once t + h rounds to t, so every quad finishes.
+    for ( ;; )
     {
-      if ( tt < hstep and guard >= AEIF_MAX_STEPS )
+      if ( lag >= ph.to )
       {
-        g_or( &d.counters[ 0 ], ERR_AEIF_STEPS );
+        if ( have )
+        {
+          vc[ dev ] = y;
+          if ( c == 0 )
+            glob( d.v[ 4 ] )[ dev ] = h;
+          if ( c == 1 )
+            glob( d.r )[ dev ] = r;
+          if ( static_cast< uint32_t >( c ) < nw )
+            spk[ local * nw + c ] = bits;
+          take();
+        }
+        if ( not SINGLE )
+          while ( local < nb and glob( d.model )[ dev0 + local ] != M_AEIF_COND_EXP )
+            take();
+        if ( local >= nb )
+          break;
+        have = true;
+        dev = dev0 + local;
+        y = vc[ dev ];
+        h = glob( d.v[ 4 ] )[ dev ];
+        r = glob( d.r )[ dev ];
+        lag = ph.from;
+        in = channel ? C.get( lag, ch, local ) : 0.0;
+        const uint32_t pi = glob( d.pidx )[ dev ];
+        if ( d.mm_int > 0 )
+        {
+          mcol = glob( d.mm_col )[ dev ];
+          next_sample = mcol != NONE ? first_sample_lag( d, ph.origin, ph.from, ph.to ) : ph.to;
+        }
+        if ( pi != pset )
+        {
+          pset = pi;
+          gref< const ParamSet > ps = glob( d.psets )[ pi ];
+          A.V_peak = ps.p[ 0 ];
+          A.V_reset = ps.p[ 1 ];
+          A.Delta_T = ps.p[ 7 ];
+          A.V_th = ps.p[ 11 ];
+          A.I_e = ps.p[ 14 ];
+          A.tol = ps.p[ 15 ];
+          A.gD = ps.p[ 2 ] * ps.p[ 7 ];
+          A.E = ps.p[ c == 1 ? 4 : c == 2 ? 5 : 6 ];
+          A.m = c == 0 ? -ps.p[ 2 ] : ps.p[ 9 ];
+          A.den = ps.p[ c == 0 ? 3 : c == 1 ? 12 : c == 2 ? 13 : 8 ];
+          A.r_den = ng_recip( A.den );
+          A.r_Delta_T = ng_recip( A.Delta_T );
+          b_adapt = ps.p[ 10 ];
+          V_peak_eff = ps.p[ 16 ];
+          hstep = ps.p[ 17 ];
+          refractory_counts = ps.refractory_counts;
+          I_reset = aeif_spike_current( A, aeif_V( A, false, A.V_reset ) );
+        }
+        tt = 0.0;
+        guard = 0;
+        bits = 0;
+        I_spk = aeif_spike_current( A, aeif_V( A, false, quad_bcast< 0 >( y ) ) );
+      }
+      // the derivative at the step's start: its spike current is the one the last step ended
+      // with, or that of the reset potential (inputs change the conductances only)
+      const bool refr = r > 0;
+      const double k1 = aeif_dynamics( A, refr, aeif_V( A, refr, quad_bcast< 0 >( y ) ), I_spk, y );
+      const double dt = hstep - tt;
+      const bool final_step = h > dt;
+      const double h_old = final_step ? dt : h;
+      double yerr, yp, I_end;
+      const double y1 = aeif_rkf45_step( A, refr, y, h_old, k1, yerr, yp, I_end );
+      const double tn = final_step ? hstep : tt + h_old;
+      double h_new = h_old;
+      const int st = aeif_yp_hadjust( A.tol, yerr, yp, &h_new );
+      h = h_new;
+      if ( st < 0 )
+      {
+        if ( fabs( h_new ) < fabs( h_old ) and tn + h_new != tn )
+          continue;  // again from the same state
+        h = h_old;
+      }
+      y = y1;
+      I_spk = I_end;
+      tt = tn;
+      ++guard;
+      const double V = quad_bcast< 0 >( y ), w = quad_bcast< 3 >( y );
+      if ( V < -1e3 or w < -1e6 or w > 1e6 )
+      {
+        if ( c == 0 )
+          g_or( &d.counters[ 0 ], ERR_AEIF_INSTABILITY );
         tt = hstep;
       }
-      if ( tt < hstep )
+      else if ( r > 0 )
       {
-        ++guard;
-        aeif_evolve( A, r > 0, &tt, hstep, &hint, y );
-        if ( y[ 0 ] < -1e3 or y[ 3 ] < -1e6 or y[ 3 ] > 1e6 )
+        y = c == 0 ? A.V_reset : y;
+        I_spk = I_reset;
+      }
+      else if ( V >= V_peak_eff )
+      {
+        y = c == 0 ? A.V_reset : c == 3 ? y + b_adapt : y;
+        I_spk = I_reset;
+        r = refractory_counts > 0 ? refractory_counts + 1 : 0;
+        if ( ( lag >> 6 ) == c )
         {
-          g_or( &d.counters[ 0 ], ERR_AEIF_INSTABILITY );
-          tt = hstep;
-        }
-        else if ( r > 0 )
-          y[ 0 ] = A.V_reset;
-        else if ( y[ 0 ] >= V_peak_eff )
-        {
-          y[ 0 ] = A.V_reset;
-          y[ 3 ] += b_adapt;
-          r = ps.refractory_counts > 0 ? ps.refractory_counts + 1 : 0;
-          const uint64_t bit = 1ull << ( lag & 63 );
-          uint64_t had = 0;
-  #pragma unroll
-          for ( int w = 0; w < 4; ++w )  // lag differs per lane: no dynamic register index
-            if ( ( lag >> 6 ) == w )
-            {
-              had = bits[ w ] & bit;
-              bits[ w ] |= bit;
-            }
-          if ( had )
+          const unsigned long long bit = 1ull << ( lag & 63 );
+          if ( bits & bit )
             g_or( &d.counters[ 0 ], ERR_AEIF_DOUBLE_SPIKE );
+          bits |= bit;
         }
       }
-      else
+      if ( tt < hstep and guard >= AEIF_MAX_STEPS )
+      {
+        if ( c == 0 )
+          g_or( &d.counters[ 0 ], ERR_AEIF_STEPS );
+        tt = hstep;
+      }
+      if ( not( tt < hstep ) )
       {
         if ( r > 0 )
           --r;
-        y[ 1 ] += C.get( lag, 0, local );
-        y[ 2 ] += C.get( lag, 1, local );
-        C.put( lag, 0, local, 0.0 );
-        C.put( lag, 1, local, 0.0 );
+        if ( channel )
+        {
+          y += in;
+          C.put( lag, ch, local, 0.0 );
+        }
         if ( lag == next_sample )
         {
-          store_sample( d, mcol, ph.origin + lag + 1, y[ 0 ], y[ 1 ], y[ 2 ], y[ 3 ] );
+          store_sample_field( d, mcol, ph.origin + lag + 1, c, y );
           next_sample += d.mm_int;
         }
         ++lag;
         tt = 0.0;
         guard = 0;
+        if ( channel and lag < ph.to )
+          in = C.get( lag, ch, local );  // arrives while the lag is integrated
       }
     }
-    for ( int q = 0; q < 4; ++q )
-      glob( d.v[ q ] )[ dev ] = y[ q ];
-    glob( d.v[ 4 ] )[ dev ] = hint;
-    glob( d.r )[ dev ] = r;
+  }
+  template < bool WIN >
+  __device__ __forceinline__ static void
+  update( const NetDev&, gref< const ParamSet >, uint32_t, uint32_t, const Cells< WIN >&, const SlicePhase&, uint64_t*,
+    uint32_t, int )
+  {
+    // aeif_cond_exp neurons are updated by update_block
   }
 };
 
@@ -333,6 +398,7 @@ template <>
 struct DeviceNode< M_IAF_PSC_ALPHA >
 {
   static constexpr bool WIDE = false;
+  static constexpr bool BLOCK = false;
   // iaf_psc_alpha::handle( SpikeEvent& ) (iaf_psc_alpha.cpp:373-383): positive weights to
   // the excitatory channel (1), others to the inhibitory one (0), signed
   __device__ __forceinline__ static void
@@ -416,6 +482,11 @@ struct DeviceNode< M_IAF_PSC_ALPHA >
 #define NG_WIDE( ID ) | ( DeviceNode< ( ID ) >::WIDE ? ( 1 << ( ID ) ) : 0 )
 constexpr int WIDE_MODELS = 0 NG_DEVICE_MODELS( NG_WIDE );
 #undef NG_WIDE
+// models updated by the whole workgroup
+#define NG_BLOCK( ID ) | ( DeviceNode< ( ID ) >::BLOCK ? ( 1 << ( ID ) ) : 0 )
+constexpr int BLOCK_MODELS = 0 NG_DEVICE_MODELS( NG_BLOCK );
+#undef NG_BLOCK
+static_assert( BLOCK_MODELS == 1 << M_AEIF_COND_EXP, "the slice kernel calls this model's update_block" );
 
 // handle( SpikeEvent& ) of model m
 __device__ __forceinline__ void
