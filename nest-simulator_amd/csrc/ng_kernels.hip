@@ -137,8 +137,11 @@ struct SliceLds
       uint32_t bst[ T::BS + 1 ];     // bucket starts
       uint8_t c_lag[ T::CH ];
     };
-    // update: spike bits of the neurons a block-wide update integrates, 64 lags per word
-    unsigned long long spk_bits[ MAX_TB * 4 ];
+    struct  // block-wide update
+    {
+      unsigned long long spk_bits[ MAX_TB * 4 ];  // spike bits per neuron, 64 lags per word
+      uint16_t order[ MAX_TB ];                   // neurons in the order they are taken
+    };
   };
 };
 
@@ -1125,19 +1128,32 @@ __global__ void __launch_bounds__( Tile< WIN >::BS, ( MASK & WIDE_MODELS ) ? 1 :
     if ( G == 0 )
       drive_adds( d, ps, m, dev, local, C, ph.origin, ph.from, 1, ph.to );
   }
-  if constexpr ( ( MASK & BLOCK_MODELS ) != 0 )
+  constexpr bool SINGLE = single_model< MASK >() >= 0;
+  if ( ( MASK & BLOCK_MODELS ) != 0 and ( SINGLE or d.uniform_model < 0 or d.uniform_model == M_AEIF_COND_EXP ) )
   {
     // the neurons of the model that the workgroup updates together
     using Node = DeviceNode< M_AEIF_COND_EXP >;
-    constexpr bool SINGLE = single_model< MASK >() >= 0;
     const lptr< uint32_t > next = ( lptr< uint32_t > )&S.pool_next;
     const lptr< unsigned long long > spk = ( lptr< unsigned long long > )S.spk_bits;
+    lptr< const uint16_t > order = nullptr;
+    if ( nb > static_cast< uint32_t >( BS / 4 ) )
+    {
+      // More neurons than quads: the ones that will probably take many steps go first, so that
+      // no quad starts a long one when the others are done.
+      uint32_t before;
+      const bool first = local < nb and Node::long_update( d, dev );
+      const uint32_t n_first = block_scan< BS >( first ? 1u : 0u, &before, S.sh );
+      if ( local < nb )
+        S.order[ first ? before : n_first + local - before ] = static_cast< uint16_t >( local );
+      order = ( lptr< const uint16_t > )S.order;
+      __syncthreads();
+    }
     if ( d.plain_div )
-      Node::template update_block< WIN, SINGLE, false >( d, dev0, nb, C, ph, next, spk );
+      Node::template update_block< WIN, SINGLE, false >( d, dev0, nb, C, ph, next, spk, order );
     else
-      Node::template update_block< WIN, SINGLE, true >( d, dev0, nb, C, ph, next, spk );
+      Node::template update_block< WIN, SINGLE, true >( d, dev0, nb, C, ph, next, spk, order );
     __syncthreads();
-    if ( local < nb and ( single_model< MASK >() >= 0 or glob( d.model )[ dev ] == M_AEIF_COND_EXP ) )
+    if ( local < nb and ( SINGLE or glob( d.model )[ dev ] == M_AEIF_COND_EXP ) )
     {
       const uint32_t nw = ( static_cast< uint32_t >( d.min_delay ) + 63u ) >> 6;
 #pragma unroll
@@ -1241,6 +1257,7 @@ nestgpu_profile_read( unsigned long long* out8, int reset )
 }
 #endif
 
+#ifndef NG_PART
 // A slice split across Run calls: NEST's per-thread registers hold spikes part by part,
 // so its receive order is (VP, part, node, lag). Rebuild that order once the slice is
 // complete. One workgroup: for each (VP, part), each thread takes one block of the VP's
@@ -1305,30 +1322,33 @@ __global__ void __launch_bounds__( FLATTEN_BS )
   }
 }
 
+#endif  // NG_PART
+
 // ------------------------------------------------------------------ launch wrappers
-template < bool WIN >
-static void
-launch_mask( const NetDev* nets, const uint32_t* blk_prefix, int n_nets, uint32_t total_blocks, int mask, int s,
-  size_t dyn_lds, hipStream_t st )
+// This file is compiled once per model set of a launch (NG_PART: the model id, or ALL_MODELS
+// for launches with several models), which instantiates that set's slice kernels, and once
+// without NG_PART for everything else, so that the instantiations build in parallel.
+#define NG_LAUNCH_ARGS                                                                                  \
+  const NetDev *nets, const uint32_t *blk_prefix, int n_nets, uint32_t total_blocks, bool win, bool stdp, \
+    int s, size_t dyn_lds, hipStream_t st
+template < int MASK >
+void launch_models( NG_LAUNCH_ARGS );
+
+#ifdef NG_PART
+template < int MASK >
+void
+launch_models( NG_LAUNCH_ARGS )
 {
-  // mask: one bit per model id of the launch, and MASK_STDP for stdp_synapse. A launch of one
-  // model takes that model's own instantiation, any other the one with every model.
-  const bool stdp = ( mask & MASK_STDP ) != 0;
-  const int models = mask & ALL_MODELS;
-#define NG_LAUNCH( M )                                                                                        \
-  ( stdp ? k_slice< M, WIN, true ><<< total_blocks, Tile< WIN >::BS, dyn_lds, st >>>( nets, blk_prefix, n_nets, s ) \
-         : k_slice< M, WIN, false ><<< total_blocks, Tile< WIN >::BS, dyn_lds, st >>>( nets, blk_prefix, n_nets, s ) )
-#define NG_ONE( ID )                 \
-  if ( models == ( 1 << ( ID ) ) ) \
-  {                                  \
-    NG_LAUNCH( 1 << ( ID ) );        \
-    return;                          \
-  }
-  NG_DEVICE_MODELS( NG_ONE )
-  NG_LAUNCH( ALL_MODELS );
-#undef NG_ONE
+#define NG_LAUNCH( WIN, STDP )                                                                     \
+  k_slice< MASK, WIN, STDP ><<< total_blocks, Tile< WIN >::BS, dyn_lds, st >>>( nets, blk_prefix, n_nets, s )
+  if ( win )
+    stdp ? NG_LAUNCH( true, true ) : NG_LAUNCH( true, false );
+  else
+    stdp ? NG_LAUNCH( false, true ) : NG_LAUNCH( false, false );
 #undef NG_LAUNCH
 }
+template void launch_models< NG_PART >( NG_LAUNCH_ARGS );
+#else
 
 // Dynamic LDS that limits the slice kernel to wg_per_cu resident workgroups per CU (0: no
 // limit): fewer resident blocks keep the ring buffers they update within the XCD's L2.
@@ -1337,24 +1357,30 @@ slice_lds_for_occupancy( int wg_per_cu, bool win )
 {
   if ( wg_per_cu <= 0 )
     return 0;
-  hipFuncAttributes a;
-  const hipError_t e = win ? hipFuncGetAttributes( &a, reinterpret_cast< const void* >( &k_slice< ALL_MODELS, true > ) )
-                           : hipFuncGetAttributes( &a, reinterpret_cast< const void* >( &k_slice< ALL_MODELS, false > ) );
-  if ( e != hipSuccess )
-    return 0;
+  const size_t own = win ? sizeof( SliceLds< true > ) : sizeof( SliceLds< false > );
   const size_t lds_per_cu = 160 * 1024;
   const size_t want = lds_per_cu / static_cast< size_t >( wg_per_cu + 1 ) + 256;  // more than 1/(k+1)
-  return want > a.sharedSizeBytes ? want - a.sharedSizeBytes : 0;
+  return want > own ? want - own : 0;
 }
 
 hipError_t
 launch_slice( const NetDev* nets, const uint32_t* blk_prefix, int n_nets, uint32_t total_blocks, int mask, bool win,
   int s, size_t dyn_lds, hipStream_t st )
 {
-  if ( win )
-    launch_mask< true >( nets, blk_prefix, n_nets, total_blocks, mask, s, dyn_lds, st );
-  else
-    launch_mask< false >( nets, blk_prefix, n_nets, total_blocks, mask, s, dyn_lds, st );
+  // mask: one bit per model id of the launch, and MASK_STDP for stdp_synapse. A launch of one
+  // model takes that model's own instantiation, any other the one with every model.
+  const bool stdp = ( mask & MASK_STDP ) != 0;
+  switch ( mask & ALL_MODELS )
+  {
+#define NG_ONE( ID )                                                                                                \
+  case 1 << ( ID ):                                                                                                 \
+    launch_models< 1 << ( ID ) >( nets, blk_prefix, n_nets, total_blocks, win, stdp, s, dyn_lds, st );              \
+    break;
+    NG_DEVICE_MODELS( NG_ONE )
+#undef NG_ONE
+  default:
+    launch_models< ALL_MODELS >( nets, blk_prefix, n_nets, total_blocks, win, stdp, s, dyn_lds, st );
+  }
   return hipGetLastError();
 }
 
@@ -1383,5 +1409,7 @@ launch_flatten( NetDev* net, int par, int n_parts, hipStream_t st )
   k_flatten<<< 1, FLATTEN_BS, 0, st >>>( net, par, n_parts );
   return hipGetLastError();
 }
+
+#endif  // NG_PART
 
 }  // namespace nestgpu

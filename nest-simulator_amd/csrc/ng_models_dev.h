@@ -190,6 +190,7 @@ struct DeviceNode< M_AEIF_COND_EXP >
 {
   static constexpr bool WIDE = false;
   static constexpr bool BLOCK = true;
+  static constexpr double LONG_DT = 3.0;  // "close": within this many Delta_T below V_th
   // aeif_cond_exp::handle( SpikeEvent& ) (aeif_cond_exp.cpp:526-541): positive weights to the
   // excitatory conductance (0), others negated to the inhibitory one (1)
   __device__ __forceinline__ static void
@@ -206,18 +207,27 @@ struct DeviceNode< M_AEIF_COND_EXP >
       v = -w;
     }
   }
+  // A neuron that is close to its threshold at the start of a slice will probably take many
+  // steps in it.
+  __device__ __forceinline__ static bool
+  long_update( const NetDev& d, uint32_t dev )
+  {
+    gref< const ParamSet > ps = glob( d.psets )[ glob( d.pidx )[ dev ] ];
+    return glob( d.r )[ dev ] == 0 and glob( d.v[ 0 ] )[ dev ] > ps.p[ 11 ] - LONG_DT * ps.p[ 7 ];
+  }
   // Updates the block's aeif_cond_exp neurons with every thread of the workgroup, four lanes
   // per neuron (ng_aeif.h). Neurons need very different numbers of steps (a slice of 15 steps
   // takes 16 attempted steps on average and up to 166), so a quad that finishes its neuron
   // takes the next one of the block from the counter *next (which starts at the number of
-  // quads) instead of waiting for the slowest lane of its wave. spk: spike bits of every
+  // quads) instead of waiting for the slowest lane of its wave. order: the order in which a block
+  // with more neurons than quads takes them (likely long updates first), or null. spk: spike bits of every
   // neuron, [local][words of 64 lags]. Which quad integrates a neuron does not change its
   // operations. Measured on the MI355X: 6,000 neurons, slices of 15 steps, 32 per block: AEIF_T1;
   // the mixed sweep of 48 networks, 512 per block: AEIF_T2.
   template < bool WIN, bool SINGLE, bool FAST >
   __device__ __forceinline__ static void
   update_block( const NetDev& d, uint32_t dev0, uint32_t nb, const Cells< WIN >& C, const SlicePhase& ph,
-    lptr< uint32_t > next, lptr< unsigned long long > spk )
+    lptr< uint32_t > next, lptr< unsigned long long > spk, lptr< const uint16_t > order )
   {
     // models/aeif_cond_exp.cpp:443-523
     const int c = static_cast< int >( threadIdx.x & 3u );
@@ -235,13 +245,14 @@ struct DeviceNode< M_AEIF_COND_EXP >
     int lag = ph.to, guard = 0, next_sample = ph.to;
     uint32_t mcol = NONE;
     unsigned long long bits = 0;  // spikes in lags [64 c, 64 c + 64)
-    uint32_t local = threadIdx.x >> 2, dev = 0;
+    auto at = [ & ]( uint32_t i ) { return i < nb and order ? static_cast< uint32_t >( order[ i ] ) : i; };
+    uint32_t local = at( threadIdx.x >> 2 ), dev = 0;
     auto take = [ & ]
     {
       uint32_t n = 0;
       if ( c == 0 )
         n = __hip_atomic_fetch_add( next, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP );
-      local = quad_bcast< 0 >( n );
+      local = at( quad_bcast< 0 >( n ) );
     };
     bool have = false;
     // Every iteration is one attempted step of the quad's neuron, preceded by the exchange of
