@@ -646,6 +646,36 @@ Runner::run( const std::vector< Engine* >& engines, const std::vector< int64_t >
 
 namespace
 {
+// The order in which a launch holds the instances: those with models that integrate
+// adaptively first (their workgroups take several times as long as the others'), larger
+// networks first among equals.
+std::vector< int >
+launch_order( const std::vector< Engine* >& engines )
+{
+  std::vector< int > order( engines.size() );
+  for ( size_t i = 0; i < order.size(); ++i )
+    order[ i ] = static_cast< int >( i );
+  std::stable_sort( order.begin(), order.end(),
+    [ & ]( int a, int b )
+    {
+      const bool ha = engines[ a ]->model_mask() & ( 1 << M_AEIF_COND_EXP );
+      const bool hb = engines[ b ]->model_mask() & ( 1 << M_AEIF_COND_EXP );
+      return ha != hb ? ha : engines[ a ]->net().n > engines[ b ]->net().n;
+    } );
+  return order;
+}
+
+// v in launch order
+template < typename T >
+std::vector< T >
+in_order( const std::vector< T >& v, const std::vector< int >& order )
+{
+  std::vector< T > out( v.size() );
+  for ( size_t i = 0; i < order.size(); ++i )
+    out[ i ] = v[ order[ i ] ];
+  return out;
+}
+
 // Launch records of one chunk: every instance's clock, first step and steps to do. Returns
 // false when no instance has work; prefix, mask, win and split describe the launch.
 bool
@@ -790,6 +820,19 @@ finish_chunk( const std::vector< Engine* >& engines, const NetDev* h_nets, const
 bool
 Runner::run_chunk( const std::vector< Engine* >& engines, std::vector< int64_t >& remaining )
 {
+  if ( engines.size() <= 1 )
+    return run_chunk_ordered( engines, remaining );
+  const std::vector< int > order = launch_order( engines );
+  std::vector< int64_t > left = in_order( remaining, order );
+  const bool more = run_chunk_ordered( in_order( engines, order ), left );
+  for ( size_t i = 0; i < order.size(); ++i )
+    remaining[ order[ i ] ] = left[ i ];
+  return more;
+}
+
+bool
+Runner::run_chunk_ordered( const std::vector< Engine* >& engines, std::vector< int64_t >& remaining )
+{
   hip_check( hipSetDevice( device_ ), "hipSetDevice" );
   const int n = static_cast< int >( engines.size() );
   if ( n == 0 )
@@ -874,8 +917,10 @@ noalloc_scratch( int device )
 }  // namespace
 
 void
-run_noalloc( int device, const std::vector< Engine* >& engines, const std::vector< int64_t >& steps, int S )
+run_noalloc( int device, const std::vector< Engine* >& unordered, const std::vector< int64_t >& steps, int S )
 {
+  const std::vector< int > order = launch_order( unordered );
+  const std::vector< Engine* > engines = in_order( unordered, order );
   const int n = static_cast< int >( engines.size() );
   if ( n > NOALLOC_MAX_NETS )
     throw std::runtime_error( "run without allocation: " + std::to_string( n ) + " instances, at most "
@@ -896,7 +941,7 @@ run_noalloc( int device, const std::vector< Engine* >& engines, const std::vecto
   const hipStream_t st = nullptr;  // the device's null stream: nothing to create
   NetDev h_nets[ NOALLOC_MAX_NETS ];
   unsigned long long h_status[ 2 * NOALLOC_MAX_NETS ];
-  std::vector< int64_t > remaining = steps;
+  std::vector< int64_t > remaining = in_order( steps, order );
   std::vector< uint32_t > prefix;
   for ( ;; )
   {

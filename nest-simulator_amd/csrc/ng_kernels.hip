@@ -146,7 +146,10 @@ struct SliceLds
 };
 
 // XCD-aware block mapping: workgroups are dispatched round-robin over 8 XCDs; give each
-// XCD a contiguous range of blocks so neighbouring blocks share its L2.
+// XCD a contiguous range of blocks so neighbouring blocks share its L2. A launch of several
+// instances keeps the dispatch order instead: the host puts the instances with the longest
+// workgroups first, which then start on different CUs of every XCD, and lighter ones fill up
+// (48 networks, half of them aeif_cond_exp, 380 workgroups: 12.8 -> 10.5 ms per 10 slices).
 __device__ inline uint32_t
 xcd_block( uint32_t w, uint32_t total )
 {
@@ -633,7 +636,7 @@ __global__ void __launch_bounds__( Tile< WIN >::BS, ( MASK & WIDE_MODELS ) ? 1 :
   constexpr int R = Tile< WIN >::R;
 
   // ---- which instance and block
-  const uint32_t gb = xcd_block( blockIdx.x, gridDim.x );
+  const uint32_t gb = n_nets > 1 ? blockIdx.x : xcd_block( blockIdx.x, gridDim.x );
   int lo = 0, hi = n_nets;
   while ( hi - lo > 1 )
   {
