@@ -104,7 +104,7 @@ struct SynRec
 
 // ring-buffer slots staged in LDS per workgroup and slice (window delivery), in doubles;
 // sized so that two window workgroups fit in a CU's LDS
-constexpr uint32_t WIN_CAP = 6264;
+constexpr uint32_t WIN_CAP = 6008;
 constexpr uint32_t MAX_TB = 512;      // targets per block = threads per workgroup
 constexpr uint32_t PMAX_WIN = 512;    // blocks per instance, window delivery
 constexpr uint32_t PMAX_GLOB = 2048;  // blocks per instance, global delivery
@@ -112,7 +112,7 @@ constexpr int MAX_PASSES = 3;         // slot-range passes of global delivery
 constexpr uint32_t MM_ROWS = 256;     // multimeter sample rows per chunk
 // LDS cell cache of cache delivery (in the window's LDS area): open addressing over the ring
 // cell index, CACHE_SLOTS keys then CACHE_SLOTS FP64 values, at most CACHE_PROBES probes
-constexpr uint32_t CACHE_SLOTS = 4096;
+constexpr uint32_t CACHE_SLOTS = 4004;
 constexpr uint32_t CACHE_PROBES = 32;
 static_assert( CACHE_SLOTS * ( 4 + 8 ) <= WIN_CAP * 8, "the cell cache must fit the window's LDS area" );
 

@@ -568,10 +568,10 @@ Runner::ensure_capacity( size_t n )
 }
 
 bool
-Runner::capture( int n_nets, uint32_t total_blocks, int mask, bool win )
+Runner::capture( int n_nets, uint32_t total_blocks, int mask, int delivery )
 {
-  const bool same_key = exec_n_ == n_nets and exec_total_ == total_blocks and exec_mask_ == mask and exec_win_ == win
-    and exec_wg_ == wg_per_cu;
+  const bool same_key = exec_n_ == n_nets and exec_total_ == total_blocks and exec_mask_ == mask
+    and exec_delivery_ == delivery and exec_wg_ == wg_per_cu;
   if ( same_key and ( exec_ or exec_failed_ ) )
     return exec_ != nullptr;
   if ( exec_ )
@@ -586,7 +586,7 @@ Runner::capture( int n_nets, uint32_t total_blocks, int mask, bool win )
   exec_n_ = n_nets;
   exec_total_ = total_blocks;
   exec_mask_ = mask;
-  exec_win_ = win;
+  exec_delivery_ = delivery;
   exec_wg_ = wg_per_cu;
   exec_failed_ = true;
   hipGraph_t g = nullptr;
@@ -597,8 +597,8 @@ Runner::capture( int n_nets, uint32_t total_blocks, int mask, bool win )
     return false;
   }
   for ( int s = 0; s < S_; ++s )
-    launch_slice( d_nets_, d_prefix_, n_nets, total_blocks, mask, win, s, slice_lds_for_occupancy( wg_per_cu, win ),
-      stream_ );
+    launch_slice( d_nets_, d_prefix_, n_nets, total_blocks, mask, delivery, s,
+      slice_lds_for_occupancy( wg_per_cu, delivery != LAUNCH_GLOBAL ), stream_ );
   const hipError_t ended = hipStreamEndCapture( stream_, &g );
   if ( ended != hipSuccess or g == nullptr or hipGraphInstantiate( &exec_, g, nullptr, nullptr, 0 ) != hipSuccess )
   {
@@ -615,11 +615,12 @@ Runner::capture( int n_nets, uint32_t total_blocks, int mask, bool win )
 }
 
 void
-Runner::launch_one( int n, uint32_t total, int mask, bool win, int s, hipEvent_t* ev )
+Runner::launch_one( int n, uint32_t total, int mask, int delivery, int s, hipEvent_t* ev )
 {
   if ( ev )
     hip_check( hipEventRecord( ev[ 0 ], stream_ ), "hipEventRecord" );
-  hip_check( launch_slice( d_nets_, d_prefix_, n, total, mask, win, s, slice_lds_for_occupancy( wg_per_cu, win ), stream_ ),
+  hip_check( launch_slice( d_nets_, d_prefix_, n, total, mask, delivery, s,
+               slice_lds_for_occupancy( wg_per_cu, delivery != LAUNCH_GLOBAL ), stream_ ),
     "launch_slice" );
   if ( ev )
   {
@@ -677,21 +678,23 @@ in_order( const std::vector< T >& v, const std::vector< int >& order )
 }
 
 // Launch records of one chunk: every instance's clock, first step and steps to do. Returns
-// false when no instance has work; prefix, mask, win and split describe the launch.
+// false when no instance has work; prefix, mask, delivery and split describe the launch.
 bool
 stage_chunk( const std::vector< Engine* >& engines, const std::vector< int64_t >& remaining, int S, NetDev* h_nets,
-  std::vector< uint32_t >& prefix, int& mask, bool& win, bool& split )
+  std::vector< uint32_t >& prefix, int& mask, int& delivery, bool& split )
 {
   const int n = static_cast< int >( engines.size() );
   mask = 0;
-  win = false;
+  delivery = LAUNCH_GLOBAL;
   split = false;
   prefix.assign( n + 1, 0 );
   for ( int i = 0; i < n; ++i )
   {
     mask |= engines[ i ]->model_mask();
-    // the window kernel also carries the cell cache of cache delivery
-    win = win or engines[ i ]->window() or engines[ i ]->cache();
+    if ( engines[ i ]->cache() )
+      delivery = LAUNCH_CACHE;
+    else if ( engines[ i ]->window() and delivery == LAUNCH_GLOBAL )
+      delivery = LAUNCH_WINDOW;
     prefix[ i + 1 ] = prefix[ i ] + engines[ i ]->net().n_blocks;
   }
   if ( prefix[ n ] == 0 )
@@ -839,11 +842,12 @@ Runner::run_chunk_ordered( const std::vector< Engine* >& engines, std::vector< i
     return false;
   ensure_capacity( n );
   int mask = 0;
-  bool win = false, split = false;
+  int delivery = LAUNCH_GLOBAL;
+  bool split = false;
   std::vector< uint32_t > prefix;
   // the window kernel runs instances with a window (at most PMAX_WIN blocks, checked at
   // build) and without one (their block prefix lives in the unused window)
-  if ( not stage_chunk( engines, remaining, S_, h_nets_, prefix, mask, win, split ) )
+  if ( not stage_chunk( engines, remaining, S_, h_nets_, prefix, mask, delivery, split ) )
     return false;
   const uint32_t total = prefix[ n ];
   if ( prefix != prefix_ )
@@ -851,13 +855,23 @@ Runner::run_chunk_ordered( const std::vector< Engine* >& engines, std::vector< i
     hip_check( hipMemcpy( d_prefix_, prefix.data(), ( n + 1 ) * sizeof( uint32_t ), hipMemcpyHostToDevice ), "prefix" );
     prefix_ = prefix;
   }
-  const bool graph = use_graph and not time_kernels and not split and capture( n, total, mask, win );
+  // slices this chunk has work for
+  int slices = 0;
+  for ( int i = 0; i < n; ++i )
+    if ( h_nets_[ i ].active )
+      slices = std::max( slices,
+        static_cast< int >( ( h_nets_[ i ].from0 + h_nets_[ i ].todo + h_nets_[ i ].min_delay - 1 ) / h_nets_[ i ].min_delay ) );
+  // A captured graph holds a launch for every slice of a full chunk (an empty one costs 1.7 us);
+  // shorter chunks launch their slices directly (2.4 us of host time each, behind the slice
+  // before): a single slice of a 500-neuron network took 98 us as a graph, 64 of them empty.
+  const bool graph =
+    use_graph and not time_kernels and not split and slices == S_ and capture( n, total, mask, delivery );
   ++( graph ? graph_chunks : direct_chunks );
   hip_check( hipMemcpyAsync( d_nets_, h_nets_, n * sizeof( NetDev ), hipMemcpyHostToDevice, stream_ ), "nets H2D" );
   hip_check( hipEventRecord( ev_chunk_[ 0 ], stream_ ), "hipEventRecord" );
   if ( not graph )
     launch_chunk_direct( h_nets_, d_nets_, n, S_, split, stream_,
-      [ & ]( int s ) { launch_one( n, total, mask, win, s, time_kernels ? ev_kernel_ : nullptr ); } );
+      [ & ]( int s ) { launch_one( n, total, mask, delivery, s, time_kernels ? ev_kernel_ : nullptr ); } );
   else
     hip_check( hipGraphLaunch( exec_, stream_ ), "hipGraphLaunch" );
   hip_check( hipEventRecord( ev_chunk_[ 1 ], stream_ ), "hipEventRecord" );
@@ -946,8 +960,9 @@ run_noalloc( int device, const std::vector< Engine* >& unordered, const std::vec
   for ( ;; )
   {
     int mask = 0;
-    bool win = false, split = false;
-    if ( not stage_chunk( engines, remaining, S, h_nets, prefix, mask, win, split ) )
+    int delivery = LAUNCH_GLOBAL;
+    bool split = false;
+    if ( not stage_chunk( engines, remaining, S, h_nets, prefix, mask, delivery, split ) )
       break;
     const uint32_t total = prefix[ n ];
     // every word the kernels read is written here for each chunk, so nothing left in the
@@ -956,7 +971,7 @@ run_noalloc( int device, const std::vector< Engine* >& unordered, const std::vec
       "prefix" );
     hip_check( hipMemcpyAsync( d_nets, h_nets, n * sizeof( NetDev ), hipMemcpyHostToDevice, st ), "nets H2D" );
     launch_chunk_direct( h_nets, d_nets, n, S, split, st,
-      [ & ]( int s ) { hip_check( launch_slice( d_nets, d_prefix, n, total, mask, win, s, 0, st ), "launch_slice" ); } );
+      [ & ]( int s ) { hip_check( launch_slice( d_nets, d_prefix, n, total, mask, delivery, s, 0, st ), "launch_slice" ); } );
     hip_check( launch_status( d_nets, n, d_status, st ), "launch_status" );
     hip_check( hipMemcpyAsync( h_status, d_status, 2 * n * sizeof( unsigned long long ), hipMemcpyDeviceToHost, st ),
       "status D2H" );

@@ -50,11 +50,20 @@ using HostArray = std::vector< T, NoInitAlloc< T > >;
 namespace nestgpu
 {
 
+// What the instances of a launch need of the slice kernel: ring cells in HBM only, an LDS
+// ring-buffer window (which instances without one can share), or the LDS cell cache.
+enum LaunchDelivery
+{
+  LAUNCH_GLOBAL = 0,
+  LAUNCH_WINDOW,
+  LAUNCH_CACHE
+};
+
 // Enqueue the slice kernel for slice s of a chunk over all blocks of n_nets instances.
-// mask: bit m set if neuron model m occurs (selects a specialised kernel); win: some
-// instance uses window delivery (selects the kernel with the LDS ring-buffer window).
+// mask: bit m set if neuron model m occurs (selects a specialised kernel); delivery: a
+// LaunchDelivery.
 hipError_t launch_slice( const NetDev* nets, const uint32_t* blk_prefix, int n_nets, uint32_t total_blocks, int mask,
-  bool win, int s, size_t dyn_lds, hipStream_t st );
+  int delivery, int s, size_t dyn_lds, hipStream_t st );
 // Dynamic LDS bytes that cap the slice kernel at wg_per_cu workgroups per CU (0: no cap).
 size_t slice_lds_for_occupancy( int wg_per_cu, bool win );
 // Rebuild the exact receive order of a slice that was split across Run calls.
@@ -283,8 +292,8 @@ public:
 private:
   bool run_chunk_ordered( const std::vector< Engine* >& engines, std::vector< int64_t >& remaining );
   void ensure_capacity( size_t n );
-  bool capture( int n_nets, uint32_t total_blocks, int mask, bool win );  // false: launch directly
-  void launch_one( int n, uint32_t total, int mask, bool win, int s, hipEvent_t* ev );
+  bool capture( int n_nets, uint32_t total_blocks, int mask, int delivery );  // false: launch directly
+  void launch_one( int n, uint32_t total, int mask, int delivery, int s, hipEvent_t* ev );
   int device_;
   int S_;
   hipStream_t stream_ = nullptr;
@@ -301,7 +310,7 @@ private:
   int exec_n_ = -1;
   uint32_t exec_total_ = 0;
   int exec_mask_ = 0;
-  bool exec_win_ = false;
+  int exec_delivery_ = 0;
   int exec_wg_ = 0;
   std::vector< uint32_t > prefix_;
   double last_ms_ = 0;

@@ -37,7 +37,7 @@ namespace nestgpu
 {
 
 constexpr int IDX_BITS = 11;  // bucket key = slot-channel << 11 | round index: sorted keys group
-                              // a target's events by cell, in key order within each cell
+                              // a bucket's events by cell, in key order within each cell
 
 // Tile shape per kernel variant. The window kernel halves chunk and round so that, with its
 // ring-buffer window, two workgroups fit in the 160 KB of LDS of a CU.
@@ -122,19 +122,20 @@ struct SliceLds
   unsigned long long log_base;
   uint32_t sh[ T::BS / 64 ];
   uint32_t cnt_base;
-  uint32_t pool_next;  // next neuron of the block-wide update
+  uint32_t pool_next;  // next neuron of a block-wide update
   union
   {
     struct  // delivery
     {
-      double bw[ T::R ];             // event values, bucketed by target
+      double sw[ T::R ];             // event values in sorted order
       uint32_t pref[ T::PMAX + 1 ];  // prefix of per-block spike counts
       uint32_t c_g0[ T::CH ];        // first synapse of each chunk spike's run
       uint32_t c_off[ T::CH + 1 ];   // exclusive prefix of run lengths
-      uint32_t bk[ T::R ];           // event keys (slot-channel << 11 | round index), bucketed by target
-      uint16_t perm[ T::R ];         // bucket position of the event at each sorted position
-      uint32_t bcnt[ 2 ][ T::BS ];   // events per target, alternating between rounds
-      uint32_t bst[ T::BS + 1 ];     // bucket starts
+      uint32_t bk[ T::R ];           // event keys (slot-channel << 11 | round index), by bucket
+      uint32_t sk[ T::R ];           // event keys in sorted order
+      uint32_t bcnt[ 2 ][ T::BS ];   // events per bucket, alternating between rounds
+      uint16_t bst[ T::BS + 2 ];     // bucket starts
+      uint16_t c_idx[ T::BS ];       // spike of every 2^sh-th event of the chunk
       uint8_t c_lag[ T::CH ];
     };
     struct  // block-wide update
@@ -144,6 +145,8 @@ struct SliceLds
     };
   };
 };
+
+static_assert( sizeof( SliceLds< true > ) <= 80 * 1024, "two window workgroups share the 160 KB of a CU" );
 
 // XCD-aware block mapping: workgroups are dispatched round-robin over 8 XCDs; give each
 // XCD a contiguous range of blocks so neighbouring blocks share its L2. A launch of several
@@ -229,7 +232,7 @@ block_scan( uint32_t v, uint32_t* excl, uint32_t* sh )
   }
   *excl = pre + x - v;
   __syncthreads();
-  return tot;
+  return __builtin_amdgcn_readfirstlane( tot );  // the same in every thread
 }
 
 // Poisson count for seeded drive: splitmix64 of (seed, stream, step) gives u in [0, 1), the
@@ -319,7 +322,7 @@ constexpr uint32_t EMPTY_KEY = 0xffffffffu;
 __device__ inline uint32_t
 cache_hash( uint32_t cell )
 {
-  return ( cell * 2654435761u ) >> 20;  // 12 bits: CACHE_SLOTS = 4096
+  return __umulhi( cell * 2654435761u, CACHE_SLOTS );
 }
 // slot of cell in the cache, or NONE when the cell is not cached
 __device__ inline uint32_t
@@ -333,7 +336,7 @@ cache_find( lptr< const uint32_t > keys, uint32_t cell )
       return h;
     if ( k == EMPTY_KEY )
       return NONE;
-    h = ( h + 1 ) & ( CACHE_SLOTS - 1 );
+    h = h + 1 < CACHE_SLOTS ? h + 1 : 0;
   }
   return NONE;
 }
@@ -350,7 +353,7 @@ cache_insert( lptr< uint32_t > keys, uint32_t cell )
       return h;
     if ( k == cell )
       return NONE;
-    h = ( h + 1 ) & ( CACHE_SLOTS - 1 );
+    h = h + 1 < CACHE_SLOTS ? h + 1 : 0;
   }
   return NONE;  // no free slot within the probe limit: the cell stays in the ring
 }
@@ -360,9 +363,9 @@ __device__ __forceinline__ void node_receive( int m, double w, uint32_t& ch, dou
 
 // spike_generator drive of this part: handle() of the target with weight * multiplicity.
 // Each lag adds into a different cell, so the cells of LB lags are read together.
-template < bool WIN >
+template < class CELLS >
 __device__ inline void
-drive_adds( const NetDev& d, gref< const ParamSet > ps, int m, uint32_t dev, uint32_t local, const Cells< WIN >& C,
+drive_adds( const NetDev& d, gref< const ParamSet > ps, int m, uint32_t dev, uint32_t local, const CELLS& C,
   int64_t origin, int from, int stride, int to )
 {
   const int32_t mode = ps.drive_mode;
@@ -621,7 +624,11 @@ stdp_spikes( const NetDev& d, uint32_t dev, int64_t origin, uint32_t par, const 
 
 // STDP: some instance of the launch has stdp_synapse connections (its own instantiation, so
 // that networks without them carry none of that code or its registers)
-template < int MASK, bool WIN, bool STDP = false >
+//
+// CACHE: some instance of the launch uses cache delivery; one instantiation, with every model,
+// serves these launches, so that the cache costs the others no registers (with it in the window
+// kernels, 389 scalar registers spilled into vector lanes).
+template < int MASK, bool WIN, bool STDP, bool CACHE >
 __global__ void __launch_bounds__( Tile< WIN >::BS, ( MASK & WIDE_MODELS ) ? 1 : 4 )
   k_slice( const NetDev* __restrict__ nets, const uint32_t* __restrict__ blk_prefix, int n_nets, int s )
 {
@@ -652,18 +659,14 @@ __global__ void __launch_bounds__( Tile< WIN >::BS, ( MASK & WIDE_MODELS ) ? 1 :
   if ( not ph.active or b >= d.n_blocks )
     return;
   // the block's targets: device indices dev0 .. dev0 + nb - 1
-  const uint32_t dev0 = glob( d.bstart )[ b ];
-  const uint32_t nb = glob( d.bstart )[ b + 1 ] - dev0;
+  const uint32_t dev0 = __builtin_amdgcn_readfirstlane( glob( d.bstart )[ b ] );
+  const uint32_t nb = __builtin_amdgcn_readfirstlane( glob( d.bstart )[ b + 1 ] ) - dev0;
   // phase timing (counters[4..6]): thread 0 reads the 100 MHz wall clock at the start, after
   // delivery and at the end of the workgroup's work
   const bool ptime = d.phase_timing != 0;
   unsigned long long tp0 = 0, tp1 = 0;
-  if ( ptime and threadIdx.x == 0 )
-    tp0 = wall_clock64();
   const uint32_t P = d.n_blocks;
   const uint32_t tb = d.tb;
-  const int par = ph.parity;
-  const int ppar = par ^ 1;
   const uint32_t t = threadIdx.x;
 
   Cells< WIN > C;
@@ -680,6 +683,10 @@ __global__ void __launch_bounds__( Tile< WIN >::BS, ( MASK & WIDE_MODELS ) ? 1 :
   const __amdgpu_buffer_rsrc_t rb_rsrc = __builtin_amdgcn_make_buffer_rsrc(
     d.rb + static_cast< size_t >( b ) * C.L * C.nct, 0, static_cast< int >( C.L * C.nct * 8u ), 0x00020000 );
 
+  const int par = ph.parity;
+  const int ppar = par ^ 1;
+  if ( ptime and threadIdx.x == 0 )
+    tp0 = wall_clock64();
   // ================================================================ 0. stage the window
   uint32_t w0 = C.s0 + C.wa;  // ring slot of the window's first slot
   if ( w0 >= C.L )
@@ -692,7 +699,7 @@ __global__ void __launch_bounds__( Tile< WIN >::BS, ( MASK & WIDE_MODELS ) ? 1 :
       S.win[ i ] = C.rbb[ i < before_wrap ? w0 * C.nct + i : i - before_wrap ];
   }
   // cache delivery: an empty cell cache for this slice (keys, then values, in the window area)
-  const bool cache = WIN and d.cache != 0 and ph.deliver;
+  const bool cache = CACHE and d.cache != 0 and ph.deliver;
   const lptr< uint32_t > ckey = ( lptr< uint32_t > )reinterpret_cast< uint32_t* >( S.win );
   const lptr< double > cval = ( lptr< double > )( S.win + CACHE_SLOTS / 2 );
   if ( cache )
@@ -708,10 +715,10 @@ __global__ void __launch_bounds__( Tile< WIN >::BS, ( MASK & WIDE_MODELS ) ? 1 :
     S.bcnt[ 0 ][ t ] = 0;
     S.bcnt[ 1 ][ t ] = 0;
     int cur = 0;  // counter buffer of the current round
-    const bool flat = glob( d.flat_meta )[ 2 + ppar ] != 0;
+    const bool flat = __builtin_amdgcn_readfirstlane( glob( d.flat_meta )[ 2 + ppar ] ) != 0;
     uint32_t K;
     if ( flat )
-      K = glob( d.flat_meta )[ ppar ];
+      K = __builtin_amdgcn_readfirstlane( glob( d.flat_meta )[ ppar ] );
     else
     {
       // prefix of the per-block spike counts of the delivered slice
@@ -733,6 +740,12 @@ __global__ void __launch_bounds__( Tile< WIN >::BS, ( MASK & WIDE_MODELS ) ? 1 :
     __syncthreads();
     NG_PHASE( 0 );
     unsigned long long events = 0;
+    // A block with few targets splits each target's bucket by slot, up to the number of
+    // counters: a bucket's events are compared with each other, and 32 targets alone would make
+    // buckets of 32 events (5,000 iaf_psc_delta neurons, 226,000 events per slice: 30 -> 25 us
+    // with the sorted arrays and the event index; 100,000 iaf_psc_exp, 4.9M events: 118 -> 103;
+    // the full 8-population circuit, 1.75M events: 46 -> 42).
+    const uint32_t sub_mask = ( 1u << ( 31 - __builtin_clz( static_cast< uint32_t >( BS ) / nb ) ) ) - 1u;
     // events received by this thread's target (local index t), counted while d.rx is set
     uint32_t rxc = 0;
     for ( uint32_t k0 = 0; k0 < K; k0 += CH )
@@ -762,8 +775,8 @@ __global__ void __launch_bounds__( Tile< WIN >::BS, ( MASK & WIDE_MODELS ) ? 1 :
           {
             while ( pref[ blk + 1 ] <= k )
               ++blk;
-            const uint32_t e =
-              glob( d.blk_spk )[ ( static_cast< size_t >( ppar ) * P + blk ) * d.spk_cap + ( k - pref[ blk ] ) ];
+            const size_t at = ( static_cast< size_t >( ppar ) * P + blk ) * d.spk_cap + ( k - pref[ blk ] );
+            const uint32_t e = glob( d.blk_spk )[ at ];
             src[ q ] = e >> 8;
             lag[ q ] = e & 0xffu;
           }
@@ -821,6 +834,21 @@ __global__ void __launch_bounds__( Tile< WIN >::BS, ( MASK & WIDE_MODELS ) ? 1 :
       }
       if ( t == 0 )
         S.c_off[ CH ] = E;
+      // The spike of every 2^sh-th event (sh the smallest with at most BS of them): an event's
+      // spike is then a table read and a short walk instead of a binary search over the chunk
+      // (11 dependent LDS reads per round).
+      const int sh = E > static_cast< uint32_t >( BS ) ? 32 - __builtin_clz( ( E - 1 ) / BS ) : 0;
+      {
+        uint32_t off = ex - mine;
+#pragma unroll
+        for ( int q = 0; q < SPT; ++q )
+        {
+          const uint32_t end = off + lens[ q ];
+          for ( uint32_t m = ( off + ( 1u << sh ) - 1 ) >> sh; ( m << sh ) < end; ++m )
+            S.c_idx[ m ] = static_cast< uint16_t >( t * SPT + q );
+          off = end;
+        }
+      }
       __syncthreads();
       NG_PHASE( 1 );
       events += E;
@@ -892,7 +920,7 @@ __global__ void __launch_bounds__( Tile< WIN >::BS, ( MASK & WIDE_MODELS ) ? 1 :
       auto load_round = [ & ]( uint32_t e0 )
       {
         const uint32_t eb = e0 + t * RQ;
-        uint32_t j = upper_bound_u32( S.c_off, CH + 1, eb < E ? eb : E - 1 ) - 1;
+        uint32_t j = S.c_idx[ ( eb < E ? eb : E - 1 ) >> sh ];
 #pragma unroll
         for ( int q = 0; q < RQ; ++q )
         {
@@ -943,19 +971,17 @@ __global__ void __launch_bounds__( Tile< WIN >::BS, ( MASK & WIDE_MODELS ) ? 1 :
             uint32_t ch;
             double v;
             node_receive( m, w, ch, v );  // static_synapse: weight * multiplicity 1
-            loc[ q ] = local;
+            const uint32_t sc = slot_rel * d.nch + ch;
+            loc[ q ] = local + nb * ( sc & sub_mask );
             val[ q ] = v;
-            key[ q ] = ( ( slot_rel * d.nch + ch ) << IDX_BITS ) | static_cast< uint32_t >( t * RQ + q );
-            dst[ q ] = atomicAdd( &S.bcnt[ cur ][ local ], 1u );
+            key[ q ] = ( sc << IDX_BITS ) | static_cast< uint32_t >( t * RQ + q );
+            dst[ q ] = atomicAdd( &S.bcnt[ cur ][ loc[ q ] ], 1u );
             lw[ q ] = C.in_window( slot_rel );
             if ( lw[ q ] )
-              ci[ q ] = ( slot_rel - C.wa ) * C.nct + ch * tb + local;
+              ci[ q ] = C.win_index( slot_rel, ch, local );
             else
             {
-              uint32_t slot = C.s0 + slot_rel;
-              if ( slot >= C.L )
-                slot -= C.L;
-              ci[ q ] = slot * C.nct + ch * tb + local;
+              ci[ q ] = C.ring_index( slot_rel, ch, local );
               const uint32_t hs = cache ? cache_find( ckey, ci[ q ] ) : NONE;
               if ( hs != NONE )
               {
@@ -994,15 +1020,16 @@ __global__ void __launch_bounds__( Tile< WIN >::BS, ( MASK & WIDE_MODELS ) ? 1 :
 #pragma unroll
           for ( int j = 0; j < CPL; ++j )
           {
-            S.bst[ CPL * t + j ] = run;
+            S.bst[ CPL * t + j ] = static_cast< uint16_t >( run );
             run += c[ j ];
           }
           if ( t == 63 )
-            S.bst[ BS ] = run;
+            S.bst[ BS ] = static_cast< uint16_t >( run );
         }
         S.bcnt[ cur ^ 1 ][ t ] = 0;
-        if ( d.rx )
-          rxc += S.bcnt[ cur ][ t ];
+        if ( d.rx and t < nb )
+          for ( uint32_t q = t; q <= t + nb * sub_mask; q += nb )
+            rxc += S.bcnt[ cur ][ q ];
         __syncthreads();
         NG_PHASE( 3 );  // bucket starts
 #pragma unroll
@@ -1011,11 +1038,11 @@ __global__ void __launch_bounds__( Tile< WIN >::BS, ( MASK & WIDE_MODELS ) ? 1 :
           {
             dst[ q ] += S.bst[ loc[ q ] ];
             S.bk[ dst[ q ] ] = key[ q ];
-            S.bw[ dst[ q ] ] = val[ q ];
           }
         __syncthreads();
         // sorted place of each event in its bucket by (cell, key): the number of smaller keys
-        uint32_t srt[ RQ ];
+        uint32_t srt[ RQ ], bhi[ RQ ];
+        bool lead[ RQ ];
 #pragma unroll
         for ( int q = 0; q < RQ; ++q )
           if ( loc[ q ] != NONE )
@@ -1032,7 +1059,10 @@ __global__ void __launch_bounds__( Tile< WIN >::BS, ( MASK & WIDE_MODELS ) ? 1 :
             for ( ; i < hi; ++i )
               r += S.bk[ i ] < key[ q ] ? 1u : 0u;
             srt[ q ] = lo + r;
-            S.perm[ srt[ q ] ] = static_cast< uint16_t >( dst[ q ] );
+            bhi[ q ] = hi;
+            lead[ q ] = r == 0;  // certainly the first of its cell's run
+            S.sk[ srt[ q ] ] = key[ q ];
+            S.sw[ srt[ q ] ] = val[ q ];
           }
         __syncthreads();
         NG_PHASE( 4 );  // place and rank
@@ -1044,8 +1074,7 @@ __global__ void __launch_bounds__( Tile< WIN >::BS, ( MASK & WIDE_MODELS ) ? 1 :
           if ( loc[ q ] == NONE )
             continue;
           const uint32_t sc = key[ q ] >> IDX_BITS;
-          const uint32_t lo = S.bst[ loc[ q ] ], hi = S.bst[ loc[ q ] + 1 ];
-          if ( srt[ q ] > lo and ( S.bk[ S.perm[ srt[ q ] - 1 ] ] >> IDX_BITS ) == sc )
+          if ( not lead[ q ] and ( S.sk[ srt[ q ] - 1 ] >> IDX_BITS ) == sc )
           {
             loc[ q ] = NONE;  // not the first of its run
             goff[ q ] = NO_CELL;
@@ -1053,13 +1082,8 @@ __global__ void __launch_bounds__( Tile< WIN >::BS, ( MASK & WIDE_MODELS ) ? 1 :
           }
           double v = lw[ q ] ? S.win[ ci[ q ] ] : lc[ q ] ? cval[ ci[ q ] ] : cv[ q ];
           v = v + val[ q ];
-          for ( uint32_t i = srt[ q ] + 1; i < hi; ++i )
-          {
-            const uint32_t pi = S.perm[ i ];
-            if ( ( S.bk[ pi ] >> IDX_BITS ) != sc )
-              break;
-            v = v + S.bw[ pi ];
-          }
+          for ( uint32_t i = srt[ q ] + 1; i < bhi[ q ] and ( S.sk[ i ] >> IDX_BITS ) == sc; ++i )
+            v = v + S.sw[ i ];
           cv[ q ] = v;
         }
 #pragma unroll
@@ -1091,7 +1115,7 @@ __global__ void __launch_bounds__( Tile< WIN >::BS, ( MASK & WIDE_MODELS ) ? 1 :
     if ( d.rx and t < nb and rxc )
       glob( d.rx )[ dev0 + t ] += rxc;
   }
-  if ( t == 0 )
+  if ( ( MASK & BLOCK_MODELS ) != 0 and t == 0 )
     S.pool_next = BS / 4;
   __syncthreads();  // window staged and delivered
   if ( ptime and t == 0 )
@@ -1152,9 +1176,9 @@ __global__ void __launch_bounds__( Tile< WIN >::BS, ( MASK & WIDE_MODELS ) ? 1 :
       __syncthreads();
     }
     if ( d.plain_div )
-      Node::template update_block< WIN, SINGLE, false >( d, dev0, nb, C, ph, next, spk, order );
+      Node::template update_block< Cells< WIN >, SINGLE, false >( d, dev0, nb, C, ph, next, spk, order );
     else
-      Node::template update_block< WIN, SINGLE, true >( d, dev0, nb, C, ph, next, spk, order );
+      Node::template update_block< Cells< WIN >, SINGLE, true >( d, dev0, nb, C, ph, next, spk, order );
     __syncthreads();
     if ( local < nb and ( SINGLE or glob( d.model )[ dev ] == M_AEIF_COND_EXP ) )
     {
@@ -1177,9 +1201,9 @@ __global__ void __launch_bounds__( Tile< WIN >::BS, ( MASK & WIDE_MODELS ) ? 1 :
     for ( uint32_t i = t; i < n_win; i += BS )
       C.rbb[ i < before_wrap ? w0 * C.nct + i : i - before_wrap ] = S.win[ i ];
   }
-  gptr< uint32_t > cnt = glob( d.blk_cnt ) + static_cast< size_t >( par ) * P + b;
   if ( t == 0 )
   {
+    gptr< uint32_t > cnt = glob( d.blk_cnt ) + static_cast< size_t >( par ) * P + b;
     const uint32_t base = ph.from == 0 ? 0u : *cnt;  // a new slice starts an empty list
     S.cnt_base = base;
     if ( base + tot > d.spk_cap )
@@ -1201,8 +1225,7 @@ __global__ void __launch_bounds__( Tile< WIN >::BS, ( MASK & WIDE_MODELS ) ? 1 :
   {
     uint32_t o = S.cnt_base + ex;
     unsigned long long li = S.log_base + ex;
-    gptr< uint32_t > lst = glob( d.blk_spk ) + ( static_cast< size_t >( par ) * P + b ) * d.spk_cap;
-    gptr< uint8_t > lpart = glob( d.blk_part ) + ( static_cast< size_t >( par ) * P + b ) * d.spk_cap;
+    const size_t list = ( static_cast< size_t >( par ) * P + b ) * d.spk_cap;
     for ( int w = 0; w < 4; ++w )
     {
       unsigned long long x = bits[ w ];
@@ -1212,8 +1235,8 @@ __global__ void __launch_bounds__( Tile< WIN >::BS, ( MASK & WIDE_MODELS ) ? 1 :
         x &= x - 1;
         if ( o < d.spk_cap )
         {
-          lst[ o ] = ( dev << 8 ) | lag;
-          lpart[ o ] = static_cast< uint8_t >( ph.part );
+          glob( d.blk_spk )[ list + o ] = ( dev << 8 ) | lag;
+          glob( d.blk_part )[ list + o ] = static_cast< uint8_t >( ph.part );
         }
         ++o;
         if ( log_on )
@@ -1332,7 +1355,7 @@ __global__ void __launch_bounds__( FLATTEN_BS )
 // for launches with several models), which instantiates that set's slice kernels, and once
 // without NG_PART for everything else, so that the instantiations build in parallel.
 #define NG_LAUNCH_ARGS                                                                                  \
-  const NetDev *nets, const uint32_t *blk_prefix, int n_nets, uint32_t total_blocks, bool win, bool stdp, \
+  const NetDev *nets, const uint32_t *blk_prefix, int n_nets, uint32_t total_blocks, int delivery, bool stdp, \
     int s, size_t dyn_lds, hipStream_t st
 template < int MASK >
 void launch_models( NG_LAUNCH_ARGS );
@@ -1342,14 +1365,18 @@ template < int MASK >
 void
 launch_models( NG_LAUNCH_ARGS )
 {
-#define NG_LAUNCH( WIN, STDP )                                                                     \
-  k_slice< MASK, WIN, STDP ><<< total_blocks, Tile< WIN >::BS, dyn_lds, st >>>( nets, blk_prefix, n_nets, s )
-  if ( win )
-    stdp ? NG_LAUNCH( true, true ) : NG_LAUNCH( true, false );
-  else
-    stdp ? NG_LAUNCH( false, true ) : NG_LAUNCH( false, false );
+#define NG_LAUNCH( WIN, STDP, CACHE )                                                                        \
+  k_slice< MASK, WIN, STDP, CACHE >                                                                   \
+    <<< total_blocks, Tile< WIN >::BS, dyn_lds, st >>>( nets, blk_prefix, n_nets, s )
+  if ( delivery == LAUNCH_WINDOW )
+    stdp ? NG_LAUNCH( true, true, false ) : NG_LAUNCH( true, false, false );
+  else if ( delivery == LAUNCH_GLOBAL )
+    stdp ? NG_LAUNCH( false, true, false ) : NG_LAUNCH( false, false, false );
+  else if constexpr ( MASK == ALL_MODELS )
+    NG_LAUNCH( true, true, true );
 #undef NG_LAUNCH
 }
+
 template void launch_models< NG_PART >( NG_LAUNCH_ARGS );
 #else
 
@@ -1367,22 +1394,22 @@ slice_lds_for_occupancy( int wg_per_cu, bool win )
 }
 
 hipError_t
-launch_slice( const NetDev* nets, const uint32_t* blk_prefix, int n_nets, uint32_t total_blocks, int mask, bool win,
-  int s, size_t dyn_lds, hipStream_t st )
+launch_slice( const NetDev* nets, const uint32_t* blk_prefix, int n_nets, uint32_t total_blocks, int mask,
+  int delivery, int s, size_t dyn_lds, hipStream_t st )
 {
   // mask: one bit per model id of the launch, and MASK_STDP for stdp_synapse. A launch of one
   // model takes that model's own instantiation, any other the one with every model.
   const bool stdp = ( mask & MASK_STDP ) != 0;
-  switch ( mask & ALL_MODELS )
+  switch ( delivery == LAUNCH_CACHE ? ALL_MODELS : mask & ALL_MODELS )
   {
 #define NG_ONE( ID )                                                                                                \
   case 1 << ( ID ):                                                                                                 \
-    launch_models< 1 << ( ID ) >( nets, blk_prefix, n_nets, total_blocks, win, stdp, s, dyn_lds, st );              \
+    launch_models< 1 << ( ID ) >( nets, blk_prefix, n_nets, total_blocks, delivery, stdp, s, dyn_lds, st );              \
     break;
     NG_DEVICE_MODELS( NG_ONE )
 #undef NG_ONE
   default:
-    launch_models< ALL_MODELS >( nets, blk_prefix, n_nets, total_blocks, win, stdp, s, dyn_lds, st );
+    launch_models< ALL_MODELS >( nets, blk_prefix, n_nets, total_blocks, delivery, stdp, s, dyn_lds, st );
   }
   return hipGetLastError();
 }

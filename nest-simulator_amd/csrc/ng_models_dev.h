@@ -50,9 +50,9 @@ struct DeviceNode< M_IAF_PSC_DELTA >
     ch = 0;
     v = w;
   }
-  template < bool WIN >
+  template < class CELLS >
   __device__ __forceinline__ static void
-  update( const NetDev& d, gref< const ParamSet > ps, uint32_t dev, uint32_t local, const Cells< WIN >& C,
+  update( const NetDev& d, gref< const ParamSet > ps, uint32_t dev, uint32_t local, const CELLS& C,
     const SlicePhase& ph, uint64_t* bits, uint32_t mcol, int next_sample )
   {
     // models/iaf_psc_delta.cpp:272-331
@@ -127,9 +127,9 @@ struct DeviceNode< M_IAF_PSC_EXP >
     ch = w > 0 ? 1u : 0u;
     v = w;
   }
-  template < bool WIN >
+  template < class CELLS >
   __device__ __forceinline__ static void
-  update( const NetDev& d, gref< const ParamSet > ps, uint32_t dev, uint32_t local, const Cells< WIN >& C,
+  update( const NetDev& d, gref< const ParamSet > ps, uint32_t dev, uint32_t local, const CELLS& C,
     const SlicePhase& ph, uint64_t* bits, uint32_t mcol, int next_sample )
   {
     // models/iaf_psc_exp.cpp:288-349 (delta = 0: deterministic threshold)
@@ -226,9 +226,9 @@ struct DeviceNode< M_AEIF_COND_EXP >
   // 64 neurons -> this): 6,000 neurons in blocks of 32, slices of 15 steps, 520 -> 325 us per
   // slice; 48 networks in blocks of 512, 1,670 -> 1,050 us. What remains is the chain of the
   // slowest neuron, 2.5 us per attempt.
-  template < bool WIN, bool SINGLE, bool FAST >
+  template < class CELLS, bool SINGLE, bool FAST >
   __device__ __forceinline__ static void
-  update_block( const NetDev& d, uint32_t dev0, uint32_t nb, const Cells< WIN >& C, const SlicePhase& ph,
+  update_block( const NetDev& d, uint32_t dev0, uint32_t nb, const CELLS& C, const SlicePhase& ph,
     lptr< uint32_t > next, lptr< unsigned long long > spk, lptr< const uint16_t > order )
   {
     // models/aeif_cond_exp.cpp:443-523
@@ -398,9 +398,9 @@ struct DeviceNode< M_AEIF_COND_EXP >
       }
     }
   }
-  template < bool WIN >
+  template < class CELLS >
   __device__ __forceinline__ static void
-  update( const NetDev&, gref< const ParamSet >, uint32_t, uint32_t, const Cells< WIN >&, const SlicePhase&, uint64_t*,
+  update( const NetDev&, gref< const ParamSet >, uint32_t, uint32_t, const CELLS&, const SlicePhase&, uint64_t*,
     uint32_t, int )
   {
     // aeif_cond_exp neurons are updated by update_block
@@ -420,9 +420,9 @@ struct DeviceNode< M_IAF_PSC_ALPHA >
     ch = w > 0 ? 1u : 0u;
     v = w;
   }
-  template < bool WIN >
+  template < class CELLS >
   __device__ __forceinline__ static void
-  update( const NetDev& d, gref< const ParamSet > ps, uint32_t dev, uint32_t local, const Cells< WIN >& C,
+  update( const NetDev& d, gref< const ParamSet > ps, uint32_t dev, uint32_t local, const CELLS& C,
     const SlicePhase& ph, uint64_t* bits, uint32_t mcol, int next_sample )
   {
     // models/iaf_psc_alpha.cpp:305-370 (the current input y0 is zero: no current sources)
