@@ -62,6 +62,9 @@ template < class T >
 using gptr = __attribute__( ( address_space( 1 ) ) ) T*;
 template < class T >
 using gref = __attribute__( ( address_space( 1 ) ) ) T&;
+// memory that no kernel writes while this one runs: uniform addresses load into scalar registers
+template < class T >
+using cptr = __attribute__( ( address_space( 4 ) ) ) T*;
 template < class T >
 using lptr = __attribute__( ( address_space( 3 ) ) ) T*;
 template < class T >
@@ -108,6 +111,28 @@ load_rec( gptr< const SynRec > p )
   r.word = p->word;
   return r;
 }
+// four consecutive entries of a spike list with n entries left, as one load where they are in it
+struct Entries
+{
+  uint32_t x[ 4 ];
+};
+__device__ inline Entries
+load_entries( gptr< const uint32_t > p, uint32_t n )
+{
+  using v4u = __attribute__( ( ext_vector_type( 4 ), aligned( 4 ) ) ) uint32_t;
+  Entries e {};
+  if ( n >= 4 )
+  {
+    const v4u v = *( gptr< const v4u > )p;
+#pragma unroll
+    for ( int j = 0; j < 4; ++j )
+      e.x[ j ] = v[ j ];
+  }
+  else
+    for ( uint32_t j = 0; j < n; ++j )
+      e.x[ j ] = p[ j ];
+  return e;
+}
 constexpr int LB = 8;  // lags of ring-buffer input loaded together in the update
 static_assert( Tile< false >::R <= ( 1 << IDX_BITS ) and Tile< true >::R <= ( 1 << IDX_BITS ),
   "round index must fit the bucket key" );
@@ -117,6 +142,7 @@ static_assert( ( PMAX_GLOB + 1 ) * sizeof( uint32_t ) <= WIN_CAP * sizeof( doubl
 template < bool WIN >
 struct SliceLds
 {
+  static_assert( Tile< WIN >::CH <= Tile< WIN >::R, "a chunk's spikes must fit the sorted keys" );
   using T = Tile< WIN >;
   double win[ T::WINDOW ];  // ring-buffer window [slot - origin][channel][tb]
   unsigned long long log_base;
@@ -132,7 +158,8 @@ struct SliceLds
       uint32_t c_g0[ T::CH ];        // first synapse of each chunk spike's run
       uint32_t c_off[ T::CH + 1 ];   // exclusive prefix of run lengths
       uint32_t bk[ T::R ];           // event keys (slot-channel << 11 | round index), by bucket
-      uint32_t sk[ T::R ];           // event keys in sorted order
+      uint32_t sk[ T::R ];           // event keys in sorted order; before the rounds of a
+                                     // slice of one chunk its spikes
       uint32_t bcnt[ 2 ][ T::BS ];   // events per bucket, alternating between rounds
       uint16_t bst[ T::BS + 2 ];     // bucket starts
       uint16_t c_idx[ T::BS ];       // spike of every 2^sh-th event of the chunk
@@ -363,31 +390,58 @@ __device__ __forceinline__ void node_receive( int m, double w, uint32_t& ch, dou
 
 // spike_generator drive of this part: handle() of the target with weight * multiplicity.
 // Each lag adds into a different cell, so the cells of LB lags are read together.
+// The drive's parameters are read like a model's (ParamValues), its column col with the state.
+struct Drive
+{
+  int64_t t0, n_steps;
+  double w;
+  int32_t mode, delay, model;
+  PoissonCache PC;
+  __device__ __forceinline__ static Drive
+  load( const NetDev& d, bool uniform, uint32_t p0, uint32_t pi )
+  {
+    Drive v;
+    if ( uniform )
+      v.read( d, ( (cptr< const ParamSet >)d.psets )[ p0 ], (cptr< const PoissonTable >)d.ptables );
+    else
+      v.read( d, glob( d.psets )[ pi ], glob( d.ptables ) );
+    return v;
+  }
+  template < class PS, class TABLES >
+  __device__ __forceinline__ void
+  read( const NetDev& d, PS& ps, TABLES tables )
+  {
+    mode = ps.drive_mode;
+    model = ps.model;
+    t0 = ps.drive_t0;
+    n_steps = ps.drive_steps;
+    w = ps.drive_w;
+    delay = ps.drive_d;
+    if ( mode == 2 )
+    {
+      const int32_t k = ps.drive_table;
+      PC.T = glob( d.ptables ) + k;
+      PC.seed = tables[ k ].seed;
+      PC.kmax = tables[ k ].kmax;
+#pragma unroll
+      for ( int i = 0; i < KC; ++i )
+        PC.c[ i ] = tables[ k ].cdf[ i ];
+    }
+  }
+};
+
 template < class CELLS >
 __device__ inline void
-drive_adds( const NetDev& d, gref< const ParamSet > ps, int m, uint32_t dev, uint32_t local, const CELLS& C,
-  int64_t origin, int from, int stride, int to )
+drive_adds( const NetDev& d, const Drive& D, uint32_t col, int m, uint32_t local, const CELLS& C, int64_t origin,
+  int from, int stride, int to )
 {
-  const int32_t mode = ps.drive_mode;
-  if ( mode == 0 )
+  const int32_t mode = D.mode;
+  if ( mode == 0 or col == NONE )
     return;
-  const uint32_t col = glob( d.drive_idx )[ dev ];
-  if ( col == NONE )
-    return;
-  // the drive parameters in registers (the ring stores below could alias them in HBM)
-  const int64_t t0 = ps.drive_t0, n_steps = ps.drive_steps;
-  const double w = ps.drive_w;
-  const int32_t dd = ps.drive_d;
-  PoissonCache PC;
-  if ( mode == 2 )
-  {
-    PC.T = glob( d.ptables ) + ps.drive_table;
-    PC.seed = PC.T->seed;
-    PC.kmax = PC.T->kmax;
-#pragma unroll
-    for ( int i = 0; i < KC; ++i )
-      PC.c[ i ] = PC.T->cdf[ i ];
-  }
+  const int64_t t0 = D.t0, n_steps = D.n_steps;
+  const double w = D.w;
+  const int32_t dd = D.delay;
+  const PoissonCache& PC = D.PC;
   // the channel and multiplier of the weight: the model's handle( SpikeEvent& )
   uint32_t ch;
   double sw;
@@ -641,6 +695,8 @@ __global__ void __launch_bounds__( Tile< WIN >::BS, ( MASK & WIDE_MODELS ) ? 1 :
   constexpr int CH = Tile< WIN >::CH;
   constexpr int RQ = Tile< WIN >::RQ;
   constexpr int R = Tile< WIN >::R;
+  constexpr bool SINGLE = single_model< MASK >() >= 0;
+  constexpr bool EARLY = WIN;  // global delivery's larger rounds leave no registers for it
 
   // ---- which instance and block
   const uint32_t gb = n_nets > 1 ? blockIdx.x : xcd_block( blockIdx.x, gridDim.x );
@@ -687,6 +743,41 @@ __global__ void __launch_bounds__( Tile< WIN >::BS, ( MASK & WIDE_MODELS ) ? 1 :
   const int ppar = par ^ 1;
   if ( ptime and threadIdx.x == 0 )
     tp0 = wall_clock64();
+  // What the workgroup needs whatever is delivered is loaded now, so that it arrives while the
+  // window is staged and the spikes are looked up: the neurons' states, the parameter index and
+  // drive column of each thread's neuron (thread t < nb updates neuron t, the spare threads add
+  // the drive of neuron (t - nb) mod nb), and the head of the delivered spike list of block t.
+  // Loaded where they are used, one after the other, they made most of the 17 us that a slice
+  // of a small network takes (EARLY_T).
+  const uint32_t local = t;
+  const uint32_t dev = dev0 + local;
+  const uint32_t G = ( static_cast< uint32_t >( BS ) - nb ) / nb;  // groups of spare threads
+  const bool drives = local < nb ? G == 0 : local < nb + G * nb;
+  const uint32_t ddl = local < nb ? local : ( local - nb ) % nb;  // the drive thread's neuron
+  using Node1 = DeviceNode< SINGLE ? single_model< MASK >() : 0 >;
+  typename Node1::State st {};
+  uint32_t pi = 0, dcol = NONE;
+  auto load_neuron = [ & ]
+  {
+    if ( local < nb or drives )
+      pi = glob( d.pidx )[ dev0 + ddl ];
+    if ( drives )
+      dcol = glob( d.drive_idx )[ dev0 + ddl ];
+    if ( SINGLE and local < nb )
+      st = Node1::load( d, dev );
+  };
+  if ( EARLY )
+    load_neuron();
+  const bool heads = EARLY and P <= static_cast< uint32_t >( BS );  // one thread per block's list
+  const size_t my_list = ( static_cast< size_t >( ppar ) * P + t ) * d.spk_cap;
+  uint32_t my_n = 0;
+  Entries head {};
+  if ( heads and t < P and ph.deliver )
+  {
+    my_n = glob( d.blk_cnt )[ static_cast< size_t >( ppar ) * P + t ];
+    head = load_entries( glob( d.blk_spk ) + my_list, d.spk_cap );
+  }
+
   // ================================================================ 0. stage the window
   uint32_t w0 = C.s0 + C.wa;  // ring slot of the window's first slot
   if ( w0 >= C.L )
@@ -709,16 +800,41 @@ __global__ void __launch_bounds__( Tile< WIN >::BS, ( MASK & WIDE_MODELS ) ? 1 :
   // ================================================================ 1. delivery
   if ( ph.deliver )
   {
-    // prefix of per-block spike counts: an instance without a window in the window kernel
-    // (up to PMAX_GLOB blocks) keeps it in the unused window
-    uint32_t* const pref = ( WIN and not C.win and not cache ) ? reinterpret_cast< uint32_t* >( S.win ) : S.pref;
+    // prefix of per-block spike counts: an instance with more blocks than threads in the window
+    // kernel (it has no window) keeps it in the unused window
+    uint32_t* const pref = WIN and P > static_cast< uint32_t >( BS ) ? reinterpret_cast< uint32_t* >( S.win ) : S.pref;
     S.bcnt[ 0 ][ t ] = 0;
     S.bcnt[ 1 ][ t ] = 0;
     int cur = 0;  // counter buffer of the current round
     const bool flat = __builtin_amdgcn_readfirstlane( glob( d.flat_meta )[ 2 + ppar ] ) != 0;
     uint32_t K;
+    bool listed = false;  // the slice's spikes are in S.sk, in order
     if ( flat )
       K = __builtin_amdgcn_readfirstlane( glob( d.flat_meta )[ ppar ] );
+    else if ( heads )
+    {
+      uint32_t my_k;  // the first spike of block t
+      K = block_scan< BS >( my_n, &my_k, S.sh );
+      // One chunk of spikes: thread t copies block t's, whose first four it has, and no thread
+      // searches the block of its spikes. More of them are looked up chunk by chunk.
+      listed = K <= static_cast< uint32_t >( CH );
+      if ( listed )
+        for ( uint32_t i = 0; i < my_n; i += 4 )
+        {
+          const Entries e = i == 0 ? head : load_entries( glob( d.blk_spk ) + my_list + i, d.spk_cap - i );
+#pragma unroll
+          for ( uint32_t j = 0; j < 4; ++j )
+            if ( i + j < my_n )
+              S.sk[ my_k + i + j ] = e.x[ j ];
+        }
+      else
+      {
+        if ( t < P )
+          pref[ t ] = my_k;
+        if ( t == 0 )
+          pref[ P ] = K;
+      }
+    }
     else
     {
       // prefix of the per-block spike counts of the delivered slice
@@ -754,7 +870,18 @@ __global__ void __launch_bounds__( Tile< WIN >::BS, ( MASK & WIDE_MODELS ) ? 1 :
       // run [g0, g1) in the source's row; the loads of one step are independent
       uint32_t src[ SPT ], lag[ SPT ];
       const uint32_t kb = k0 + t * SPT;
-      if ( flat )
+      if ( listed )
+      {
+#pragma unroll
+        for ( int q = 0; q < SPT; ++q )
+          if ( kb + q < K )
+          {
+            const uint32_t e = S.sk[ kb + q ];
+            src[ q ] = e >> 8;
+            lag[ q ] = e & 0xffu;
+          }
+      }
+      else if ( flat )
       {
 #pragma unroll
         for ( int q = 0; q < SPT; ++q )
@@ -1126,36 +1253,40 @@ __global__ void __launch_bounds__( Tile< WIN >::BS, ( MASK & WIDE_MODELS ) ? 1 :
   // cells at least min_delay ahead (every delay, the drive's included, is >= min_delay), which
   // the update does not touch, and in distinct cells per lag: when nb <= BS / 2 the spare
   // threads add it concurrently, G groups of nb threads splitting the lags.
-  const uint32_t local = t;
-  const uint32_t dev = dev0 + local;
-  const uint32_t G = ( static_cast< uint32_t >( BS ) - nb ) / nb;
   uint64_t bits[ 4 ] = { 0, 0, 0, 0 };
-  if ( local >= nb and local < nb + G * nb )
+  if ( not EARLY )
+    load_neuron();
+  // whether the neurons of this wave's threads share one parameter set
+  const uint32_t p0 = __builtin_amdgcn_readfirstlane( pi );
+  const bool uniform = __ballot( pi != p0 and ( local < nb or drives ) ) == 0;
+  if ( local >= nb and drives )
   {
-    const uint32_t dl = ( local - nb ) % nb, g = ( local - nb ) / nb, ddev = dev0 + dl;
-    {
-      gref< const ParamSet > dps = glob( d.psets )[ glob( d.pidx )[ ddev ] ];
-      const int dm = single_model< MASK >() >= 0 ? single_model< MASK >() : dps.model;
-      drive_adds( d, dps, dm, ddev, dl, C, ph.origin, ph.from + static_cast< int >( g ), static_cast< int >( G ), ph.to );
-    }
+    const uint32_t g = ( local - nb ) / nb;
+    const Drive D = Drive::load( d, uniform, p0, pi );
+    const int dm = SINGLE ? single_model< MASK >() : D.model;
+    drive_adds( d, D, dcol, dm, ddl, C, ph.origin, ph.from + static_cast< int >( g ), static_cast< int >( G ), ph.to );
   }
   if ( local < nb )
   {
-    gref< const ParamSet > ps = glob( d.psets )[ glob( d.pidx )[ dev ] ];
     // multimeter: the next step of this part whose state is sampled (ph.to: none)
     const uint32_t mcol = d.mm_int > 0 ? glob( d.mm_col )[ dev ] : NONE;
     int next_sample = mcol != NONE ? first_sample_lag( d, ph.origin, ph.from, ph.to ) : ph.to;
-    const int m = single_model< MASK >() >= 0 ? single_model< MASK >() : ps.model;
+    const int m = SINGLE ? single_model< MASK >() : glob( d.psets )[ pi ].model;
     // Node::update of the neuron's model (each model of the launch's mask is compiled in)
-#define NG_UPDATE( ID )                                                                 \
-  if ( ( MASK & ( 1 << ( ID ) ) ) and m == ( ID ) )                                   \
-    DeviceNode< ( ID ) >::update( d, ps, dev, local, C, ph, bits, mcol, next_sample );
-    NG_DEVICE_MODELS( NG_UPDATE )
+    if constexpr ( SINGLE )
+      Node1::update( d, Node1::Params::load( d.psets, uniform, p0, pi ), st, dev, local, C, ph, bits, mcol, next_sample );
+    else
+    {
+#define NG_UPDATE( ID )                                                                                             \
+  if ( ( MASK & ( 1 << ( ID ) ) ) and m == ( ID ) )                                                               \
+    DeviceNode< ( ID ) >::update( d, DeviceNode< ( ID ) >::Params::load( d.psets, uniform, p0, pi ),              \
+      DeviceNode< ( ID ) >::load( d, dev ), dev, local, C, ph, bits, mcol, next_sample );
+      NG_DEVICE_MODELS( NG_UPDATE )
 #undef NG_UPDATE
-    if ( G == 0 )
-      drive_adds( d, ps, m, dev, local, C, ph.origin, ph.from, 1, ph.to );
+    }
+    if ( drives )
+      drive_adds( d, Drive::load( d, uniform, p0, pi ), dcol, m, local, C, ph.origin, ph.from, 1, ph.to );
   }
-  constexpr bool SINGLE = single_model< MASK >() >= 0;
   if ( ( MASK & BLOCK_MODELS ) != 0 and ( SINGLE or d.uniform_model < 0 or d.uniform_model == M_AEIF_COND_EXP ) )
   {
     // the neurons of the model that the workgroup updates together

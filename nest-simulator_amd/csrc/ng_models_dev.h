@@ -4,11 +4,12 @@
 // nest::Node gives the reference's update loop (nestkernel/node.h:297,572):
 //   - receive: handle( SpikeEvent& ) -- the ring-buffer channel an event of weight w (weight
 //     times multiplicity) goes to, and the value added there;
+//   - load: its state (fields v0..v4 and r of its device index), read when the workgroup starts;
 //   - update: update( origin, from, to ) of one neuron over the lags [ph.from, ph.to) of the
-//     slice at ph.origin: read its state (fields v0..v4 and r of its device index), consume and
-//     clear its ring-buffer cells lag by lag, set the bit of every lag it spikes in, store the
-//     multimeter samples due (store_sample at lag next_sample, then every mm_int lags) and
-//     write the state back. The parameters are the ParamSet its host half's pre_run_hook made.
+//     slice at ph.origin: consume and clear its ring-buffer cells lag by lag, set the bit of
+//     every lag it spikes in, store the multimeter samples due (store_sample at lag
+//     next_sample, then every mm_int lags) and write the state back. The parameters are the
+//     first values (Params) of the ParamSet its host half's pre_run_hook made.
 // The slice kernel dispatches on the model id (a compile-time id when a launch holds one
 // model), so every model is inlined into the fused kernel. Included by ng_kernels.hip after
 // the ring-buffer cell and sampling helpers it uses.
@@ -19,6 +20,35 @@ namespace nestgpu
 
 template < int ID >
 struct DeviceNode;
+
+// The first N values of a parameter set and its refractory steps, in registers. Neurons of a
+// wave that share one set (uniform: its index p0) read it through scalar loads, which the
+// scalar cache serves for all waves of a CU; others read their own (index pi).
+template < int N >
+struct ParamValues
+{
+  double p[ N > 0 ? N : 1 ];
+  int32_t refractory_counts;
+  __device__ __forceinline__ static ParamValues
+  load( const ParamSet* psets, bool uniform, uint32_t p0, uint32_t pi )
+  {
+    ParamValues v;
+    if ( uniform )
+      v.read( ( (cptr< const ParamSet >)psets )[ p0 ] );
+    else
+      v.read( glob( psets )[ pi ] );
+    return v;
+  }
+  template < class PS >
+  __device__ __forceinline__ void
+  read( PS& ps )
+  {
+#pragma unroll
+    for ( int q = 0; q < N; ++q )
+      p[ q ] = ps.p[ q ];
+    refractory_counts = ps.refractory_counts;
+  }
+};
 
 // The device model ids, in the order ModelManager registers them: a model with a DeviceNode
 // specialization joins the slice kernel by its entry here. WIDE marks models whose launches
@@ -50,9 +80,20 @@ struct DeviceNode< M_IAF_PSC_DELTA >
     ch = 0;
     v = w;
   }
+  struct State
+  {
+    double y3, refr_buf;  // refr_spikes_buffer_
+    int32_t r;
+  };
+  __device__ __forceinline__ static State
+  load( const NetDev& d, uint32_t dev )
+  {
+    return { glob( d.v[ 0 ] )[ dev ], glob( d.v[ 1 ] )[ dev ], glob( d.r )[ dev ] };
+  }
+  using Params = ParamValues< 9 >;
   template < class CELLS >
   __device__ __forceinline__ static void
-  update( const NetDev& d, gref< const ParamSet > ps, uint32_t dev, uint32_t local, const CELLS& C,
+  update( const NetDev& d, const Params& ps, const State& st, uint32_t dev, uint32_t local, const CELLS& C,
     const SlicePhase& ph, uint64_t* bits, uint32_t mcol, int next_sample )
   {
     // models/iaf_psc_delta.cpp:272-331
@@ -60,9 +101,9 @@ struct DeviceNode< M_IAF_PSC_DELTA >
                  V_min = ps.p[ 5 ];
     const bool refr_input = ps.p[ 6 ] != 0.0;
     const double h = ps.p[ 7 ], tau_m = ps.p[ 8 ];
-    double y3 = glob( d.v[ 0 ] )[ dev ];
-    double refr_buf = refr_input ? glob( d.v[ 1 ] )[ dev ] : 0.0;  // refr_spikes_buffer_
-    int32_t r = glob( d.r )[ dev ];
+    double y3 = st.y3;
+    double refr_buf = refr_input ? st.refr_buf : 0.0;
+    int32_t r = st.r;
     // ring-buffer cells are read LB lags at a time (independent loads), then consumed in
     // lag order and cleared
     for ( int l0 = ph.from; l0 < ph.to; l0 += LB )
@@ -127,18 +168,27 @@ struct DeviceNode< M_IAF_PSC_EXP >
     ch = w > 0 ? 1u : 0u;
     v = w;
   }
+  struct State
+  {
+    double V, iex, iin;
+    int32_t r;
+  };
+  __device__ __forceinline__ static State
+  load( const NetDev& d, uint32_t dev )
+  {
+    return { glob( d.v[ 0 ] )[ dev ], glob( d.v[ 1 ] )[ dev ], glob( d.v[ 2 ] )[ dev ], glob( d.r )[ dev ] };
+  }
+  using Params = ParamValues< 10 >;
   template < class CELLS >
   __device__ __forceinline__ static void
-  update( const NetDev& d, gref< const ParamSet > ps, uint32_t dev, uint32_t local, const CELLS& C,
+  update( const NetDev& d, const Params& ps, const State& st, uint32_t dev, uint32_t local, const CELLS& C,
     const SlicePhase& ph, uint64_t* bits, uint32_t mcol, int next_sample )
   {
     // models/iaf_psc_exp.cpp:288-349 (delta = 0: deterministic threshold)
     const double P22 = ps.p[ 0 ], P21ex = ps.p[ 1 ], P21in = ps.p[ 2 ], P20 = ps.p[ 3 ], P11ex = ps.p[ 4 ],
                  P11in = ps.p[ 5 ], IeI0 = ps.p[ 6 ], Theta = ps.p[ 7 ], V_reset = ps.p[ 8 ], exI1 = ps.p[ 9 ];
-    double V = glob( d.v[ 0 ] )[ dev ];
-    double iex = glob( d.v[ 1 ] )[ dev ];
-    double iin = glob( d.v[ 2 ] )[ dev ];
-    int32_t r = glob( d.r )[ dev ];
+    double V = st.V, iex = st.iex, iin = st.iin;
+    int32_t r = st.r;
     for ( int l0 = ph.from; l0 < ph.to; l0 += LB )
     {
       double w_in[ LB ], w_ex[ LB ];
@@ -398,12 +448,21 @@ struct DeviceNode< M_AEIF_COND_EXP >
       }
     }
   }
+  // aeif_cond_exp neurons are loaded and updated by update_block
+  struct State
+  {
+  };
+  __device__ __forceinline__ static State
+  load( const NetDev&, uint32_t )
+  {
+    return {};
+  }
+  using Params = ParamValues< 0 >;
   template < class CELLS >
   __device__ __forceinline__ static void
-  update( const NetDev&, gref< const ParamSet >, uint32_t, uint32_t, const CELLS&, const SlicePhase&, uint64_t*,
+  update( const NetDev&, const Params&, const State&, uint32_t, uint32_t, const CELLS&, const SlicePhase&, uint64_t*,
     uint32_t, int )
   {
-    // aeif_cond_exp neurons are updated by update_block
   }
 };
 
@@ -420,9 +479,21 @@ struct DeviceNode< M_IAF_PSC_ALPHA >
     ch = w > 0 ? 1u : 0u;
     v = w;
   }
+  struct State
+  {
+    double V, iex, iin, diex, diin;
+    int32_t r;
+  };
+  __device__ __forceinline__ static State
+  load( const NetDev& d, uint32_t dev )
+  {
+    return { glob( d.v[ 0 ] )[ dev ], glob( d.v[ 1 ] )[ dev ], glob( d.v[ 2 ] )[ dev ], glob( d.v[ 3 ] )[ dev ],
+      glob( d.v[ 4 ] )[ dev ], glob( d.r )[ dev ] };
+  }
+  using Params = ParamValues< 16 >;
   template < class CELLS >
   __device__ __forceinline__ static void
-  update( const NetDev& d, gref< const ParamSet > ps, uint32_t dev, uint32_t local, const CELLS& C,
+  update( const NetDev& d, const Params& ps, const State& st, uint32_t dev, uint32_t local, const CELLS& C,
     const SlicePhase& ph, uint64_t* bits, uint32_t mcol, int next_sample )
   {
     // models/iaf_psc_alpha.cpp:305-370 (the current input y0 is zero: no current sources)
@@ -430,12 +501,8 @@ struct DeviceNode< M_IAF_PSC_ALPHA >
                  P32in = ps.p[ 5 ], expm1_tau_m = ps.p[ 6 ], P21ex = ps.p[ 7 ], P11ex = ps.p[ 8 ],
                  P21in = ps.p[ 9 ], P11in = ps.p[ 10 ], EPSCInit = ps.p[ 11 ], IPSCInit = ps.p[ 12 ],
                  Theta = ps.p[ 13 ], V_reset = ps.p[ 14 ], LowerBound = ps.p[ 15 ];
-    double V = glob( d.v[ 0 ] )[ dev ];
-    double iex = glob( d.v[ 1 ] )[ dev ];
-    double iin = glob( d.v[ 2 ] )[ dev ];
-    double diex = glob( d.v[ 3 ] )[ dev ];
-    double diin = glob( d.v[ 4 ] )[ dev ];
-    int32_t r = glob( d.r )[ dev ];
+    double V = st.V, iex = st.iex, iin = st.iin, diex = st.diex, diin = st.diin;
+    int32_t r = st.r;
     // ring-buffer cells read LA lags at a time (its 16 propagators and 5 state variables
     // leave fewer registers for them than the other iaf models)
     constexpr int LA = 4;
