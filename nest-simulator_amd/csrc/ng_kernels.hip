@@ -161,7 +161,7 @@ struct SliceLds
       uint32_t sk[ T::R ];           // event keys in sorted order; before the rounds of a
                                      // slice of one chunk its spikes
       uint32_t bcnt[ 2 ][ T::BS ];   // events per bucket, alternating between rounds
-      uint16_t bst[ T::BS + 2 ];     // bucket starts
+      alignas( 4 ) uint16_t bst[ T::BS + 2 ];  // bucket starts
       uint16_t c_idx[ T::BS ];       // spike of every 2^sh-th event of the chunk
       uint8_t c_lag[ T::CH ];
     };
@@ -239,7 +239,8 @@ wave_incl_scan( uint32_t x )
   return x;
 }
 
-// block-wide exclusive scan of one value per thread; returns the total
+// block-wide exclusive scan of one value per thread; returns the total. One barrier: sh must not
+// be written again (by the next scan) before another one.
 template < int BS >
 __device__ inline uint32_t
 block_scan( uint32_t v, uint32_t* excl, uint32_t* sh )
@@ -258,7 +259,6 @@ block_scan( uint32_t v, uint32_t* excl, uint32_t* sh )
     tot += sh[ q ];
   }
   *excl = pre + x - v;
-  __syncthreads();
   return __builtin_amdgcn_readfirstlane( tot );  // the same in every thread
 }
 
@@ -784,11 +784,21 @@ __global__ void __launch_bounds__( Tile< WIN >::BS, ( MASK & WIDE_MODELS ) ? 1 :
     w0 -= C.L;
   const uint32_t n_win = C.wn * C.nct;
   const uint32_t before_wrap = ( C.L - w0 ) * C.nct;
+  auto ring_of = [ & ]( uint32_t i ) { return i < before_wrap ? w0 * C.nct + i : i - before_wrap; };
+  // four cells per thread and step, whose loads are in flight together
+  constexpr uint32_t WQ = 4;
   if ( WIN and C.win )
-  {
-    for ( uint32_t i = t; i < n_win; i += BS )
-      S.win[ i ] = C.rbb[ i < before_wrap ? w0 * C.nct + i : i - before_wrap ];
-  }
+    for ( uint32_t i0 = t; i0 < n_win; i0 += WQ * BS )
+    {
+      double x[ WQ ];
+#pragma unroll
+      for ( uint32_t q = 0; q < WQ; ++q )
+        x[ q ] = cell_load( rb_rsrc, i0 + q * BS < n_win ? ring_of( i0 + q * BS ) * 8u : NO_CELL );
+#pragma unroll
+      for ( uint32_t q = 0; q < WQ; ++q )
+        if ( i0 + q * BS < n_win )
+          S.win[ i0 + q * BS ] = x[ q ];
+    }
   // cache delivery: an empty cell cache for this slice (keys, then values, in the window area)
   const bool cache = CACHE and d.cache != 0 and ph.deliver;
   const lptr< uint32_t > ckey = ( lptr< uint32_t > )reinterpret_cast< uint32_t* >( S.win );
@@ -796,6 +806,9 @@ __global__ void __launch_bounds__( Tile< WIN >::BS, ( MASK & WIDE_MODELS ) ? 1 :
   if ( cache )
     for ( uint32_t i = t; i < CACHE_SLOTS; i += BS )
       ckey[ i ] = EMPTY_KEY;
+
+  // scratch of every other block scan: the bucket starts, which are not in use at those times
+  uint32_t* const sh1 = reinterpret_cast< uint32_t* >( S.bst );
 
   // ================================================================ 1. delivery
   if ( ph.deliver )
@@ -848,6 +861,7 @@ __global__ void __launch_bounds__( Tile< WIN >::BS, ( MASK & WIDE_MODELS ) ? 1 :
         if ( p0 + t < P )
           pref[ p0 + t ] = carry + ex;
         carry += tot;
+        __syncthreads();
       }
       if ( t == 0 )
         pref[ P ] = carry;
@@ -952,7 +966,7 @@ __global__ void __launch_bounds__( Tile< WIN >::BS, ( MASK & WIDE_MODELS ) ? 1 :
         mine += lens[ q ];
       }
       uint32_t ex;
-      const uint32_t E = block_scan< BS >( mine, &ex, S.sh );
+      const uint32_t E = block_scan< BS >( mine, &ex, sh1 );
 #pragma unroll
       for ( int q = 0; q < SPT; ++q )
       {
@@ -1300,7 +1314,7 @@ __global__ void __launch_bounds__( Tile< WIN >::BS, ( MASK & WIDE_MODELS ) ? 1 :
       // no quad starts a long one when the others are done.
       uint32_t before;
       const bool first = local < nb and Node::long_update( d, dev );
-      const uint32_t n_first = block_scan< BS >( first ? 1u : 0u, &before, S.sh );
+      const uint32_t n_first = block_scan< BS >( first ? 1u : 0u, &before, sh1 );
       if ( local < nb )
         S.order[ first ? before : n_first + local - before ] = static_cast< uint16_t >( local );
       order = ( lptr< const uint16_t > )S.order;
@@ -1458,6 +1472,7 @@ __global__ void __launch_bounds__( FLATTEN_BS )
         }
         uint32_t ex;
         const uint32_t tot = block_scan< FLATTEN_BS >( cnt, &ex, sh );
+        __syncthreads();
         uint32_t w = o + ex;
         for ( uint32_t q = 0; q < n; ++q )
         {
