@@ -313,6 +313,12 @@ struct Cells
   {
     return WIN and win and slot_rel - wa < wn;
   }
+  // every slot of [from, to) is in the window
+  __device__ bool
+  covers( int from, int to ) const
+  {
+    return WIN and win and static_cast< uint32_t >( from ) >= wa and static_cast< uint32_t >( to ) <= wa + wn;
+  }
   __device__ uint32_t
   win_index( uint32_t slot_rel, uint32_t ch, uint32_t local ) const
   {
@@ -745,15 +751,20 @@ __global__ void __launch_bounds__( Tile< WIN >::BS, ( MASK & WIDE_MODELS ) ? 1 :
     tp0 = wall_clock64();
   // What the workgroup needs whatever is delivered is loaded now, so that it arrives while the
   // window is staged and the spikes are looked up: the neurons' states, the parameter index and
-  // drive column of each thread's neuron (thread t < nb updates neuron t, the spare threads add
-  // the drive of neuron (t - nb) mod nb), and the head of the delivered spike list of block t.
-  // Loaded where they are used, one after the other, they made most of the 17 us that a slice
-  // of a small network takes (EARLY_T).
+  // drive column of each thread's neuron (thread t < nb updates neuron t, spare threads add the
+  // drive), and the head of the delivered spike list of block t.
+  // A load takes about 3,000 cycles here, and a slice of a small network is a chain of them
+  // (8-population circuit, 7,700 neurons: 16.7 -> 14.9 us per slice with these loads early).
   const uint32_t local = t;
   const uint32_t dev = dev0 + local;
-  const uint32_t G = ( static_cast< uint32_t >( BS ) - nb ) / nb;  // groups of spare threads
-  const bool drives = local < nb ? G == 0 : local < nb + G * nb;
-  const uint32_t ddl = local < nb ? local : ( local - nb ) % nb;  // the drive thread's neuron
+  // G groups of spare threads, from thread g0 on: from the next whole wave if a group fits
+  // there, so that no wave runs the update and the drive one after the other
+  uint32_t g0 = ( nb + 63u ) & ~63u;
+  if ( g0 + nb > static_cast< uint32_t >( BS ) )
+    g0 = nb;
+  const uint32_t G = ( static_cast< uint32_t >( BS ) - g0 ) / nb;
+  const bool drives = local < nb ? G == 0 : local >= g0 and local < g0 + G * nb;
+  const uint32_t ddl = local < nb ? local : drives ? ( local - g0 ) % nb : 0u;  // the drive thread's neuron
   using Node1 = DeviceNode< SINGLE ? single_model< MASK >() : 0 >;
   typename Node1::State st {};
   uint32_t pi = 0, dcol = NONE;
@@ -1266,7 +1277,8 @@ __global__ void __launch_bounds__( Tile< WIN >::BS, ( MASK & WIDE_MODELS ) ? 1 :
   // Threads [0, nb) update one neuron each. The spike_generator drive of the slice lands in
   // cells at least min_delay ahead (every delay, the drive's included, is >= min_delay), which
   // the update does not touch, and in distinct cells per lag: when nb <= BS / 2 the spare
-  // threads add it concurrently, G groups of nb threads splitting the lags.
+  // threads add it concurrently, G groups of nb threads splitting the lags (a wave that held
+  // neurons and drive threads ran the two one after the other, 4,000-6,000 cycles more).
   uint64_t bits[ 4 ] = { 0, 0, 0, 0 };
   if ( not EARLY )
     load_neuron();
@@ -1275,7 +1287,7 @@ __global__ void __launch_bounds__( Tile< WIN >::BS, ( MASK & WIDE_MODELS ) ? 1 :
   const bool uniform = __ballot( pi != p0 and ( local < nb or drives ) ) == 0;
   if ( local >= nb and drives )
   {
-    const uint32_t g = ( local - nb ) / nb;
+    const uint32_t g = ( local - g0 ) / nb;
     const Drive D = Drive::load( d, uniform, p0, pi );
     const int dm = SINGLE ? single_model< MASK >() : D.model;
     drive_adds( d, D, dcol, dm, ddl, C, ph.origin, ph.from + static_cast< int >( g ), static_cast< int >( G ), ph.to );
