@@ -229,6 +229,12 @@ nestgpu_recorder_events( nestgpu_kernel* h, int64_t recorder_id, int64_t* sender
   return guarded( h,
     [ & ]
     {
+      if ( senders == nullptr )
+      {
+        if ( n )
+          *n = static_cast< int64_t >( h->k->recorder_event_count( recorder_id ) );
+        return;
+      }
       std::vector< int64_t > s, st;
       h->k->recorder_events( recorder_id, s, st );
       if ( n )
@@ -254,6 +260,12 @@ nestgpu_multimeter_events( nestgpu_kernel* h, int64_t multimeter_id, int64_t* se
   return guarded( h,
     [ & ]
     {
+      if ( senders == nullptr )
+      {
+        if ( n )
+          *n = static_cast< int64_t >( h->k->multimeter_event_count( multimeter_id ) );
+        return;
+      }
       std::vector< int64_t > s, st;
       std::vector< double > v;
       h->k->multimeter_events( multimeter_id, s, st, v );

@@ -440,6 +440,7 @@ Kernel::reset()
   meter_gid_.clear();
   mm_col_gid_.clear();
   rec_events_.clear();
+  rec_sorted_.clear();
   conns_.assign( 1, ConnList() );
   dev_conns_.clear();
   d_min_seen_ = -1;
@@ -452,6 +453,7 @@ Kernel::reset()
   gid_to_dev_.clear();
   dev_to_gid_.clear();
   rec_events_.clear();
+  rec_sorted_.clear();
   spike_count_ = 0;
   targets_per_block_ = 0;
   balanced_blocks_ = true;
@@ -1089,13 +1091,17 @@ Kernel::collect_log()
     const auto& rec = recorders_[ r ];
     if ( rec.empty() )
       continue;
+    if ( src.empty() )
+      continue;
     const DeviceWindow& w = rec_window_[ r ];
+    // the observed senders by device index: a spike costs one byte instead of a search
+    std::vector< uint8_t > observed( dev_to_gid_.size(), 0 );
+    for ( int64_t g : rec )
+      if ( g < static_cast< int64_t >( gid_to_dev_.size() ) and gid_to_dev_[ g ] >= 0 )
+        observed[ gid_to_dev_[ g ] ] = 1;
     for ( size_t i = 0; i < src.size(); ++i )
-    {
-      const int64_t g = dev_to_gid_[ src[ i ] ];
-      if ( std::binary_search( rec.begin(), rec.end(), g ) and ( not w.set or w.active( st[ i ] ) ) )
-        rec_events_[ r ].emplace_back( st[ i ], g );
-    }
+      if ( observed[ src[ i ] ] and ( not w.set or w.active( st[ i ] ) ) )
+        rec_events_[ r ].emplace_back( st[ i ], dev_to_gid_[ src[ i ] ] );
   }
   spike_count_ += src.size();
   src.clear();
@@ -1185,9 +1191,11 @@ Kernel::multimeter_events( int64_t mm_gid, std::vector< int64_t >& senders, std:
   std::vector< size_t > order( m.ev_gid.size() );
   for ( size_t i = 0; i < order.size(); ++i )
     order[ i ] = i;
-  std::stable_sort( order.begin(), order.end(), [ &m ]( size_t a, size_t b ) {
+  auto before = [ &m ]( size_t a, size_t b ) {
     return m.ev_stamp[ a ] != m.ev_stamp[ b ] ? m.ev_stamp[ a ] < m.ev_stamp[ b ] : m.ev_gid[ a ] < m.ev_gid[ b ];
-  } );
+  };
+  if ( not std::is_sorted( order.begin(), order.end(), before ) )
+    std::stable_sort( order.begin(), order.end(), before );
   senders.resize( order.size() );
   steps.resize( order.size() );
   values.resize( order.size() * nf );
@@ -1199,6 +1207,16 @@ Kernel::multimeter_events( int64_t mm_gid, std::vector< int64_t >& senders, std:
     for ( size_t j = 0; j < nf; ++j )
       values[ e * nf + j ] = m.ev_vals[ i * nf + j ];
   }
+}
+
+size_t
+Kernel::multimeter_event_count( int64_t mm_gid )
+{
+  const NodeRec& r = node( mm_gid );
+  if ( r.kind != 3 )
+    throw std::runtime_error( "BadProperty: node is not a multimeter" );
+  collect_log();
+  return meters_[ r.idx ].ev_gid.size();
 }
 
 std::string
@@ -1258,9 +1276,48 @@ Kernel::get_values( const std::vector< int64_t >& gids, const std::string& key, 
   const bool live = engine_ and engine_->built() and simulated_;
   std::vector< double > cache[ 5 ];
   std::vector< int32_t > rcache;
+  // state fields of neurons on the device: the field per model, one read-back per field, and
+  // per neuron a gather and its offset (13 ns per value through the registry and the parameter
+  // records, 3 ms of the 24 ms that 200 ms of a 100,000-neuron network take)
+  constexpr int UNKNOWN = -2;
+  int field_of_model[ 256 ];
+  std::fill( field_of_model, field_of_model + 256, UNKNOWN );
+  if ( live and read_model_.size() != params_.size() )
+  {
+    read_model_.resize( params_.size() );
+    for ( size_t q = 0; q < params_.size(); ++q )
+      read_model_[ q ] = static_cast< uint8_t >( params_[ q ].model );
+  }
   for ( size_t i = 0; i < gids.size(); ++i )
   {
     const NodeRec& r = node( gids[ i ] );
+    if ( live and r.kind == 0 )
+    {
+      const uint8_t model = read_model_[ r.idx ];
+      int& f = field_of_model[ model ];
+      if ( f == UNKNOWN )
+      {
+        const NodeModel& M = ModelManager::instance().get( model );
+        f = M.state_field( key );
+        if ( f >= 0 )
+        {
+          if ( cache[ f ].empty() )
+            engine_->get_state( f, cache[ f ] );
+          if ( read_offset_[ f ].size() != params_.size() )
+          {
+            read_offset_[ f ].resize( params_.size() );
+            for ( size_t q = 0; q < params_.size(); ++q )
+              read_offset_[ f ][ q ] =
+                ModelManager::instance().get( params_[ q ].model ).state_offset( params_[ q ], f );
+          }
+        }
+      }
+      if ( f >= 0 )
+      {
+        out[ i ] = cache[ f ][ gid_to_dev_[ gids[ i ] ] ] + read_offset_[ f ][ r.idx ];
+        continue;
+      }
+    }
     if ( r.kind == 3 and ( key == "interval" or key == "offset" ) )
     {
       const Meter& m = meters_[ r.idx ];
@@ -1275,15 +1332,8 @@ Kernel::get_values( const std::vector< int64_t >& gids, const std::string& key, 
                                           : gens_[ r.idx ].window;
       if ( key == "n_events" )
       {
-        std::vector< int64_t > senders, steps;
-        if ( r.kind == 2 )
-          recorder_events( gids[ i ], senders, steps );
-        else
-        {
-          std::vector< double > vals;
-          multimeter_events( gids[ i ], senders, steps, vals );
-        }
-        out[ i ] = static_cast< double >( senders.size() );
+        out[ i ] = static_cast< double >(
+          r.kind == 2 ? recorder_event_count( gids[ i ] ) : multimeter_event_count( gids[ i ] ) );
       }
       else if ( key == "stop" and w.stop_inf )
         out[ i ] = std::numeric_limits< double >::infinity();
@@ -2090,6 +2140,9 @@ Kernel::prepare()
     collect_log();
     if ( host_connections_freed_ )
       throw std::runtime_error( "KernelException: the host connection table was released; cannot rebuild the device copy" );
+    read_model_.clear();
+    for ( auto& o : read_offset_ )
+      o.clear();
     BuildSpec b;
     build_spec( b );
     engine_->build( b, simulated_ );
@@ -2123,6 +2176,7 @@ Kernel::reset_device()
   rx_steps_ = 0;
   for ( auto& e : rec_events_ )
     e.clear();
+  rec_sorted_.clear();
   for ( Meter& m : meters_ )
   {
     m.ev_gid.clear();
@@ -2342,15 +2396,37 @@ Kernel::synaptic_events() const
   return engine_->read_counter( 1 );
 }
 
-void
-Kernel::recorder_events( int64_t rec_gid, std::vector< int64_t >& senders, std::vector< int64_t >& steps )
+const std::vector< std::pair< int64_t, int64_t > >&
+Kernel::sorted_events( int64_t rec_gid )
 {
   const NodeRec& r = node( rec_gid );
   if ( r.kind != 2 )
     throw std::runtime_error( "BadProperty: node is not a spike_recorder" );
   collect_log();
-  std::vector< std::pair< int64_t, int64_t > > ev = rec_events_[ r.idx ];
-  std::sort( ev.begin(), ev.end() );
+  // events arrive chunk by chunk in time: only the new ones are sorted, and merged where they
+  // reach back
+  auto& ev = rec_events_[ r.idx ];
+  rec_sorted_.resize( rec_events_.size(), 0 );
+  size_t& n = rec_sorted_[ r.idx ];
+  n = std::min( n, ev.size() );
+  const auto mid = ev.begin() + static_cast< std::ptrdiff_t >( n );
+  std::sort( mid, ev.end() );
+  if ( n > 0 and mid != ev.end() and *mid < *( mid - 1 ) )
+    std::inplace_merge( ev.begin(), mid, ev.end() );
+  n = ev.size();
+  return ev;
+}
+
+size_t
+Kernel::recorder_event_count( int64_t rec_gid )
+{
+  return sorted_events( rec_gid ).size();
+}
+
+void
+Kernel::recorder_events( int64_t rec_gid, std::vector< int64_t >& senders, std::vector< int64_t >& steps )
+{
+  const auto& ev = sorted_events( rec_gid );
   senders.resize( ev.size() );
   steps.resize( ev.size() );
   for ( size_t i = 0; i < ev.size(); ++i )

@@ -394,6 +394,8 @@ public:
   void simulate( double t_ms );
 
   // spike_recorder events (senders, stamp steps), sorted by (time, sender)
+  size_t recorder_event_count( int64_t rec_gid );
+  size_t multimeter_event_count( int64_t mm_gid );
   void recorder_events( int64_t rec_gid, std::vector< int64_t >& senders, std::vector< int64_t >& steps );
   // multimeter events sorted by (time, sender): values[i * record_from.size() + j] is the
   // value of record_from[j] of event i
@@ -587,6 +589,12 @@ private:
   // events of each spike_recorder (stamp, sender), recorded with the senders it observed and
   // the window it had when the spikes were read back
   std::vector< std::vector< std::pair< int64_t, int64_t > > > rec_events_;
+  std::vector< size_t > rec_sorted_;  // events at the front of each that are in (stamp, sender) order
+  const std::vector< std::pair< int64_t, int64_t > >& sorted_events( int64_t rec_gid );
+  // model of every neuron and, per state field once asked for, the offset its model adds to the
+  // device's values; dropped when the device copy is built (parameters change only before that)
+  std::vector< uint8_t > read_model_;
+  std::vector< double > read_offset_[ 5 ];
   uint64_t spike_count_ = 0;
   double last_kernel_ms_ = 0, last_wall_ms_ = 0;
   int slices_per_chunk_ = 64;
