@@ -459,12 +459,14 @@ Engine::clear_error_flags()
 void
 Engine::drain_log()
 {
+  if ( not net_.log_enabled )
+    return;  // without a recorder nothing is logged
   hip_check( hipSetDevice( device_ ), "hipSetDevice" );
   unsigned long long n = 0;
   hip_check( hipMemcpy( &n, net_.log_n, sizeof n, hipMemcpyDeviceToHost ), "log_n" );
   if ( n > net_.log_cap )
     throw std::runtime_error( "spike log overflow: more spikes in one chunk than the log holds" );
-  if ( not net_.log_enabled )
+  if ( n == 0 )
     return;
   const size_t old = log_src.size();
   log_src.resize( old + n );
@@ -520,8 +522,6 @@ Runner::~Runner()
     hipFree( d_prefix_ );
   if ( h_nets_ )
     hipHostFree( h_nets_ );
-  if ( d_status_ )
-    hipFree( d_status_ );
   if ( h_status_ )
     hipHostFree( h_status_ );
   for ( int q = 0; q < 2; ++q )
@@ -553,12 +553,9 @@ Runner::ensure_capacity( size_t n )
     hipFree( d_prefix_ );
   if ( h_nets_ )
     hipHostFree( h_nets_ );
-  if ( d_status_ )
-    hipFree( d_status_ );
   if ( h_status_ )
     hipHostFree( h_status_ );
   hip_check( hipMalloc( &d_nets_, n * sizeof( NetDev ) ), "hipMalloc nets" );
-  hip_check( hipMalloc( &d_status_, 2 * n * sizeof( unsigned long long ) ), "hipMalloc status" );
   hip_check( hipHostMalloc( &h_status_, 2 * n * sizeof( unsigned long long ), hipHostMallocDefault ),
     "hipHostMalloc status" );
   hip_check( hipMalloc( &d_prefix_, ( n + 1 ) * sizeof( uint32_t ) ), "hipMalloc prefix" );
@@ -867,7 +864,10 @@ Runner::run_chunk_ordered( const std::vector< Engine* >& engines, std::vector< i
   const bool graph =
     use_graph and not time_kernels and not split and slices == S_ and capture( n, total, mask, delivery );
   ++( graph ? graph_chunks : direct_chunks );
-  hip_check( hipMemcpyAsync( d_nets_, h_nets_, n * sizeof( NetDev ), hipMemcpyHostToDevice, stream_ ), "nets H2D" );
+  if ( n == 1 )
+    hip_check( launch_stage( h_nets_[ 0 ], d_nets_, stream_ ), "launch_stage" );
+  else
+    hip_check( hipMemcpyAsync( d_nets_, h_nets_, n * sizeof( NetDev ), hipMemcpyHostToDevice, stream_ ), "nets H2D" );
   hip_check( hipEventRecord( ev_chunk_[ 0 ], stream_ ), "hipEventRecord" );
   if ( not graph )
     launch_chunk_direct( h_nets_, d_nets_, n, S_, split, stream_,
@@ -875,10 +875,8 @@ Runner::run_chunk_ordered( const std::vector< Engine* >& engines, std::vector< i
   else
     hip_check( hipGraphLaunch( exec_, stream_ ), "hipGraphLaunch" );
   hip_check( hipEventRecord( ev_chunk_[ 1 ], stream_ ), "hipEventRecord" );
-  // error flags and spike-log fill of every instance in one read-back
-  hip_check( launch_status( d_nets_, n, d_status_, stream_ ), "launch_status" );
-  hip_check( hipMemcpyAsync( h_status_, d_status_, 2 * n * sizeof( unsigned long long ), hipMemcpyDeviceToHost, stream_ ),
-    "status D2H" );
+  // error flags and spike-log fill of every instance, written to host memory by the kernel
+  hip_check( launch_status( d_nets_, n, h_status_, stream_ ), "launch_status" );
   hip_check( hipStreamSynchronize( stream_ ), "hipStreamSynchronize" );
   float ms = 0;
   hipEventElapsedTime( &ms, ev_chunk_[ 0 ], ev_chunk_[ 1 ] );

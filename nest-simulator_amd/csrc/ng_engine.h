@@ -68,6 +68,8 @@ hipError_t launch_slice( const NetDev* nets, const uint32_t* blk_prefix, int n_n
 size_t slice_lds_for_occupancy( int wg_per_cu, bool win );
 // Rebuild the exact receive order of a slice that was split across Run calls.
 hipError_t launch_flatten( NetDev* net, int par, int n_parts, hipStream_t st );
+// Enqueue the copy of one launch record into device memory.
+hipError_t launch_stage( const NetDev& net, NetDev* out, hipStream_t st );
 // out[2 i] = error flags, out[2 i + 1] = spike-log fill of instance i
 hipError_t launch_status( const NetDev* nets, int n_nets, unsigned long long* out, hipStream_t st );
 
@@ -300,8 +302,7 @@ private:
   NetDev* d_nets_ = nullptr;
   NetDev* h_nets_ = nullptr;  // pinned
   uint32_t* d_prefix_ = nullptr;
-  unsigned long long* d_status_ = nullptr;
-  unsigned long long* h_status_ = nullptr;  // pinned
+  unsigned long long* h_status_ = nullptr;  // pinned, written by the device
   hipEvent_t ev_chunk_[ 2 ] = { nullptr, nullptr };
   hipEvent_t ev_kernel_[ 2 ] = { nullptr, nullptr };
   size_t cap_ = 0;
