@@ -39,15 +39,15 @@ namespace nestgpu
 constexpr int IDX_BITS = 11;  // bucket key = slot-channel << 11 | round index: sorted keys group
                               // a bucket's events by cell, in key order within each cell
 
-// Tile shape per kernel variant. The window kernel halves chunk and round so that, with its
-// ring-buffer window, two workgroups fit in the 160 KB of LDS of a CU.
+// Tile shape per kernel variant. With its ring-buffer window, two window workgroups fit in the
+// 160 KB of LDS of a CU; global delivery runs two or three (global_waves).
 template < bool WIN >
 struct Tile
 {
   static constexpr int BS = static_cast< int >( MAX_TB );  // threads per workgroup
-  static constexpr int SPT = WIN ? 2 : 4;      // spikes per thread per chunk
+  static constexpr int SPT = 2;                // spikes per thread per chunk
   static constexpr int CH = SPT * BS;          // spikes per chunk
-  static constexpr int RQ = WIN ? 2 : 4;       // events per thread per round
+  static constexpr int RQ = 2;                 // events per thread per round
   static constexpr int R = RQ * BS;            // events per round
   static constexpr uint32_t WINDOW = WIN ? WIN_CAP : 1;
   static constexpr uint32_t PMAX = WIN ? PMAX_WIN : PMAX_GLOB;
@@ -689,7 +689,8 @@ stdp_spikes( const NetDev& d, uint32_t dev, int64_t origin, uint32_t par, const 
 // serves these launches, so that the cache costs the others no registers (with it in the window
 // kernels, 389 scalar registers spilled into vector lanes).
 template < int MASK, bool WIN, bool STDP, bool CACHE >
-__global__ void __launch_bounds__( Tile< WIN >::BS, ( MASK & WIDE_MODELS ) ? 1 : 4 )
+__global__ void __launch_bounds__( Tile< WIN >::BS,
+  ( MASK & WIDE_MODELS ) ? 1 : WIN or STDP ? 4 : global_waves< MASK >() )
   k_slice( const NetDev* __restrict__ nets, const uint32_t* __restrict__ blk_prefix, int n_nets, int s )
 {
 #ifdef NG_PROFILE

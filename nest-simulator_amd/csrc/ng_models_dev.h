@@ -60,6 +60,13 @@ constexpr int N_DEVICE_MODELS = 4;
 constexpr int ALL_MODELS = ( 1 << N_DEVICE_MODELS ) - 1;
 static_assert( ALL_MODELS < MASK_STDP, "model bits must stay below the stdp bit" );
 
+// GLOBAL_WAVES: waves per SIMD of a model's global delivery kernel. That kernel serves networks
+// of more than 512 blocks, whose workgroups mostly wait for run table entries and ring cells; at
+// 6 (three workgroups per CU, 80 VGPRs) all blocks of up to 393,000 neurons are resident at once.
+// Measured per slice with rounds of 1,024 events, 4 against 6 waves (rounds of 2,048 at 4 waves
+// before): 300,000 iaf_psc_delta neurons 592 / 390 us (629), 450,000 - / 986 (1,035);
+// iaf_psc_alpha 300,000 - / 251 (385), 450,000 - / 592 (613); iaf_psc_exp, which spills 164
+// registers at 6, 300,000 195 / 174 (208), 450,000 297 / 353 (325).
 // the one model id of a launch mask with a single model bit, else -1
 template < int MASK >
 __device__ constexpr int
@@ -141,6 +148,7 @@ struct DeviceNode< M_IAF_PSC_DELTA >
 {
   static constexpr bool WIDE = false;
   static constexpr bool BLOCK = false;
+  static constexpr int GLOBAL_WAVES = 6;
   // iaf_psc_delta::handle( SpikeEvent& ) (iaf_psc_delta.cpp:332-341): one channel, the weight
   __device__ __forceinline__ static void
   receive( double w, uint32_t& ch, double& v )
@@ -216,6 +224,7 @@ struct DeviceNode< M_IAF_PSC_EXP >
 {
   static constexpr bool WIDE = false;
   static constexpr bool BLOCK = false;
+  static constexpr int GLOBAL_WAVES = 4;
   // iaf_psc_exp::handle( SpikeEvent& ) (iaf_psc_exp.cpp:351-362): positive weights to the
   // excitatory channel (1), others to the inhibitory one (0), signed
   __device__ __forceinline__ static void
@@ -282,6 +291,7 @@ struct DeviceNode< M_AEIF_COND_EXP >
 {
   static constexpr bool WIDE = false;
   static constexpr bool BLOCK = true;
+  static constexpr int GLOBAL_WAVES = 4;
   static constexpr double LONG_DT = 3.0;  // "close": within this many Delta_T below V_th
   // aeif_cond_exp::handle( SpikeEvent& ) (aeif_cond_exp.cpp:526-541): positive weights to the
   // excitatory conductance (0), others negated to the inhibitory one (1)
@@ -513,6 +523,7 @@ struct DeviceNode< M_IAF_PSC_ALPHA >
 {
   static constexpr bool WIDE = false;
   static constexpr bool BLOCK = false;
+  static constexpr int GLOBAL_WAVES = 6;
   // iaf_psc_alpha::handle( SpikeEvent& ) (iaf_psc_alpha.cpp:373-383): positive weights to
   // the excitatory channel (1), others to the inhibitory one (0), signed
   __device__ __forceinline__ static void
@@ -589,6 +600,19 @@ struct DeviceNode< M_IAF_PSC_ALPHA >
 #define NG_WIDE( ID ) | ( DeviceNode< ( ID ) >::WIDE ? ( 1 << ( ID ) ) : 0 )
 constexpr int WIDE_MODELS = 0 NG_DEVICE_MODELS( NG_WIDE );
 #undef NG_WIDE
+// waves per SIMD of the global delivery kernel of a launch mask
+template < int MASK >
+__host__ __device__ constexpr int
+global_waves()
+{
+  int waves = 4;  // several models
+#define NG_WAVES( ID )               \
+  if ( MASK == ( 1 << ( ID ) ) )   \
+    waves = DeviceNode< ( ID ) >::GLOBAL_WAVES;
+  NG_DEVICE_MODELS( NG_WAVES )
+#undef NG_WAVES
+  return waves;
+}
 // models updated by the whole workgroup
 #define NG_BLOCK( ID ) | ( DeviceNode< ( ID ) >::BLOCK ? ( 1 << ( ID ) ) : 0 )
 constexpr int BLOCK_MODELS = 0 NG_DEVICE_MODELS( NG_BLOCK );
