@@ -721,9 +721,6 @@ __global__ void __launch_bounds__( Tile< WIN >::BS,
   const SlicePhase ph = slice_phase( d, s );
   if ( not ph.active or b >= d.n_blocks )
     return;
-  // the block's targets: device indices dev0 .. dev0 + nb - 1
-  const uint32_t dev0 = __builtin_amdgcn_readfirstlane( glob( d.bstart )[ b ] );
-  const uint32_t nb = __builtin_amdgcn_readfirstlane( glob( d.bstart )[ b + 1 ] ) - dev0;
   // phase timing (counters[4..6]): thread 0 reads the 100 MHz wall clock at the start, after
   // delivery and at the end of the workgroup's work
   const bool ptime = d.phase_timing != 0;
@@ -731,6 +728,23 @@ __global__ void __launch_bounds__( Tile< WIN >::BS,
   const uint32_t P = d.n_blocks;
   const uint32_t tb = d.tb;
   const uint32_t t = threadIdx.x;
+
+  const int par = ph.parity;
+  const int ppar = par ^ 1;
+  // the first of the loads that the delivery waits for one after the other (list heads, run
+  // table, records, ring cells)
+  const bool heads = EARLY and P <= static_cast< uint32_t >( BS );  // one thread per block's list
+  const size_t my_list = ( static_cast< size_t >( ppar ) * P + t ) * d.spk_cap;
+  uint32_t my_n = 0;
+  Entries head {};
+  if ( heads and t < P and ph.deliver )
+  {
+    my_n = glob( d.blk_cnt )[ static_cast< size_t >( ppar ) * P + t ];
+    head = load_entries( glob( d.blk_spk ) + my_list, d.spk_cap );
+  }
+  // the block's targets: device indices dev0 .. dev0 + nb - 1
+  const uint32_t dev0 = __builtin_amdgcn_readfirstlane( glob( d.bstart )[ b ] );
+  const uint32_t nb = __builtin_amdgcn_readfirstlane( glob( d.bstart )[ b + 1 ] ) - dev0;
 
   Cells< WIN > C;
   C.lds = ( lptr< double > )S.win;
@@ -746,14 +760,12 @@ __global__ void __launch_bounds__( Tile< WIN >::BS,
   const __amdgpu_buffer_rsrc_t rb_rsrc = __builtin_amdgcn_make_buffer_rsrc(
     d.rb + static_cast< size_t >( b ) * C.L * C.nct, 0, static_cast< int >( C.L * C.nct * 8u ), 0x00020000 );
 
-  const int par = ph.parity;
-  const int ppar = par ^ 1;
   if ( ptime and threadIdx.x == 0 )
     tp0 = wall_clock64();
   // What the workgroup needs whatever is delivered is loaded now, so that it arrives while the
   // window is staged and the spikes are looked up: the neurons' states, the parameter index and
   // drive column of each thread's neuron (thread t < nb updates neuron t, spare threads add the
-  // drive), and the head of the delivered spike list of block t.
+  // drive).
   // A load takes about 3,000 cycles here, and a slice of a small network is a chain of them
   // (8-population circuit, 7,700 neurons: 16.7 -> 14.9 us per slice with these loads early).
   const uint32_t local = t;
@@ -780,16 +792,6 @@ __global__ void __launch_bounds__( Tile< WIN >::BS,
   };
   if ( EARLY )
     load_neuron();
-  const bool heads = EARLY and P <= static_cast< uint32_t >( BS );  // one thread per block's list
-  const size_t my_list = ( static_cast< size_t >( ppar ) * P + t ) * d.spk_cap;
-  uint32_t my_n = 0;
-  Entries head {};
-  if ( heads and t < P and ph.deliver )
-  {
-    my_n = glob( d.blk_cnt )[ static_cast< size_t >( ppar ) * P + t ];
-    head = load_entries( glob( d.blk_spk ) + my_list, d.spk_cap );
-  }
-
   // ================================================================ 0. stage the window
   uint32_t w0 = C.s0 + C.wa;  // ring slot of the window's first slot
   if ( w0 >= C.L )
