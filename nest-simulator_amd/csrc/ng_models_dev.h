@@ -77,6 +77,7 @@ single_model()
 
 // Runs step( lag, in0, in1 ) over the lags of a slice part with the neuron's input of each
 // channel, read and cleared, and collects the lags for which it returns true (a spike) in bits.
+// The lags are a serial chain: steps select instead of branching.
 // Lags whose cells are all in the LDS window take a loop of one lag per turn with the next lag's
 // input in flight; a body unrolled over LB lags was 5 KB of code fetched anew in every launch,
 // 890 cycles per lag against 540 (1,777 iaf_psc_exp, slices of ten steps, 16.5 -> 13.9 us with the
@@ -183,28 +184,24 @@ struct DeviceNode< M_IAF_PSC_DELTA >
     for_lags< LB, 1 >( C, ph, local, bits,
       [ & ]( int lag, double in, double )
       {
-        if ( r == 0 )
+        const bool active = r == 0;
+        double y = P30 * y0I + P33 * y3 + in;
+        if ( refr_input )
         {
-          y3 = P30 * y0I + P33 * y3 + in;
-          if ( refr_input and refr_buf != 0.0 )
+          if ( not active )
+            refr_buf += in * ng_exp( -static_cast< double >( r ) * h / tau_m );
+          else if ( refr_buf != 0.0 )
           {
-            y3 += refr_buf;
+            y += refr_buf;
             refr_buf = 0.0;
           }
-          y3 = ( y3 < V_min ? V_min : y3 );
         }
-        else
-        {
-          if ( refr_input )
-            refr_buf += in * ng_exp( -static_cast< double >( r ) * h / tau_m );
-          --r;
-        }
+        y = ( y < V_min ? V_min : y );
+        y3 = active ? y : y3;
+        r -= active ? 0 : 1;
         const bool spike = y3 >= V_th;
-        if ( spike )
-        {
-          r = ps.refractory_counts;
-          y3 = V_reset;
-        }
+        r = spike ? ps.refractory_counts : r;
+        y3 = spike ? V_reset : y3;
         if ( lag == next_sample )
         {
           store_sample( d, mcol, ph.origin + lag + 1, y3, 0.0, 0.0, 0.0 );
@@ -257,21 +254,18 @@ struct DeviceNode< M_IAF_PSC_EXP >
     for_lags< LB, 2 >( C, ph, local, bits,
       [ & ]( int lag, double w_in, double w_ex )
       {
-        if ( r == 0 )
-          V = V * P22 + iex * P21ex + iin * P21in + IeI0 * P20;
-        else
-          --r;
+        const bool active = r == 0;
+        const double Vn = V * P22 + iex * P21ex + iin * P21in + IeI0 * P20;
+        V = active ? Vn : V;
+        r -= active ? 0 : 1;
         iex *= P11ex;
         iin *= P11in;
         iex += exI1;
         iex += w_ex;
         iin += w_in;
         const bool spike = V >= Theta;
-        if ( spike )
-        {
-          r = ps.refractory_counts;
-          V = V_reset;
-        }
+        r = spike ? ps.refractory_counts : r;
+        V = spike ? V_reset : V;
         if ( lag == next_sample )
         {
           store_sample( d, mcol, ph.origin + lag + 1, V, iex, iin, 0.0 );
@@ -561,13 +555,10 @@ struct DeviceNode< M_IAF_PSC_ALPHA >
     for_lags< 4, 2 >( C, ph, local, bits,
       [ & ]( int lag, double w_in, double w_ex )
       {
-        if ( r == 0 )
-        {
-          V = P30 * y0I + P31ex * diex + P32ex * iex + P31in * diin + P32in * iin + expm1_tau_m * V + V;
-          V = ( V < LowerBound ? LowerBound : V );
-        }
-        else
-          --r;
+        const bool active = r == 0;
+        const double Vn = P30 * y0I + P31ex * diex + P32ex * iex + P31in * diin + P32in * iin + expm1_tau_m * V + V;
+        V = active ? ( Vn < LowerBound ? LowerBound : Vn ) : V;
+        r -= active ? 0 : 1;
         iex = P21ex * diex + P11ex * iex;  // P22_ex = P11_ex
         diex *= P11ex;
         diex += EPSCInit * w_ex;
@@ -575,11 +566,8 @@ struct DeviceNode< M_IAF_PSC_ALPHA >
         diin *= P11in;
         diin += IPSCInit * w_in;
         const bool spike = V >= Theta;
-        if ( spike )
-        {
-          r = ps.refractory_counts;
-          V = V_reset;
-        }
+        r = spike ? ps.refractory_counts : r;
+        V = spike ? V_reset : V;
         if ( lag == next_sample )
         {
           store_sample( d, mcol, ph.origin + lag + 1, V, iex, iin, 0.0 );
