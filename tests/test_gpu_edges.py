@@ -1,0 +1,153 @@
+"""The slice kernel at the sizes where its branches change, against the oracle.
+
+- aeif_cond_exp blocks below, at and above the number of lane quads (a block's neurons are then
+  taken from a pool, likely long updates first), several parameter sets in one block, slices of
+  more than 64 steps, divisors that rule out the reciprocal division, Delta_T = 0;
+- spike lists of more entries than are loaded with the counts, slices of more than one chunk of
+  spikes, more blocks than threads (global delivery), blocks of one to 512 targets (the split of
+  a target's bucket, the drive's thread groups);
+- updates whose lags lie inside and outside the LDS window, and across a 64-lag word;
+- results read between runs: two recorders and every state variable of a mixed network.
+
+iaf models: identical spikes and bit-identical state. aeif_cond_exp: identical senders, times
+within one step, states within 1e-6 relative (the repository's bar for that model).
+"""
+
+import numpy as np
+import pytest
+
+import nestgpu
+import netbuild as nb
+
+pytestmark = pytest.mark.gpu
+
+
+def _spikes_equal(sr, o, exact=True):
+    ev = sr.get("events")
+    og, os_ = nb.sorted_spikes_oracle(o)
+    print("spikes gpu=%d oracle=%d" % (len(ev["senders"]), len(og)), flush=True)
+    assert len(og) > 0
+    assert np.array_equal(ev["senders"], og)
+    assert np.max(np.abs(ev["times"] - os_ * 0.1)) <= (1e-9 if exact else 0.1 + 1e-9)
+
+
+def _run(desc, layout, fields, parts=None, exact=True):
+    k, pops, sr = nb.build_gpu(desc, layout=layout)
+    o, opops = nb.build_oracle(desc, portable_math=True)
+    for t in parts or [desc["T"]]:
+        k.Simulate(t)
+        o.simulate(t)
+    _spikes_equal(sr, o, exact)
+    for p, op in zip(pops, opops):
+        for f in fields:
+            a, b = np.atleast_1d(p.get(f)), o.get(op, f)
+            if exact:
+                assert np.array_equal(a, b), "%s: max abs diff %g" % (f, np.max(np.abs(a - b)))
+            else:
+                assert np.max(np.abs(a - b) / np.maximum(np.abs(b), 1e-12)) <= 1e-6, f
+    return k
+
+
+AEIF_FIELDS = ("V_m", "g_ex", "g_in", "w")
+
+
+@pytest.mark.parametrize("n, tb, delay", [(1, 0, 1.5), (127, 127, 1.5), (128, 128, 1.5), (129, 129, 1.5), (700, 512, 1.5),
+                                          (300, 300, 7.0)])
+def test_aeif_blocks(n, tb, delay):
+    # delay 7.0: slices of 70 steps, two words of spike bits per neuron
+    rng = np.random.default_rng(n)
+    T = 60.0
+    k = max(1, min(40, n // 4))
+    desc = dict(n_vp=2, seed=17 + n, pops=[("aeif_cond_exp", n, dict(nb.AEIF_C4))], v0={0: rng.uniform(-70.6, -48.0, n)},
+                conns=[((0, 0, n), (0, 0, n), "fixed_indegree", k, 1.5, delay)],
+                drive=[(0, rng.poisson(2.0, size=(600, n)).astype(np.uint8), 6.0, delay)], T=T)
+    _run(desc, {"targets_per_block": tb} if tb else {}, AEIF_FIELDS, exact=False)
+
+
+@pytest.mark.parametrize("change", [{"tau_w": 1e201}, {"Delta_T": 0.0}, {"C_m": 120.0, "g_L": 12.0, "E_ex": 3.0}])
+def test_aeif_parameter_sets_in_one_block(change):
+    # two populations of one block with different parameters: the first pair of values changes
+    # the division of the whole network, the second one's neurons have no spike current
+    rng = np.random.default_rng(3)
+    second = dict(nb.AEIF_C4, **change)
+    if second.get("Delta_T") == 0.0:
+        second["V_peak"] = -40.0
+    desc = dict(n_vp=1, seed=5, pops=[("aeif_cond_exp", 90, dict(nb.AEIF_C4)), ("aeif_cond_exp", 70, second)],
+                v0={0: rng.uniform(-70.6, -50.0, 90), 1: rng.uniform(-70.6, -52.0, 70)},
+                conns=[((0, 0, 90), (1, 0, 70), "fixed_indegree", 10, 2.0, 1.5),
+                       ((1, 0, 70), (0, 0, 90), "fixed_indegree", 10, -2.0, 1.5)],
+                drive=[(0, rng.poisson(2.0, size=(600, 90)).astype(np.uint8), 6.0, 1.5),
+                       (1, rng.poisson(2.0, size=(600, 70)).astype(np.uint8), 6.0, 1.5)], T=60.0)
+    _run(desc, {"targets_per_block": 160}, AEIF_FIELDS, exact=False)
+
+
+@pytest.mark.parametrize("layout", [{"targets_per_block": 1, "delivery_mode": "global"}, {"targets_per_block": 5},
+                                    {"targets_per_block": 64}, {"targets_per_block": 65}, {"targets_per_block": 257},
+                                    {"targets_per_block": 512}, {"targets_per_block": 2, "delivery_mode": "global"}],
+                         ids=lambda x: "%s%d" % (x.get("delivery_mode", "auto"), x["targets_per_block"]))
+def test_block_sizes(layout):
+    # 1 and 2 targets per block: more blocks than threads; 257 and 512: no room for a drive group
+    n = 1100 if layout["targets_per_block"] > 2 else 1030
+    _run(nb.exp_random(N=n, KE=40, KI=10, T=40.0, seed=layout["targets_per_block"]), layout,
+         ("V_m", "I_syn_ex", "I_syn_in"))
+
+
+@pytest.mark.parametrize("layout", [{"targets_per_block": 512}, {"targets_per_block": 160, "delivery_mode": "global"}, {}],
+                         ids=["win512", "global160", "auto"])
+def test_many_spikes_per_slice(layout):
+    # every neuron spikes every few steps: lists of hundreds of entries and several chunks of
+    # spikes in a slice of 20 steps
+    n, T = 1500, 30.0
+    rng = np.random.default_rng(8)
+    params = {"C_m": 1.0, "tau_m": 20.0, "V_th": 20.0, "V_reset": 10.0, "E_L": 0.0, "t_ref": 0.2}
+    desc = dict(n_vp=3, seed=4, pops=[("iaf_psc_delta", n, params)], v0={0: rng.uniform(0, 20, n)},
+                conns=[((0, 0, n), (0, 0, n), "fixed_indegree", 20, ("normal", 0.05, 0.2), ("uniform", 2.0, 3.0))],
+                drive=[(0, rng.poisson(8.0, size=(300, n)).astype(np.uint8), 0.8, 2.0)], T=T)
+    _run(desc, layout, ("V_m",))
+
+
+@pytest.mark.parametrize("model, fields", [("iaf_psc_exp", ("V_m", "I_syn_ex", "I_syn_in")),
+                                           ("iaf_psc_alpha", ("V_m", "I_syn_ex", "I_syn_in")), ("iaf_psc_delta", ("V_m",))])
+@pytest.mark.parametrize("delay, slots", [(7.0, 0), (7.0, 20), (0.1, 0)])
+def test_update_inside_and_outside_the_window(model, fields, delay, slots):
+    # delay 7.0: slices of 70 steps (two words of lags), all or 20 of their slots in LDS; parts
+    # that end inside a slice
+    n = 260
+    rng = np.random.default_rng(6)
+    params = {"tau_m": 10.0, "C_m": 250.0, "V_th": -55.0, "V_reset": -70.0, "t_ref": 2.0, "E_L": -70.0}
+    w = 90.0
+    if model == "iaf_psc_delta":
+        params, w = {"C_m": 1.0, "tau_m": 20.0, "V_th": 20.0, "V_reset": 10.0, "E_L": 0.0, "t_ref": 2.0}, 0.3
+    else:
+        params.update(tau_syn_ex=0.5, tau_syn_in=0.5)
+    lo, hi = (params["V_reset"], params["V_th"])
+    desc = dict(n_vp=2, seed=31, pops=[(model, n, params)], v0={0: rng.uniform(lo, hi, n)},
+                conns=[((0, 0, n), (0, 0, n), "fixed_indegree", 20, ("normal", w, 0.1 * w), ("uniform", delay, delay + 2.0))],
+                drive=[(0, rng.poisson(1.5, size=(420, n)).astype(np.uint8), w, delay)], T=42.0)
+    _run(desc, {"window_slots": slots} if slots else {}, fields, parts=[10.3, 7.0, 24.7])
+
+
+def test_results_read_between_runs():
+    # two recorders on parts of a mixed network, read after every run, and all state variables
+    desc = nb.mixed_models(T=60.0)
+    k, pops, sr = nb.build_gpu(desc)
+    few = k.Create("spike_recorder")
+    k.Connect(pops[1][10:60], few)
+    o, opops = nb.build_oracle(desc, portable_math=True)
+    ids = set(pops[1][10:60].tolist())
+    for t in (7.3, 20.0, 0.4, 32.3):
+        k.Simulate(t)
+        o.simulate(t)
+        og, os_ = nb.sorted_spikes_oracle(o)
+        keep = np.isin(og, list(ids))
+        for rec, g, s in ((sr, og, os_), (few, og[keep], os_[keep])):
+            ev = rec.get("events")
+            assert rec.get("n_events") == len(g) == len(ev["senders"])
+            assert np.array_equal(ev["senders"], g)
+        for p, op in zip(pops[:2], opops[:2]):
+            assert np.array_equal(np.atleast_1d(p.get("V_m")), o.get(op, "V_m"))
+        assert np.array_equal(pops[1].get("I_syn_in"), o.get(opops[1], "I_syn_in"))
+        everyone = (pops[2] + pops[0]).get("V_m")
+        assert np.array_equal(everyone[len(pops[2]):], np.atleast_1d(pops[0].get("V_m")))
+        w = o.get(opops[2], "w")
+        assert np.max(np.abs(pops[2].get("w") - w) / np.maximum(np.abs(w), 1e-12)) <= 1e-6
