@@ -134,8 +134,9 @@ load_entries( gptr< const uint32_t > p, uint32_t n )
       e.x[ j ] = v[ j ];
   }
   else
-    for ( uint32_t j = 0; j < n; ++j )
-      e.x[ j ] = p[ j ];
+#pragma unroll
+    for ( uint32_t j = 0; j < 3; ++j )
+      e.x[ j ] = j < n ? p[ j ] : 0u;
   return e;
 }
 constexpr int LB = 8;  // lags of ring-buffer input loaded together in the update
@@ -304,6 +305,7 @@ poisson_count( const PoissonCache& P, uint64_t stream, int64_t step )
 template < bool WIN >
 struct Cells
 {
+  static constexpr bool WINDOW = WIN;
   lptr< double > lds;
   gptr< double > rbb;  // block's ring: [slot][channel][tb]
   uint32_t nct;  // doubles per slot (channels * tb)

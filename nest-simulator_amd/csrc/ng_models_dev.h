@@ -82,28 +82,21 @@ single_model()
 // input in flight; a body unrolled over LB lags was 5 KB of code fetched anew in every launch,
 // 890 cycles per lag against 540 (1,777 iaf_psc_exp, slices of ten steps, 16.5 -> 13.9 us with the
 // drive in waves of its own). Cells in HBM are read LU lags at a time, so that their loads
-// overlap.
+// overlap. The words of bits are selected, not indexed: indexed, they lived in scratch memory, 24
+// bytes per thread written in every launch and read back before the spike lists (20 ms passes of
+// 1,777 iaf_psc_exp 368 -> 349 us, 60 ms of 5,000 iaf_psc_delta 934 -> 859, 200 ms of 100,000
+// iaf_psc_exp 21.4 -> 21.0 ms). The words take registers during the update, so the global delivery
+// kernels of 80 registers read half as many lags at a time (300,000 iaf_psc_delta 390 -> 382 us
+// per slice; 280,000 iaf_psc_alpha 5 % slower, all its variants spilled more).
 template < int LU, int NCH, class CELLS, class STEP >
 __device__ __forceinline__ void
 for_lags( const CELLS& C, const SlicePhase& ph, uint32_t local, uint64_t* bits, STEP&& step )
 {
-  uint64_t acc = 0;
-  auto collect = [ & ]( int lag, bool spike )
-  {
-    acc |= spike ? 1ull << ( lag & 63 ) : 0ull;
-    if ( ( lag & 63 ) == 63 or lag + 1 == ph.to )
-    {
-#pragma unroll
-      for ( int w = 0; w < 4; ++w )
-        if ( ( lag >> 6 ) == w )
-          bits[ w ] |= acc;
-      acc = 0;
-    }
-  };
   if ( C.covers( ph.from, ph.to ) )
   {
     lptr< double > p = C.lds + C.win_index( ph.from, 0, local );
     double in0 = p[ 0 ], in1 = NCH > 1 ? p[ C.tb ] : 0.0;
+    uint64_t acc = 0;  // spikes in lags [64 w, 64 w + 64) of the current lag
 #pragma unroll 1
     for ( int lag = ph.from; lag < ph.to; ++lag )
     {
@@ -118,13 +111,21 @@ for_lags( const CELLS& C, const SlicePhase& ph, uint32_t local, uint64_t* bits, 
         if ( NCH > 1 )
           in1 = p[ C.tb ];
       }
-      collect( lag, step( lag, w0, w1 ) );
+      acc |= step( lag, w0, w1 ) ? 1ull << ( lag & 63 ) : 0ull;
+      if ( ( lag & 63 ) == 63 or lag + 1 == ph.to )
+      {
+#pragma unroll
+        for ( int w = 0; w < 4; ++w )
+          bits[ w ] |= ( lag >> 6 ) == w ? acc : 0ull;
+        acc = 0;
+      }
     }
     return;
   }
   for ( int l0 = ph.from; l0 < ph.to; l0 += LU )
   {
     double w0[ LU ], w1[ LU ];
+    uint64_t acc = 0;  // spikes in lags [l0, l0 + LU)
 #pragma unroll
     for ( int q = 0; q < LU; ++q )
       if ( l0 + q < ph.to )
@@ -139,8 +140,14 @@ for_lags( const CELLS& C, const SlicePhase& ph, uint32_t local, uint64_t* bits, 
         C.put( l0 + q, 0, local, 0.0 );
         if ( NCH > 1 )
           C.put( l0 + q, 1, local, 0.0 );
-        collect( l0 + q, step( l0 + q, w0[ q ], w1[ q ] ) );
+        acc |= step( l0 + q, w0[ q ], w1[ q ] ) ? 1ull << q : 0ull;
       }
+#pragma unroll
+    for ( int w = 0; w < 4; ++w )
+    {
+      const int at = l0 - 64 * w;  // the group may cross a word
+      bits[ w ] |= at >= 64 or at <= -64 ? 0ull : at >= 0 ? acc << at : acc >> -at;
+    }
   }
 }
 
@@ -181,7 +188,7 @@ struct DeviceNode< M_IAF_PSC_DELTA >
     double y3 = st.y3;
     double refr_buf = refr_input ? st.refr_buf : 0.0;
     int32_t r = st.r;
-    for_lags< LB, 1 >( C, ph, local, bits,
+    for_lags< CELLS::WINDOW ? LB : 4, 1 >( C, ph, local, bits,
       [ & ]( int lag, double in, double )
       {
         const bool active = r == 0;
@@ -550,9 +557,9 @@ struct DeviceNode< M_IAF_PSC_ALPHA >
                  Theta = ps.p[ 13 ], V_reset = ps.p[ 14 ], LowerBound = ps.p[ 15 ];
     double V = st.V, iex = st.iex, iin = st.iin, diex = st.diex, diin = st.diin;
     int32_t r = st.r;
-    // 4 lags of cells in HBM at a time: its 16 propagators and 5 state variables leave fewer
-    // registers for them than the other iaf models
-    for_lags< 4, 2 >( C, ph, local, bits,
+    // its 16 propagators and 5 state variables leave fewer registers for cells of HBM than the
+    // other iaf models
+    for_lags< CELLS::WINDOW ? 4 : 2, 2 >( C, ph, local, bits,
       [ & ]( int lag, double w_in, double w_ex )
       {
         const bool active = r == 0;

@@ -127,6 +127,25 @@ def test_update_inside_and_outside_the_window(model, fields, delay, slots):
     _run(desc, {"window_slots": slots} if slots else {}, fields, parts=[10.3, 7.0, 24.7])
 
 
+@pytest.mark.parametrize("model", ["iaf_psc_exp", "iaf_psc_alpha", "iaf_psc_delta"])
+@pytest.mark.parametrize("layout", [{"delivery_mode": "global"}, {"window_slots": 20}, {}])
+def test_update_of_four_words_of_lags(model, layout):
+    # slices of 250 steps in parts that start at odd lags: groups of lags cross all three words
+    n = 200
+    rng = np.random.default_rng(9)
+    params = {"tau_m": 10.0, "C_m": 250.0, "V_th": -55.0, "V_reset": -70.0, "t_ref": 0.2, "E_L": -70.0}
+    w = 200.0
+    if model == "iaf_psc_delta":
+        params, w = {"C_m": 1.0, "tau_m": 20.0, "V_th": 20.0, "V_reset": 10.0, "E_L": 0.0, "t_ref": 0.2}, 1.5
+    else:
+        params.update(tau_syn_ex=0.5, tau_syn_in=0.5)
+    desc = dict(n_vp=2, seed=37, pops=[(model, n, params)], v0={0: rng.uniform(params["V_reset"], params["V_th"], n)},
+                conns=[((0, 0, n), (0, 0, n), "fixed_indegree", 10, ("normal", w, 0.1 * w), ("uniform", 25.0, 27.0))],
+                drive=[(0, rng.poisson(2.0, size=(900, n)).astype(np.uint8), w, 25.0)], T=90.0)
+    fields = ("V_m",) if model == "iaf_psc_delta" else ("V_m", "I_syn_ex", "I_syn_in")
+    _run(desc, layout, fields, parts=[5.9, 24.1, 60.0])
+
+
 def test_results_read_between_runs():
     # two recorders on parts of a mixed network, read after every run, and all state variables
     desc = nb.mixed_models(T=60.0)
