@@ -493,7 +493,7 @@ def run_plain(args, nestgpu, workload, steps, warmup, with_cpu):
         n_neurons = args.n
         drive_nz_per_step = args.n * (1.0 - np.exp(-8000.0 * 0.1e-3))
     else:
-        if args.stdp:
+        if args.stdp and args.stdp_history:
             k.SetKernelStatus({"stdp_history_capacity": args.stdp_history})
         _, n_neurons, drive_nz_per_step = build_c3(k, nestgpu, args.n_vp, args.seed, args.drive_seed,
                                                    stdp=C3_STDP if args.stdp else None)
@@ -724,7 +724,8 @@ def main():
                     help="c3: connections between excitatory populations are stdp_synapse")
     ap.add_argument("--no-c3-stdp", action="store_true",
                     help="c3: skip the extra measurement of the circuit with stdp_synapse between excitatory populations")
-    ap.add_argument("--stdp-history", type=int, default=256, help="c3 --stdp: post-spike history entries per neuron")
+    ap.add_argument("--stdp-history", type=int, default=0,
+                    help="c3 --stdp: post-spike history entries per neuron, fixed (0: grown as needed)")
     ap.add_argument("--c2-steps", type=int, default=5, help="c3: timed steps of the extra c2 measurement")
     ap.add_argument("--workload", default="c3", choices=["c2", "c3", "c4", "c5"],
                     help="c3: 77k-neuron 8-population circuit with min_delay one step (default); c2: 100k-neuron "

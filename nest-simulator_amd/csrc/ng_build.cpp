@@ -820,6 +820,7 @@ Kernel::build_spec( BuildSpec& b )
       b.tau_minus_inv[ dev_of[ i ] ] = 1. / params_[ i ].tau_minus;
   }
   b.stdp_hcap = stdp_history_;
+  b.stdp_hgrow = not stdp_history_set_;
   b.ms_per_tic = tb_.ms_per_tic;
   b.ms_per_step = tb_.ms_per_step;
   b.tics_per_step = tb_.tics_per_step;

@@ -80,10 +80,20 @@ struct alignas( 128 ) StdpPre
 // synapse record word: local target (bits 0-15), delay - min_delay (bits 16-30), stdp (bit 31)
 constexpr uint32_t PLASTIC_BIT = 0x80000000u;
 constexpr uint32_t DELAY_MASK = 0x7fffu;
-// post-spike history kept per neuron with incoming stdp synapses (ArchivingNode::history_):
-// a ring of the last stdp_hcap spikes (time, Kminus), a power of two
+// post-spike history of a neuron with incoming stdp synapses (ArchivingNode::history_): a ring
+// of its last mask + 1 spikes (time, Kminus) at hist_t / hist_k + base, a power of two of them.
+// The reference keeps every spike that some incoming synapse has yet to read; the host does the
+// same between chunks: a neuron that gets past lim spikes asks for room (REQ_HISTORY), and its
+// ring grows if its unread entries call for it. One 16-byte load gives an event all of it.
+struct alignas( 16 ) HistRing
+{
+  uint32_t n;  // spikes so far
+  uint32_t mask;
+  uint32_t base;
+  uint32_t lim;  // 0xffffffff: never asks
+};
 constexpr uint32_t STDP_HIST_DEFAULT = 256;
-constexpr uint32_t STDP_HIST_MAX = 65536;
+constexpr uint32_t STDP_HIST_MAX = 65536;  // largest capacity that can be set
 
 struct PoissonTable
 {
@@ -155,10 +165,10 @@ struct NetDev
   //      delivery work that target blocks are balanced by
   uint32_t* rx;
   // ---- stdp_synapse (stdp != 0): parameter sets, per-record state, per-neuron flags,
-  //      1/tau_minus and post-spike history [neuron][stdp_hcap] with its count, trace and last
-  //      spike time; the time base turns step stamps into ms as nest::Time does
+  //      1/tau_minus and post-spike history with its ring, trace and last spike time; the time
+  //      base turns step stamps into ms as nest::Time does
   uint32_t stdp;
-  uint32_t stdp_hcap;  // history entries per neuron, a power of two
+  uint32_t stdp_hcap;  // history entries per neuron as set, a power of two
   StdpPre* spre;             // presynaptic traces, rows [pre_row0[s], pre_row0[s + 1]) of source s
   const uint32_t* pre_row0;
   const uint32_t* srow;      // per synapse record: its trace row (stdp records only)
@@ -166,7 +176,7 @@ struct NetDev
   const double* tau_minus_inv;
   double* hist_t;
   double* hist_k;
-  uint32_t* hist_n;
+  HistRing* hist;
   double* kminus;
   double* last_spike;
   double ms_per_tic;
@@ -248,7 +258,8 @@ enum ErrorFlag : unsigned long long
   ERR_AEIF_STEPS = 16,
   ERR_SAMPLES = 32,
   ERR_STDP_HISTORY = 64,  // a post-spike history ring held too few entries for an stdp synapse
-  ERR_STDP_TWICE = 128    // a neuron with outgoing stdp synapses spiked twice in one slice
+  ERR_STDP_TWICE = 128,   // a neuron with outgoing stdp synapses spiked twice in one slice
+  REQ_HISTORY = 256       // no error: a post-spike history ring may run out of room in the next chunk
 };
 
 // First step of [from, to) whose stamp origin + lag + 1 is a sampling stamp of the instance's

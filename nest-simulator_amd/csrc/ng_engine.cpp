@@ -213,17 +213,29 @@ Engine::build_layout( const BuildSpec& b, bool keep_state, bool relayout )
     rx_ = static_cast< uint32_t* >( T( alloc( sizeof( uint32_t ) * std::max< uint32_t >( b.n, 1 ) ) ) );
     net_.rx = nullptr;
     net_.hist_t = net_.hist_k = net_.kminus = net_.last_spike = nullptr;
-    net_.hist_n = nullptr;
+    net_.hist = nullptr;
+    hist_grow_ = hist_due = false;
+    hist_span_ = 0;
+    hist_cap_.clear();
     if ( net_.stdp )
     {
       // ArchivingNode state: no history, Kminus 0, last spike -1 ms (archiving_node.cpp:38-48)
       if ( b.stdp_hcap < 2 or b.stdp_hcap > STDP_HIST_MAX or ( b.stdp_hcap & ( b.stdp_hcap - 1 ) ) )
         throw std::runtime_error( "stdp_synapse: history capacity must be a power of two in [2, 65536]" );
       net_.stdp_hcap = b.stdp_hcap;
-      const size_t nh = static_cast< size_t >( b.n ) * b.stdp_hcap;
+      hist_grow_ = b.stdp_hgrow;
+      hist_cap_.assign( b.n, 0 );
+      std::vector< HistRing > rings( b.n, HistRing { 0, 0, 0, 0xffffffffu } );
+      for ( uint32_t i = 0; i < b.n; ++i )
+        if ( b.stdp_in[ i ] )
+        {
+          hist_cap_[ i ] = b.stdp_hcap;
+          rings[ i ].mask = b.stdp_hcap - 1;
+        }
+      const size_t nh = hist_bases( rings );
       net_.hist_t = static_cast< double* >( T( alloc( sizeof( double ) * nh ) ) );
       net_.hist_k = static_cast< double* >( T( alloc( sizeof( double ) * nh ) ) );
-      net_.hist_n = static_cast< uint32_t* >( T( alloc( sizeof( uint32_t ) * b.n ) ) );
+      net_.hist = static_cast< HistRing* >( T( upload( rings ) ) );
       net_.kminus = static_cast< double* >( T( alloc( sizeof( double ) * b.n ) ) );
       net_.last_spike = static_cast< double* >( T( upload( std::vector< double >( b.n, -1.0 ) ) ) );
     }
@@ -362,6 +374,94 @@ Engine::relayout( const BuildSpec& b )
   h2d( net_.blk_spk, spk1.data(), spk1.size() * sizeof( uint32_t ) );
   h2d( net_.blk_part, part1.data(), part1.size() );
   return true;
+}
+
+// The first entry of each ring, one ring after the other by hist_cap_; returns their total.
+size_t
+Engine::hist_bases( std::vector< HistRing >& rings ) const
+{
+  size_t total = 0;
+  for ( size_t i = 0; i < rings.size(); ++i )
+  {
+    rings[ i ].base = static_cast< uint32_t >( total );
+    total += hist_cap_[ i ];
+  }
+  if ( total >= ( uint64_t( 1 ) << 32 ) )
+    throw std::runtime_error( "NotImplemented: post-spike histories of 2^32 or more entries in one instance" );
+  return total;
+}
+
+void
+Engine::make_history_room( int64_t span )
+{
+  if ( not hist_grow_ or net_.n == 0 or ( not hist_due and span <= hist_span_ ) )
+    return;
+  span = std::max( span, hist_span_ );
+  hip_check( hipSetDevice( device_ ), "hipSetDevice" );
+  const hipStream_t st = nullptr;
+  struct Scratch  // freed on every way out
+  {
+    void* p = nullptr;
+    ~Scratch()
+    {
+      if ( p )
+        hipFree( p );
+    }
+  } need, plan;
+  std::vector< HistRing > rings( net_.n );
+  hip_check( hipMalloc( &plan.p, net_.n * sizeof( HistRing ) ), "hipMalloc history plan" );
+  if ( clock > 0 or from_step > 0 )
+  {
+    hip_check( hipMalloc( &need.p, net_.n * sizeof( long long ) ), "hipMalloc history need" );
+    hip_check( hipMemsetAsync( need.p, 0x7f, net_.n * sizeof( long long ), st ), "history need" );
+    // spikes of the slice before the clock are delivered at the start of the slice at the clock
+    hip_check( launch_hist_need( net_, from_step > 0 ? clock : clock - net_.min_delay,
+                 static_cast< long long* >( need.p ), st ),
+      "launch_hist_need" );
+  }
+  HistRing* const d_plan = static_cast< HistRing* >( plan.p );
+  hip_check( launch_hist_plan( net_, static_cast< long long* >( need.p ), span, d_plan, st ), "launch_hist_plan" );
+  hip_check( hipMemcpy( rings.data(), d_plan, net_.n * sizeof( HistRing ), hipMemcpyDeviceToHost ), "history plan" );
+  bool grown = false;
+  const std::vector< uint32_t > before = hist_cap_;
+  for ( uint32_t i = 0; i < net_.n; ++i )
+    if ( hist_cap_[ i ] and rings[ i ].mask + 1 != hist_cap_[ i ] )
+    {
+      hist_cap_[ i ] = rings[ i ].mask + 1;
+      grown = true;
+    }
+  if ( not grown )
+    hip_check( hipMemcpy( net_.hist, rings.data(), net_.n * sizeof( HistRing ), hipMemcpyHostToDevice ), "history rings" );
+  else
+  {
+    double *t = nullptr, *k = nullptr;
+    try
+    {
+      const size_t total = hist_bases( rings );
+      t = static_cast< double* >( alloc( sizeof( double ) * total ) );
+      k = static_cast< double* >( alloc( sizeof( double ) * total ) );
+    }
+    catch ( ... )
+    {
+      hist_cap_ = before;
+      std::vector< void* > one( 1, t );
+      if ( t )
+        free_list( one );
+      throw;
+    }
+    hip_check( hipMemcpy( d_plan, rings.data(), net_.n * sizeof( HistRing ), hipMemcpyHostToDevice ), "history plan" );
+    hip_check( launch_hist_move( net_, d_plan, t, k, st ), "launch_hist_move" );
+    hip_check( hipStreamSynchronize( st ), "history move" );
+    std::vector< void* > old = { net_.hist_t, net_.hist_k };
+    for ( auto& q : state_allocs_ )
+      q = q == net_.hist_t ? t : q == net_.hist_k ? k : q;
+    free_list( old );
+    net_.hist_t = t;
+    net_.hist_k = k;
+    hip_check( hipMemcpy( net_.hist, rings.data(), net_.n * sizeof( HistRing ), hipMemcpyHostToDevice ), "history rings" );
+  }
+  hist_span_ = span;
+  hist_due = false;
 }
 
 void
@@ -772,10 +872,14 @@ finish_chunk( const std::vector< Engine* >& engines, const NetDev* h_nets, const
     const NetDev& d = h_nets[ i ];
     if ( not d.active )
       continue;
-    const unsigned long long flags = h_status[ 2 * i ];
+    unsigned long long flags = h_status[ 2 * i ];
+    if ( flags )
+      E.clear_error_flags();
+    if ( flags & REQ_HISTORY )
+      E.hist_due = true;
+    flags &= ~static_cast< unsigned long long >( REQ_HISTORY );
     if ( flags )
     {
-      E.clear_error_flags();
       std::string why;
       if ( flags & ERR_AEIF_INSTABILITY )
         why += " NumericalInstability in aeif_cond_exp;";
@@ -838,6 +942,9 @@ Runner::run_chunk_ordered( const std::vector< Engine* >& engines, std::vector< i
   if ( n == 0 )
     return false;
   ensure_capacity( n );
+  for ( int i = 0; i < n; ++i )
+    if ( remaining[ i ] > 0 )
+      engines[ i ]->make_history_room( static_cast< int64_t >( S_ ) * engines[ i ]->net().min_delay );
   int mask = 0;
   int delivery = LAUNCH_GLOBAL;
   bool split = false;

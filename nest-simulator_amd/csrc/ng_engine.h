@@ -70,6 +70,12 @@ size_t slice_lds_for_occupancy( int wg_per_cu, bool win );
 hipError_t launch_flatten( NetDev* net, int par, int n_parts, hipStream_t st );
 // Enqueue the copy of one launch record into device memory.
 hipError_t launch_stage( const NetDev& net, NetDev* out, hipStream_t st );
+// Post-spike history rings (HistRing) between chunks, by a launch record passed by value: the
+// earliest time each neuron's stdp synapses have yet to read from, the rings that chunks of up
+// to span steps want, and the move of the entries into them.
+hipError_t launch_hist_need( const NetDev& net, int64_t stamp0, long long* need, hipStream_t st );
+hipError_t launch_hist_plan( const NetDev& net, const long long* need, int64_t span, HistRing* plan, hipStream_t st );
+hipError_t launch_hist_move( const NetDev& net, const HistRing* plan, double* hist_t, double* hist_k, hipStream_t st );
 // out[2 i] = error flags, out[2 i + 1] = spike-log fill of instance i
 hipError_t launch_status( const NetDev* nets, int n_nets, unsigned long long* out, hipStream_t st );
 
@@ -124,6 +130,7 @@ struct BuildSpec
   std::vector< double > tau_minus_inv;
   double ms_per_tic = 0.001, ms_per_step = 0.1;
   uint32_t stdp_hcap = STDP_HIST_DEFAULT;  // post-spike history entries per neuron (power of two)
+  bool stdp_hgrow = true;                  // the rings grow with what the synapses have yet to read
   int64_t tics_per_step = 100;
   // multimeter sampling: per neuron sample column (~0 none), interval and offset in steps
   std::vector< uint32_t > mm_col;
@@ -161,6 +168,12 @@ public:
   {
     return bstart_;
   }
+
+  // Room in the post-spike history rings for a chunk of up to span steps: looked after between
+  // chunks, when a neuron asked for it (hist_due) or chunks get longer. Allocates where a ring
+  // has to grow.
+  void make_history_room( int64_t span );
+  bool hist_due = false;
 
   // weights of the synapse records in store order (stdp_synapse changes them)
   void read_weights( std::vector< double >& w ) const;
@@ -242,6 +255,7 @@ private:
   T* upload( const std::vector< T, A >& v );
   void free_list( std::vector< void* >& l );
   void build_layout( const BuildSpec& b, bool keep_state, bool relayout );
+  size_t hist_bases( std::vector< HistRing >& rings ) const;
 
   int device_;
   bool built_ = false;
@@ -251,6 +265,9 @@ private:
   std::vector< uint32_t > bstart_;  // target-block bounds of the current layout
   uint32_t* rx_ = nullptr;          // received-event counts (state allocation)
   size_t n_syn_ = 0;                // synapse records of the store
+  bool hist_grow_ = false;
+  int64_t hist_span_ = 0;            // chunk steps the rings have room for
+  std::vector< uint32_t > hist_cap_;  // entries of each neuron's ring
   std::unordered_map< void*, size_t > sizes_;  // bytes of every live allocation
   uint64_t bytes_ = 0;
 };

@@ -568,6 +568,14 @@ __device__ unsigned long long g_phase_ticks[ 8 ];
 // phase.
 constexpr double STDP_EPS = 1.0e-6;  // ConnectionManager::stdp_eps_ (connection_manager.cpp:78)
 
+__device__ inline HistRing
+load_ring( gptr< const HistRing > p )
+{
+  using v4u = __attribute__( ( ext_vector_type( 4 ) ) ) uint32_t;
+  const v4u v = *( gptr< const v4u > )p;
+  return { v[ 0 ], v[ 1 ], v[ 2 ], v[ 3 ] };
+}
+
 __device__ inline double
 stdp_event( const NetDev& d, uint32_t ridx, double w, uint32_t tdev, int64_t stamp, uint32_t dsteps, uint32_t par )
 {
@@ -580,11 +588,11 @@ stdp_event( const NetDev& d, uint32_t ridx, double w, uint32_t tdev, int64_t sta
   // ArchivingNode::get_history( t_last - d, t_spike - d ): entries t1 + eps <= t < t2 + eps
   const double t1_lim = ( t_last - dd ) + STDP_EPS;
   const double t2_lim = ( t_spike - dd ) + STDP_EPS;
-  const uint32_t n = glob( d.hist_n )[ tdev ];
-  const uint32_t cap = d.stdp_hcap, hm = cap - 1;
-  const uint32_t first = n > cap ? n - cap : 0u;  // entries before first left the ring
-  gptr< const double > ht = glob( d.hist_t ) + static_cast< size_t >( tdev ) * cap;
-  gptr< const double > hk = glob( d.hist_k ) + static_cast< size_t >( tdev ) * cap;
+  const HistRing ring = load_ring( glob( d.hist ) + tdev );
+  const uint32_t n = ring.n, hm = ring.mask;
+  const uint32_t first = n > hm ? n - hm - 1u : 0u;  // entries before first left the ring
+  gptr< const double > ht = glob( d.hist_t ) + ring.base;
+  gptr< const double > hk = glob( d.hist_k ) + ring.base;
   auto t_at = [ & ]( uint32_t i ) -> double { return ht[ i & hm ]; };
   // the times are increasing: walk back from the newest entry to the range [lo, hi) of
   // entries t1 + eps <= t < t2 + eps, so that an event costs the target spikes in its range
@@ -646,7 +654,9 @@ stdp_spikes( const NetDev& d, uint32_t dev, int64_t origin, uint32_t par, const 
   const double slice_start = d.ms_per_tic * static_cast< double >( ( origin + 1 ) * d.tics_per_step );
   int count = 0;
   double km = in ? glob( d.kminus )[ dev ] : 0.0;
-  uint32_t n = in ? glob( d.hist_n )[ dev ] : 0u;
+  HistRing ring {};
+  if ( in )
+    ring = load_ring( glob( d.hist ) + dev );
   for ( int w = 0; w < 4; ++w )
   {
     uint64_t x = bits[ w ];
@@ -661,10 +671,10 @@ stdp_spikes( const NetDev& d, uint32_t dev, int64_t origin, uint32_t par, const 
       if ( in )
       {
         km = km * ng_exp( ( last - t_sp ) * glob( d.tau_minus_inv )[ dev ] ) + 1.0;
-        const size_t at = static_cast< size_t >( dev ) * d.stdp_hcap + ( n & ( d.stdp_hcap - 1 ) );
+        const uint32_t at = ring.base + ( ring.n & ring.mask );
         glob( d.hist_t )[ at ] = t_sp;
         glob( d.hist_k )[ at ] = km;
-        ++n;
+        ++ring.n;
       }
       for ( uint32_t r = row0; r < row1; ++r )
       {
@@ -684,7 +694,9 @@ stdp_spikes( const NetDev& d, uint32_t dev, int64_t origin, uint32_t par, const 
     if ( in )
     {
       glob( d.kminus )[ dev ] = km;
-      glob( d.hist_n )[ dev ] = n;
+      glob( d.hist )[ dev ].n = ring.n;
+      if ( ring.n > ring.lim )
+        g_or( &d.counters[ 0 ], REQ_HISTORY );
     }
   }
 }
@@ -1618,6 +1630,131 @@ hipError_t
 launch_stage( const NetDev& net, NetDev* out, hipStream_t st )
 {
   k_stage<<< 1, 64, 0, st >>>( net, out );
+  return hipGetLastError();
+}
+
+// ---- room in the post-spike history rings, between chunks
+
+// doubles as signed integers of the same order
+__device__ inline long long
+ordered_key( double x )
+{
+  const long long b = __double_as_longlong( x );
+  return b < 0 ? b ^ 0x7fffffffffffffffll : b;
+}
+
+// need[t]: (as an ordered key) the least t_lastspike - delay over the stdp synapses onto t, the
+// t1 of the next get_history of each. One workgroup per source. stamp0: the source's spikes with
+// later stamps are not delivered yet; their synapses will read from the spike before.
+__global__ void
+k_hist_need( const NetDev d, int64_t stamp0, long long* need )
+{
+  const uint32_t s = blockIdx.x;
+  if ( glob( d.pre_row0 )[ s + 1 ] == glob( d.pre_row0 )[ s ] )
+    return;
+  gptr< const uint32_t > bo = glob( d.boff ) + static_cast< size_t >( s ) * ( d.n_blocks + 1 );
+  for ( uint32_t b = threadIdx.x; b < d.n_blocks; b += blockDim.x )
+  {
+    const uint32_t dev0 = glob( d.bstart )[ b ], end = bo[ b + 1 ];
+    for ( uint32_t k = bo[ b ]; k < end; ++k )
+    {
+      const uint32_t word = glob( d.syn )[ k ].word;
+      if ( not( word & PLASTIC_BIT ) )
+        continue;
+      gref< const StdpPre > pre = glob( const_cast< const StdpPre* >( d.spre ) )[ glob( d.srow )[ k ] ];
+      double t_last = pre.cur_tl;
+      const int64_t stamp = llrint( t_last / d.ms_per_step );
+      if ( stamp > stamp0 )
+        t_last = pre.tl[ ( ( stamp - 1 ) / d.min_delay ) & 1 ];
+      const uint32_t dsteps = ( ( word >> 16 ) & DELAY_MASK ) + static_cast< uint32_t >( d.min_delay );
+      __hip_atomic_fetch_min( glob( need ) + dev0 + ( word & 0xffffu ),
+        ordered_key( t_last - static_cast< double >( dsteps ) * d.ms_per_step ), __ATOMIC_RELAXED,
+        __HIP_MEMORY_SCOPE_AGENT );
+    }
+  }
+}
+
+// The ring each neuron wants for chunks of up to span steps: the entries that a synapse has yet
+// to read and the one before them (need; null: all entries), and the spikes of one chunk (a
+// neuron spikes again after its refractory steps at the earliest), in half the ring: looking
+// takes about 2 ms (21 million synapses), so a neuron asks again after half a ring of spikes.
+__global__ void
+k_hist_plan( const NetDev d, const long long* need, int64_t span, HistRing* plan )
+{
+  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+  if ( i >= d.n )
+    return;
+  HistRing r = load_ring( glob( d.hist ) + i );
+  if ( not glob( d.stdp_in )[ i ] )
+  {
+    plan[ i ] = r;
+    return;
+  }
+  uint32_t lo = r.n > r.mask ? r.n - r.mask - 1u : 0u;
+  if ( need )
+  {
+    const uint32_t first = lo;
+    uint32_t hi = r.n;
+    const long long key = glob( need )[ i ];
+    while ( lo < hi )  // the first entry at t1 + eps or later
+    {
+      const uint32_t mid = lo + ( hi - lo ) / 2;
+      const double t = glob( d.hist_t )[ r.base + ( mid & r.mask ) ];
+      if ( ordered_key( t - STDP_EPS ) >= key )
+        hi = mid;
+      else
+        lo = mid + 1;
+    }
+    // one more before it, and one for the rounding of t - eps against t1 + eps
+    lo = lo > first + 2u ? lo - 2u : first;
+  }
+  const int64_t ref = max( glob( d.psets )[ glob( d.pidx )[ i ] ].refractory_counts, 0 );
+  const uint64_t chunk = static_cast< uint64_t >( ( span + ref ) / ( ref + 1 ) );
+  const uint64_t want = r.n - lo + chunk + 1u;
+  uint64_t cap = static_cast< uint64_t >( r.mask ) + 1u;
+  while ( want > cap / 2 and cap < ( 1ull << 31 ) )
+    cap *= 2;
+  r.mask = static_cast< uint32_t >( cap - 1u );
+  const uint64_t lim = lo + cap - 1u - chunk;
+  r.lim = lim < NONE ? static_cast< uint32_t >( lim ) : NONE - 1u;
+  plan[ i ] = r;
+}
+
+// Entries into the rings of plan. One wave per neuron.
+__global__ void
+k_hist_move( const NetDev d, const HistRing* plan, double* hist_t, double* hist_k )
+{
+  const uint32_t i = ( blockIdx.x * blockDim.x + threadIdx.x ) >> 6;
+  if ( i >= d.n or not glob( d.stdp_in )[ i ] )
+    return;
+  const HistRing r = load_ring( glob( d.hist ) + i ), q = load_ring( glob( plan ) + i );
+  const uint32_t first = r.n > r.mask ? r.n - r.mask - 1u : 0u;
+  for ( uint32_t k = first + ( threadIdx.x & 63u ); k < r.n; k += 64u )
+  {
+    const uint32_t from = r.base + ( k & r.mask ), to = q.base + ( k & q.mask );
+    glob( hist_t )[ to ] = glob( d.hist_t )[ from ];
+    glob( hist_k )[ to ] = glob( d.hist_k )[ from ];
+  }
+}
+
+hipError_t
+launch_hist_need( const NetDev& net, int64_t stamp0, long long* need, hipStream_t st )
+{
+  k_hist_need<<< net.n, 256, 0, st >>>( net, stamp0, need );
+  return hipGetLastError();
+}
+
+hipError_t
+launch_hist_plan( const NetDev& net, const long long* need, int64_t span, HistRing* plan, hipStream_t st )
+{
+  k_hist_plan<<< ( net.n + 255 ) / 256, 256, 0, st >>>( net, need, span, plan );
+  return hipGetLastError();
+}
+
+hipError_t
+launch_hist_move( const NetDev& net, const HistRing* plan, double* hist_t, double* hist_k, hipStream_t st )
+{
+  k_hist_move<<< ( net.n + 3 ) / 4, 256, 0, st >>>( net, plan, hist_t, hist_k );
   return hipGetLastError();
 }
 

@@ -473,6 +473,7 @@ Kernel::reset()
   graph_chunks_ = direct_chunks_ = capture_failures_ = 0;
   window_slots_ = 0;
   stdp_history_ = STDP_HIST_DEFAULT;
+  stdp_history_set_ = false;
   delivery_passes_ = 0;
   keep_host_connections_ = true;
   host_connections_freed_ = false;
@@ -602,8 +603,9 @@ Kernel::set_kernel_status( const Json& d )
     }
     else if ( k == "stdp_history_capacity" )
     {
-      // entries of the post-spike history ring kept per neuron; NEST keeps an unbounded
-      // history (ArchivingNode::history_), a run that needs an entry the ring dropped fails
+      // entries of the post-spike history ring kept per neuron. Left alone, the rings grow with
+      // the entries their synapses have yet to read, as the reference's history does
+      // (ArchivingNode::history_); with a capacity set, a run that needs a dropped entry fails
       const double v = kv.second.number();
       const uint32_t u = static_cast< uint32_t >( v );
       if ( not( v >= 2 and v <= STDP_HIST_MAX ) or static_cast< double >( u ) != v or ( u & ( u - 1 ) ) )
@@ -611,6 +613,7 @@ Kernel::set_kernel_status( const Json& d )
       if ( simulated_ and u != stdp_history_ )
         throw std::runtime_error( "KernelException: stdp_history_capacity cannot change after Simulate" );
       stdp_history_ = u;
+      stdp_history_set_ = true;
       store_dirty_ = true;
     }
     else if ( k == "keep_host_connections" )

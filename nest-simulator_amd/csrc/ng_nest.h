@@ -601,6 +601,7 @@ private:
   int wg_per_cu_ = 0;
   int window_slots_ = 0;  // cap on the ring slots staged in LDS (0: as many as fit)
   uint32_t stdp_history_ = STDP_HIST_DEFAULT;  // post-spike history entries per neuron
+  bool stdp_history_set_ = false;              // set by the user: the rings keep that size
   int delivery_passes_ = 0;  // global delivery in this many slot-range passes (0, 1: one)
   bool time_kernels_ = false;
   bool phase_timing_ = false;

@@ -8,9 +8,8 @@ neuron states and every final weight must be bit-identical, on every delivery la
 split runs and in the batched form.
 
 This path's limits raise instead of diverging: a neuron with outgoing stdp_synapse
-connections that spikes twice within one min_delay slice, and a target whose post-spike
-history between two presynaptic spikes outgrows the entries kept per neuron
-(stdp_history_capacity).
+connections that spikes twice within one min_delay slice, and, where stdp_history_capacity is
+set, a target whose post-spike history between two presynaptic spikes outgrows it.
 """
 
 import numpy as np
@@ -200,6 +199,90 @@ def test_stdp_history_capacity():
     w = o.connections()[2]
     print("weight gpu %r oracle %r" % (c["weight"][0], w[0]), flush=True)
     assert c["weight"][0] == w[0] and w[0] != 10.0
+
+
+def _history_needed(o, opops):
+    """The most target spikes between two spikes of a source of a stdp synapse onto it, over the
+    synapses whose source spikes again (what the post-spike history has to hold)."""
+    g, st = o.spikes()
+    ids = np.concatenate(opops)
+    rank = {x: np.sort(st[g == x]) for x in ids}
+    s, t, _, d = o.connections()
+    most = 0
+    for a, b, dd in set(zip(s.tolist(), t.tolist(), d.tolist())):
+        pre, post = rank[a], rank[b]
+        if len(post) > 256 and len(pre):
+            last = np.concatenate([[0], pre[:-1]]) - dd
+            most = max(most, int((np.searchsorted(post, pre - dd) - np.searchsorted(post, last)).max()))
+    return most
+
+
+def _rare_sources(T):
+    """300 neurons: a third rarely spikes, a third spikes at about 250 Hz, the rest in between;
+    all excitatory connections are weak stdp synapses, delays 1.0-3.0 ms."""
+    desc = stdp_net(N=300, KE=25, KI=4, T=T, n_vp=3, seed=17, lam_stdp=0.01)
+    pre, post, rule, deg, _, d, aut, mult, stdp = desc["conns"][0]
+    desc["conns"][0] = (pre, post, rule, deg, ("normal", 8.0, 0.8), d, aut, mult, stdp)
+    desc["conns"][1] = desc["conns"][1][:4] + (-8.0,) + desc["conns"][1][5:]
+    rng = np.random.default_rng(23)
+    lam = np.repeat([0.62, 4.0, 0.8], 100)[rng.permutation(300)]
+    desc["drive"] = [(0, rng.poisson(lam, size=(int(round(T / 0.1)), 300)).astype(np.uint8), 87.8, 1.0)]
+    return desc
+
+
+@pytest.mark.parametrize("how", ["run", "split", "batch"])
+def test_stdp_history_grows_past_the_default(how):
+    # sources that stay silent for longer than their targets need for 256 spikes: the history
+    # grows with what its synapses have yet to read, in one Run, in Runs that end inside slices
+    # and in a batch with a network that has no plastic synapses
+    T = 2400.0
+    desc = _rare_sources(T)
+    o, opops = nb.build_oracle(desc, portable_math=True)
+    o.simulate(T)
+    need = _history_needed(o, opops)
+    print("entries needed: %d" % need, flush=True)
+    assert need > 300
+    k, pops, sr = nb.build_gpu(desc)
+    w0 = _weights_gpu(k, pops)[2].copy()
+    if how == "run":
+        k.Simulate(T)
+    elif how == "split":
+        for t in (700.3, 0.1, 899.9, T - 1600.3):
+            k.Simulate(t)
+    else:
+        other = nb.build_gpu(nb.exp_random(N=900, T=200.0, seed=5, n_vp=2))
+        nestgpu.batch_simulate([other[0], k], 1200.0)
+        nestgpu.batch_simulate([other[0], k], T - 1200.0)
+    _check(k, pops, sr, o, opops, w0)
+
+
+def test_stdp_history_grows_several_times():
+    # one silent source, one target at about 750 Hz (1,400 spikes by the source's first), one
+    # source that reads the same target all along, and a slow target
+    T, h = 2000.0, 0.1
+    counts = np.zeros((int(round(T / h)), 1), np.uint8)
+    counts[[18500, 19500], 0] = 1
+    models = [{}, {"I_e": 500.0}, {"I_e": 5000.0, "t_ref": 0.5}, {"I_e": 400.0}]
+    k = nestgpu.Kernel(0)
+    p = [k.Create("iaf_psc_exp", 1, m) for m in models]
+    o = Oracle(portable_math=True)
+    q = [o.create("iaf_psc_exp", 1, m) for m in models]
+    for a in (0, 1):
+        for b in (2, 3):
+            k.Connect(p[a], p[b], "one_to_one", {"synapse_model": "stdp_synapse", "weight": 10.0, "delay": 1.0})
+            o.connect(q[a], q[b], "one_to_one", weight=10.0, delay=1.0, stdp={})
+    sg = k.Create("spike_generator", 1)
+    k.SetSpikeCounts(sg, counts)
+    k.Connect(sg, p[0], "one_to_one", {"weight": 1e4, "delay": 1.0})
+    sr = k.Create("spike_recorder")
+    k.Connect(p[0] + p[1] + p[2] + p[3], sr)
+    o.add_drive(q[0][0], counts, 1e4, 1.0)
+    k.Simulate(T)
+    o.simulate(T)
+    need = _history_needed(o, q)
+    print("entries needed: %d" % need, flush=True)
+    assert need > 1200
+    _check(k, p, sr, o, q)
 
 
 def test_stdp_circuit_scaled():
