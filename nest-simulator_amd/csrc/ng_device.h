@@ -37,7 +37,7 @@ constexpr int MASK_STDP = 1 << 30;
 //   aeif_cond_exp: p[0]=V_peak p[1]=V_reset p[2]=g_L p[3]=C_m p[4]=E_ex p[5]=E_in p[6]=E_L
 //                  p[7]=Delta_T p[8]=tau_w p[9]=a p[10]=b p[11]=V_th p[12]=tau_syn_ex
 //                  p[13]=tau_syn_in p[14]=I_e p[15]=gsl_error_tol p[16]=V_peak_eff p[17]=h
-//                  p[18]=1 if every divisor (Delta_T or 0, C_m, the taus) is within [1e-200, 1e200]
+//                  p[18]=1 if divisions by the constants may go through their reciprocals
 // Current inputs (I0/I1, currents_) carry only CurrentEvents, which this path does not
 // produce; their zero contributions are folded into p[] so the arithmetic is unchanged.
 struct ParamSet

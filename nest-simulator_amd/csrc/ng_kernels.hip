@@ -1355,10 +1355,7 @@ __global__ void __launch_bounds__( Tile< WIN >::BS,
       order = ( lptr< const uint16_t > )S.order;
       __syncthreads();
     }
-    if ( d.plain_div )
-      Node::template update_block< Cells< WIN >, SINGLE, false >( d, dev0, nb, C, ph, next, spk, order );
-    else
-      Node::template update_block< Cells< WIN >, SINGLE, true >( d, dev0, nb, C, ph, next, spk, order );
+    Node::template update_block< Cells< WIN >, SINGLE >( d, dev0, nb, C, ph, next, spk, order );
     __syncthreads();
     if ( local < nb and ( SINGLE or glob( d.model )[ dev ] == M_AEIF_COND_EXP ) )
     {

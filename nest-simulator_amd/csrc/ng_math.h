@@ -16,8 +16,9 @@ namespace nestgpu
 // estimate a y, one residual correction by fused multiply-adds, and the hardware's fixup of
 // zeros, infinities and NaN. On the device y comes from two Newton steps, which is how a / b
 // itself is computed when neither operand needs scaling, so the result is that of a / b bit
-// for bit while |a| >= 2^-900 (or a == 0) and the quotient is far from over- and underflow.
-// 4 operations instead of 11, one of them at quarter rate.
+// for bit while |a| >= 2^-900 (or a == 0) and the quotient is far from over- and underflow; where
+// the estimate overflows the result is NaN. 4 operations instead of 11, one of them at quarter
+// rate.
 __host__ __device__ inline double
 ng_recip( double b )
 {

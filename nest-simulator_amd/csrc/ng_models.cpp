@@ -594,10 +594,14 @@ public:
       p.V_th, p.tau_ex, p.tau_in, p.I_e, p.tol, p.Delta_T > 0. ? p.V_peak : p.V_th, h };
     for ( int q = 0; q < 18; ++q )
       ps.p[ q ] = vals[ q ];
-    // whether divisions by the constants may go through their reciprocals (ng_div)
-    auto in_range = []( double x ) { return x >= 1e-200 and x <= 1e200; };
-    ps.p[ 18 ] = ( p.Delta_T == 0.0 or in_range( p.Delta_T ) ) and in_range( p.c_m ) and in_range( p.tau_w )
-        and in_range( p.tau_ex ) and in_range( p.tau_in )
+    // whether divisions by the constants may go through their reciprocals (ng_div): the
+    // parameters are 0, where they may be, or between 1e-6 and 1e6 in size (see aeif_fast_state)
+    auto in_range = []( double x ) { return std::fabs( x ) >= 1e-6 and std::fabs( x ) <= 1e6; };
+    auto in_range_or_0 = [ & ]( double x ) { return x == 0.0 or in_range( x ); };
+    ps.p[ 18 ] = in_range( p.c_m ) and in_range( p.tau_w ) and in_range( p.tau_ex ) and in_range( p.tau_in )
+        and in_range( p.E_L ) and in_range( p.g_L ) and in_range_or_0( p.Delta_T ) and in_range_or_0( p.a )
+        and in_range_or_0( p.I_e ) and in_range_or_0( p.E_ex ) and in_range_or_0( p.E_in )
+        and in_range_or_0( p.V_reset ) and in_range_or_0( p.V_peak ) and p.tol >= 1e-100
       ? 1.0
       : 0.0;
   }

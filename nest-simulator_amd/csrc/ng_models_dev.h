@@ -329,7 +329,7 @@ struct DeviceNode< M_AEIF_COND_EXP >
   // 64 neurons -> this): 6,000 neurons in blocks of 32, slices of 15 steps, 520 -> 325 us per
   // slice; 48 networks in blocks of 512, 1,670 -> 1,050 us. What remains is the chain of the
   // slowest neuron, 2.5 us per attempt.
-  template < class CELLS, bool SINGLE, bool FAST >
+  template < class CELLS, bool SINGLE >
   __device__ __forceinline__ static void
   update_block( const NetDev& d, uint32_t dev0, uint32_t nb, const CELLS& C, const SlicePhase& ph,
     lptr< uint32_t > next, lptr< unsigned long long > spk, lptr< const uint16_t > order )
@@ -340,7 +340,7 @@ struct DeviceNode< M_AEIF_COND_EXP >
     const bool channel = c == 1 or c == 2;
     const uint32_t ch = static_cast< uint32_t >( c - 1 );
     gptr< double > const vc = glob( c == 0 ? d.v[ 0 ] : c == 1 ? d.v[ 1 ] : c == 2 ? d.v[ 2 ] : d.v[ 3 ] );
-    AeifLane< FAST > A;
+    AeifLane A;
     A.c = c;
     uint32_t pset = NONE;  // parameter set in A
     double b_adapt = 0, V_peak_eff = 0, hstep = 0, I_reset = 0;
@@ -359,146 +359,172 @@ struct DeviceNode< M_AEIF_COND_EXP >
         n = __hip_atomic_fetch_add( next, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP );
       local = at( quad_bcast< 0 >( n ) );
     };
-    bool have = false;
+    bool have = false, done = false;
     // Every iteration is one attempted step of the quad's neuron, preceded by the exchange of
     // a finished neuron for the next one. More than AEIF_MAX_STEPS accepted steps within one
     // time step stop the neuron's lag and raise ERR_AEIF_STEPS, which fails the run (the
     // oracle stops with the same limit); a rejected attempt shrinks h by a factor of at most
     // 0.9 * 1.1^(-1/5) < 0.89 and is accepted once t + h rounds to t, so every quad finishes.
-    for ( ;; )
+    // integrate: the loop with divisions by reciprocals (FAST) ends, for its wave, where a neuron's
+    // state or an overflow rules them out (aeif_fast_state, aeif_finite), the one with plain
+    // divisions after at least one attempt, once it is fit again.
+    auto integrate = [ & ]( auto fast )
     {
-      if ( lag >= ph.to )
+      constexpr bool FAST = decltype( fast )::value;
+      bool tried = false;
+      for ( ;; )
       {
-        if ( have )
+        if ( lag >= ph.to )
         {
-          vc[ dev ] = y;
-          if ( c == 0 )
-            glob( d.v[ 4 ] )[ dev ] = h;
-          if ( c == 1 )
-            glob( d.r )[ dev ] = r;
-          if ( static_cast< uint32_t >( c ) < nw )
-            spk[ local * nw + c ] = bits;
-          take();
-        }
-        if ( not SINGLE )
-          while ( local < nb and glob( d.model )[ dev0 + local ] != M_AEIF_COND_EXP )
+          if ( have )
+          {
+            vc[ dev ] = y;
+            if ( c == 0 )
+              glob( d.v[ 4 ] )[ dev ] = h;
+            if ( c == 1 )
+              glob( d.r )[ dev ] = r;
+            if ( static_cast< uint32_t >( c ) < nw )
+              spk[ local * nw + c ] = bits;
             take();
-        if ( local >= nb )
-          break;
-        have = true;
-        dev = dev0 + local;
-        y = vc[ dev ];
-        h = glob( d.v[ 4 ] )[ dev ];
-        r = glob( d.r )[ dev ];
-        lag = ph.from;
-        in = channel ? C.get( lag, ch, local ) : 0.0;
-        const uint32_t pi = glob( d.pidx )[ dev ];
-        if ( d.mm_int > 0 )
-        {
-          mcol = glob( d.mm_col )[ dev ];
-          next_sample = mcol != NONE ? first_sample_lag( d, ph.origin, ph.from, ph.to ) : ph.to;
+          }
+          if ( not SINGLE )
+            while ( local < nb and glob( d.model )[ dev0 + local ] != M_AEIF_COND_EXP )
+              take();
+          if ( local >= nb )
+          {
+            done = true;
+            return;
+          }
+          have = true;
+          dev = dev0 + local;
+          y = vc[ dev ];
+          h = glob( d.v[ 4 ] )[ dev ];
+          r = glob( d.r )[ dev ];
+          lag = ph.from;
+          in = channel ? C.get( lag, ch, local ) : 0.0;
+          const uint32_t pi = glob( d.pidx )[ dev ];
+          if ( d.mm_int > 0 )
+          {
+            mcol = glob( d.mm_col )[ dev ];
+            next_sample = mcol != NONE ? first_sample_lag( d, ph.origin, ph.from, ph.to ) : ph.to;
+          }
+          if ( pi != pset )
+          {
+            pset = pi;
+            gref< const ParamSet > ps = glob( d.psets )[ pi ];
+            A.V_peak = ps.p[ 0 ];
+            A.V_reset = ps.p[ 1 ];
+            A.Delta_T = ps.p[ 7 ];
+            A.V_th = ps.p[ 11 ];
+            A.I_e = ps.p[ 14 ];
+            A.tol = ps.p[ 15 ];
+            A.gD = ps.p[ 2 ] * ps.p[ 7 ];
+            A.E = ps.p[ c == 1 ? 4 : c == 2 ? 5 : 6 ];
+            A.m = c == 0 ? -ps.p[ 2 ] : ps.p[ 9 ];
+            A.zero_fits = channel or ( c == 3 and ps.p[ 9 ] == 0.0 );
+            A.den = ps.p[ c == 0 ? 3 : c == 1 ? 12 : c == 2 ? 13 : 8 ];
+            A.r_den = ng_recip( A.den );
+            A.r_Delta_T = ng_recip( A.Delta_T );
+            b_adapt = ps.p[ 10 ];
+            V_peak_eff = ps.p[ 16 ];
+            hstep = ps.p[ 17 ];
+            refractory_counts = ps.refractory_counts;
+            I_reset = aeif_spike_current< FAST >( A, aeif_V( A, false, A.V_reset ) );
+          }
+          tt = 0.0;
+          guard = 0;
+          bits = 0;
+          I_spk = aeif_spike_current< FAST >( A, aeif_V( A, false, quad_bcast< 0 >( y ) ) );
         }
-        if ( pi != pset )
+        // the derivative at the step's start: its spike current is the one the last step ended
+        // with, or that of the reset potential (inputs change the conductances only)
+        const bool refr = r > 0;
+        const double dt = hstep - tt;
+        const bool final_step = h > dt;
+        const double h_old = final_step ? dt : h;
+        const double k1 = aeif_dynamics< FAST >( A, refr, aeif_V( A, refr, quad_bcast< 0 >( y ) ), I_spk, y );
+        // looked at behind k1, as the end of the step behind its control, which hides the latency
+        const bool unfit = __any( not aeif_fast_state( A, y ) );
+        if ( FAST ? unfit : tried and not unfit and not d.plain_div )
+          return;
+        tried = true;
+        double yerr, yp, I_end;
+        const double y1 = aeif_rkf45_step< FAST >( A, refr, y, h_old, k1, yerr, yp, I_end );
+        const double tn = final_step ? hstep : tt + h_old;
+        double h_new = h_old;
+        const int st = aeif_yp_hadjust( A.tol, yerr, yp, &h_new );
+        if ( FAST and __any( not aeif_finite( y1, yp ) ) )
+          return;
+        h = h_new;
+        if ( st < 0 )
         {
-          pset = pi;
-          gref< const ParamSet > ps = glob( d.psets )[ pi ];
-          A.V_peak = ps.p[ 0 ];
-          A.V_reset = ps.p[ 1 ];
-          A.Delta_T = ps.p[ 7 ];
-          A.V_th = ps.p[ 11 ];
-          A.I_e = ps.p[ 14 ];
-          A.tol = ps.p[ 15 ];
-          A.gD = ps.p[ 2 ] * ps.p[ 7 ];
-          A.E = ps.p[ c == 1 ? 4 : c == 2 ? 5 : 6 ];
-          A.m = c == 0 ? -ps.p[ 2 ] : ps.p[ 9 ];
-          A.den = ps.p[ c == 0 ? 3 : c == 1 ? 12 : c == 2 ? 13 : 8 ];
-          A.r_den = ng_recip( A.den );
-          A.r_Delta_T = ng_recip( A.Delta_T );
-          b_adapt = ps.p[ 10 ];
-          V_peak_eff = ps.p[ 16 ];
-          hstep = ps.p[ 17 ];
-          refractory_counts = ps.refractory_counts;
-          I_reset = aeif_spike_current( A, aeif_V( A, false, A.V_reset ) );
+          if ( fabs( h_new ) < fabs( h_old ) and tn + h_new != tn )
+            continue;  // again from the same state
+          h = h_old;
         }
-        tt = 0.0;
-        guard = 0;
-        bits = 0;
-        I_spk = aeif_spike_current( A, aeif_V( A, false, quad_bcast< 0 >( y ) ) );
-      }
-      // the derivative at the step's start: its spike current is the one the last step ended
-      // with, or that of the reset potential (inputs change the conductances only)
-      const bool refr = r > 0;
-      const double k1 = aeif_dynamics( A, refr, aeif_V( A, refr, quad_bcast< 0 >( y ) ), I_spk, y );
-      const double dt = hstep - tt;
-      const bool final_step = h > dt;
-      const double h_old = final_step ? dt : h;
-      double yerr, yp, I_end;
-      const double y1 = aeif_rkf45_step( A, refr, y, h_old, k1, yerr, yp, I_end );
-      const double tn = final_step ? hstep : tt + h_old;
-      double h_new = h_old;
-      const int st = aeif_yp_hadjust( A.tol, yerr, yp, &h_new );
-      h = h_new;
-      if ( st < 0 )
-      {
-        if ( fabs( h_new ) < fabs( h_old ) and tn + h_new != tn )
-          continue;  // again from the same state
-        h = h_old;
-      }
-      y = y1;
-      I_spk = I_end;
-      tt = tn;
-      ++guard;
-      const double V = quad_bcast< 0 >( y ), w = quad_bcast< 3 >( y );
-      if ( V < -1e3 or w < -1e6 or w > 1e6 )
-      {
-        if ( c == 0 )
-          g_or( &d.counters[ 0 ], ERR_AEIF_INSTABILITY );
-        tt = hstep;
-      }
-      else if ( r > 0 )
-      {
-        y = c == 0 ? A.V_reset : y;
-        I_spk = I_reset;
-      }
-      else if ( V >= V_peak_eff )
-      {
-        y = c == 0 ? A.V_reset : c == 3 ? y + b_adapt : y;
-        I_spk = I_reset;
-        r = refractory_counts > 0 ? refractory_counts + 1 : 0;
-        if ( ( lag >> 6 ) == c )
+        y = y1;
+        I_spk = I_end;
+        tt = tn;
+        ++guard;
+        const double V = quad_bcast< 0 >( y ), w = quad_bcast< 3 >( y );
+        if ( V < -1e3 or w < -1e6 or w > 1e6 )
         {
-          const unsigned long long bit = 1ull << ( lag & 63 );
-          if ( bits & bit )
-            g_or( &d.counters[ 0 ], ERR_AEIF_DOUBLE_SPIKE );
-          bits |= bit;
+          if ( c == 0 )
+            g_or( &d.counters[ 0 ], ERR_AEIF_INSTABILITY );
+          tt = hstep;
         }
-      }
-      if ( tt < hstep and guard >= AEIF_MAX_STEPS )
-      {
-        if ( c == 0 )
-          g_or( &d.counters[ 0 ], ERR_AEIF_STEPS );
-        tt = hstep;
-      }
-      if ( not( tt < hstep ) )
-      {
-        if ( r > 0 )
-          --r;
-        if ( channel )
+        else if ( r > 0 )
         {
-          y += in;
-          C.put( lag, ch, local, 0.0 );
+          y = c == 0 ? A.V_reset : y;
+          I_spk = I_reset;
         }
-        if ( lag == next_sample )
+        else if ( V >= V_peak_eff )
         {
-          store_sample_field( d, mcol, ph.origin + lag + 1, c, y );
-          next_sample += d.mm_int;
+          y = c == 0 ? A.V_reset : c == 3 ? y + b_adapt : y;
+          I_spk = I_reset;
+          r = refractory_counts > 0 ? refractory_counts + 1 : 0;
+          if ( ( lag >> 6 ) == c )
+          {
+            const unsigned long long bit = 1ull << ( lag & 63 );
+            if ( bits & bit )
+              g_or( &d.counters[ 0 ], ERR_AEIF_DOUBLE_SPIKE );
+            bits |= bit;
+          }
         }
-        ++lag;
-        tt = 0.0;
-        guard = 0;
-        if ( channel and lag < ph.to )
-          in = C.get( lag, ch, local );  // arrives while the lag is integrated
+        if ( tt < hstep and guard >= AEIF_MAX_STEPS )
+        {
+          if ( c == 0 )
+            g_or( &d.counters[ 0 ], ERR_AEIF_STEPS );
+          tt = hstep;
+        }
+        if ( not( tt < hstep ) )
+        {
+          if ( r > 0 )
+            --r;
+          if ( channel )
+          {
+            y += in;
+            C.put( lag, ch, local, 0.0 );
+          }
+          if ( lag == next_sample )
+          {
+            store_sample_field( d, mcol, ph.origin + lag + 1, c, y );
+            next_sample += d.mm_int;
+          }
+          ++lag;
+          tt = 0.0;
+          guard = 0;
+          if ( channel and lag < ph.to )
+            in = C.get( lag, ch, local );  // arrives while the lag is integrated
+        }
       }
+    };
+    while ( not done )
+    {
+      if ( not d.plain_div )
+        integrate( std::true_type {} );
+      if ( not done )
+        integrate( std::false_type {} );
     }
   }
   // aeif_cond_exp neurons are loaded and updated by update_block

@@ -81,6 +81,48 @@ def test_aeif_parameter_sets_in_one_block(change):
     _run(desc, {"targets_per_block": 160}, AEIF_FIELDS, exact=False)
 
 
+@pytest.mark.parametrize("change, quiet", [
+    ({}, [(95, 1), (1, 170)]),  # conductances: denormal from 142 ms (0.2) and 248 ms (0.35) after the last input
+    # w too (1 ms, driven by spikes only), and no spike current; V_m in a network that settles at 0
+    ({"tau_w": 1.0, "a": 0.0}, [(95, 1), (1, 170), (380, 1), (1, 120)]),
+    ({"Delta_T": 0.0, "E_L": 0.0, "V_reset": -10.0, "V_th": 12.0, "V_peak": 20.0, "E_ex": 60.0, "E_in": -20.0, "C_m": 30.0,
+      "tau_w": 1.0, "a": 0.0}, [(95, 1), (1, 170), (380, 1), (1, 120)]),
+])
+def test_aeif_division_by_reciprocals_equals_plain_division(change, quiet):
+    # a neuron without connections whose tau_w rules out the reciprocals makes the whole network
+    # divide plainly: the other neurons' states keep every bit, down to denormal values
+    rng = np.random.default_rng(12)
+    n, T = 450, 40.0
+    prm = dict(nb.AEIF_C4, tau_syn_ex=0.2, tau_syn_in=0.35, **change)
+    lo, hi = prm.get("V_reset", -70.6), prm.get("V_th", -52.0)
+    v0, counts = rng.uniform(lo, hi, n), rng.poisson(2.0, size=(int(T / 0.1), n)).astype(np.uint8)
+    sims = []
+    for tau_w in (144.0, 1e201):
+        desc = dict(n_vp=1, seed=3, pops=[("aeif_cond_exp", n, prm), ("aeif_cond_exp", 1, dict(nb.AEIF_C4, tau_w=tau_w))],
+                    v0={0: v0}, conns=[((0, 0, 360), (0, 0, n), "fixed_indegree", 10, 2.0, 1.5),
+                                       ((0, 360, n), (0, 0, n), "fixed_indegree", 10, -2.0, 1.5)],
+                    drive=[(0, counts, 6.0, 1.5)], T=T)
+        sims.append(nb.build_gpu(desc, layout={"targets_per_block": n + 1}))
+    smallest = 1.0
+    at = 0.0
+    for t in [T] + [float(t) for step, count in quiet for t in [step] * count]:
+        at += t
+        state = []
+        for k, pops, sr in sims:
+            k.Simulate(t)
+            state.append({f: pops[0].get(f) for f in AEIF_FIELDS})
+        for f in AEIF_FIELDS:
+            a, b = state[0][f], state[1][f]
+            bad = np.flatnonzero(a.view(np.uint64) != b.view(np.uint64))
+            assert len(bad) == 0, "%g ms, %s: %d of %d differ, first %r, plain %r" % (at, f, len(bad), n, a[bad[0]], b[bad[0]])
+            if np.any(a != 0.0):
+                smallest = min(smallest, np.min(np.abs(a[a != 0.0])))
+    ev = [sr.get("events") for _, _, sr in sims]
+    assert np.array_equal(ev[0]["senders"], ev[1]["senders"]) and np.array_equal(ev[0]["times"], ev[1]["times"])
+    print("spikes %d, smallest state value %g" % (len(ev[0]["senders"]), smallest), flush=True)
+    assert len(ev[0]["senders"]) > 100 and smallest < 2.0 ** -1022
+
+
 @pytest.mark.parametrize("layout", [{"targets_per_block": 1, "delivery_mode": "global"}, {"targets_per_block": 5},
                                     {"targets_per_block": 64}, {"targets_per_block": 65}, {"targets_per_block": 257},
                                     {"targets_per_block": 512}, {"targets_per_block": 2, "delivery_mode": "global"}],
