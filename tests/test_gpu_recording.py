@@ -137,3 +137,45 @@ def test_spike_recorder_window_against_oracle():
     assert np.array_equal(ev["senders"], g[keep])
     assert np.allclose(ev["times"], s[keep] * 0.1, rtol=0, atol=1e-9)
     assert sr.get("n_events") == keep.sum()
+
+
+def test_collecting_few_spikes_of_many_observed_neurons():
+    # one-step Runs of 300,000 neurons of which 1,000 spike: in the steps with spikes, a recorder
+    # on all neurons costs what one on a single neuron does (a table of the observed neurons made
+    # for each call took 100 us more). Both recorders hold what their neurons emitted.
+    import time
+
+    def build(n_observed):
+        k = nestgpu.Kernel(0)
+        k.SetKernelStatus({"total_num_virtual_procs": 8})
+        quiet = k.Create("iaf_psc_exp", 299000)
+        busy = k.Create("iaf_psc_exp", 1000)
+        busy.set(I_e=np.random.default_rng(2).uniform(1500.0, 3500.0, 1000))
+        sr = k.Create("spike_recorder")
+        k.Connect(quiet + busy if n_observed > 1 else busy[:1], sr)
+        k.Prepare()
+        k.Run(40.0)
+        return k, busy, sr
+
+    sims = [build(300000), build(1)]
+    took, seen = [[], []], sims[0][2].get("n_events")
+    for _ in range(120):
+        t0 = time.perf_counter()
+        sims[0][0].Run(0.1)
+        t1 = time.perf_counter()
+        sims[1][0].Run(0.1)
+        t2 = time.perf_counter()
+        n = sims[0][2].get("n_events")
+        if n > seen:  # a step with spikes (the same in both)
+            took[0].append(t1 - t0)
+            took[1].append(t2 - t1)
+        seen = n
+    took = [sorted(x)[len(x) // 2] for x in took]
+    evs = [sr.get("events") for _, _, sr in sims]
+    first = sims[0][1].global_id[0]
+    assert np.array_equal(evs[0]["times"][evs[0]["senders"] == first], evs[1]["times"])
+    assert np.all(evs[0]["senders"] >= first)
+    print("Run(0.1): all observed %.0f us, one %.0f us, %d and %d events" % (
+        took[0] * 1e6, took[1] * 1e6, len(evs[0]["senders"]), len(evs[1]["senders"])), flush=True)
+    assert len(evs[1]["senders"]) > 2 and len(evs[0]["senders"]) > 4000
+    assert took[0] - took[1] < 40e-6
