@@ -763,6 +763,16 @@ launch_order( const std::vector< Engine* >& engines )
   return order;
 }
 
+// the places of a launch in the caller's order of the instances
+std::vector< int >
+callers_order( const std::vector< int >& order )
+{
+  std::vector< int > at( order.size() );
+  for ( size_t i = 0; i < order.size(); ++i )
+    at[ order[ i ] ] = static_cast< int >( i );
+  return at;
+}
+
 // v in launch order
 template < typename T >
 std::vector< T >
@@ -860,13 +870,13 @@ launch_chunk_direct( const NetDev* h_nets, NetDev* d_nets, int n, int S, bool sp
 }
 
 // After the status read-back: raise device errors, advance every instance's clock and run
-// part, and drain spike logs that are half full.
+// part, and drain spike logs that are half full. The instances' turns are in the caller's order,
+// as is the error that is raised when several fail.
 void
 finish_chunk( const std::vector< Engine* >& engines, const NetDev* h_nets, const unsigned long long* h_status,
-  std::vector< int64_t >& remaining )
+  std::vector< int64_t >& remaining, const std::vector< int >& turns )
 {
-  const int n = static_cast< int >( engines.size() );
-  for ( int i = 0; i < n; ++i )
+  for ( int i : turns )
   {
     Engine& E = *engines[ i ];
     const NetDev& d = h_nets[ i ];
@@ -925,17 +935,18 @@ bool
 Runner::run_chunk( const std::vector< Engine* >& engines, std::vector< int64_t >& remaining )
 {
   if ( engines.size() <= 1 )
-    return run_chunk_ordered( engines, remaining );
+    return run_chunk_ordered( engines, remaining, std::vector< int >( engines.size(), 0 ) );
   const std::vector< int > order = launch_order( engines );
   std::vector< int64_t > left = in_order( remaining, order );
-  const bool more = run_chunk_ordered( in_order( engines, order ), left );
+  const bool more = run_chunk_ordered( in_order( engines, order ), left, callers_order( order ) );
   for ( size_t i = 0; i < order.size(); ++i )
     remaining[ order[ i ] ] = left[ i ];
   return more;
 }
 
 bool
-Runner::run_chunk_ordered( const std::vector< Engine* >& engines, std::vector< int64_t >& remaining )
+Runner::run_chunk_ordered( const std::vector< Engine* >& engines, std::vector< int64_t >& remaining,
+  const std::vector< int >& turns )
 {
   hip_check( hipSetDevice( device_ ), "hipSetDevice" );
   const int n = static_cast< int >( engines.size() );
@@ -988,7 +999,7 @@ Runner::run_chunk_ordered( const std::vector< Engine* >& engines, std::vector< i
   float ms = 0;
   hipEventElapsedTime( &ms, ev_chunk_[ 0 ], ev_chunk_[ 1 ] );
   last_ms_ += ms;
-  finish_chunk( engines, h_nets_, h_status_, remaining );
+  finish_chunk( engines, h_nets_, h_status_, remaining, turns );
   return true;
 }
 
@@ -1040,6 +1051,7 @@ run_noalloc( int device, const std::vector< Engine* >& unordered, const std::vec
 {
   const std::vector< int > order = launch_order( unordered );
   const std::vector< Engine* > engines = in_order( unordered, order );
+  const std::vector< int > turns = callers_order( order );
   const int n = static_cast< int >( engines.size() );
   if ( n > NOALLOC_MAX_NETS )
     throw std::runtime_error( "run without allocation: " + std::to_string( n ) + " instances, at most "
@@ -1081,7 +1093,7 @@ run_noalloc( int device, const std::vector< Engine* >& unordered, const std::vec
     hip_check( hipMemcpyAsync( h_status, d_status, 2 * n * sizeof( unsigned long long ), hipMemcpyDeviceToHost, st ),
       "status D2H" );
     hip_check( hipStreamSynchronize( st ), "hipStreamSynchronize" );
-    finish_chunk( engines, h_nets, h_status, remaining );
+    finish_chunk( engines, h_nets, h_status, remaining, turns );
   }
 }
 

@@ -309,7 +309,8 @@ public:
   int64_t kernel_launches[ N_KINDS ] = { 0, 0 };
 
 private:
-  bool run_chunk_ordered( const std::vector< Engine* >& engines, std::vector< int64_t >& remaining );
+  bool run_chunk_ordered( const std::vector< Engine* >& engines, std::vector< int64_t >& remaining,
+    const std::vector< int >& turns );
   void ensure_capacity( size_t n );
   bool capture( int n_nets, uint32_t total_blocks, int mask, int delivery );  // false: launch directly
   void launch_one( int n, uint32_t total, int mask, int delivery, int s, hipEvent_t* ev );

@@ -109,3 +109,34 @@ def test_batch_mixes_window_and_large_global_instances():
         a, c = _result(b[1][0], b[2][0]), _result(p[1][0], p[2][0])
         assert len(a[0]) > 0
         assert _same(a, c)
+
+
+@pytest.mark.parametrize("noalloc", [False, True])
+def test_the_first_of_several_failing_instances_is_reported(noalloc):
+    # two instances that both fail in the first chunk: the error is that of the first one passed,
+    # whatever the order of their launch
+    def twice():  # a source of stdp synapses that spikes twice in a slice
+        k = nestgpu.Kernel(0)
+        pre, post = k.Create("iaf_psc_exp", 4, {"I_e": 3000.0, "t_ref": 0.5}), k.Create("iaf_psc_exp", 4)
+        k.Connect(pre, post, "one_to_one", {"synapse_model": "stdp_synapse", "weight": 10.0, "delay": 5.0})
+        return k
+
+    def unstable():
+        k = nestgpu.Kernel(0)
+        k.Create("aeif_cond_exp", 50, {"I_e": -1e6})
+        return k
+
+    def quiet():
+        k = nestgpu.Kernel(0)
+        k.Create("iaf_psc_exp", 20)
+        return k
+
+    simulate = nestgpu.batch_simulate_noalloc if noalloc else nestgpu.batch_simulate
+    for build, message in (((quiet, twice, unstable), "twice"), ((quiet, unstable, twice), "NumericalInstability")):
+        ks = [f() for f in build]
+        for k in ks:
+            k.Prepare()
+        with pytest.raises(nestgpu.NESTError) as e:
+            simulate(ks, [50.0] * 3)
+        both = [w for w in ("twice", "NumericalInstability") if w in str(e.value)]
+        assert both == [message], str(e.value)
