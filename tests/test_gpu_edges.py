@@ -148,6 +148,42 @@ def test_many_spikes_per_slice(layout):
     _run(desc, layout, ("V_m",))
 
 
+def _volleys(n, of, T):
+    # every slice (15 steps) the first `of` neurons of each half spike
+    params = {"C_m": 1.0, "tau_m": 20.0, "V_th": 20.0, "V_reset": 10.0, "E_L": 0.0, "t_ref": 1.0}
+    counts = np.zeros((int(round(T / 0.1)), n), np.uint8)
+    for first in (0, n // 2):
+        counts[::15, first:first + of] = 1
+    return dict(n_vp=1, seed=6, pops=[("iaf_psc_delta", n, params)], v0={0: np.random.default_rng(n).uniform(0, 10, n)},
+                conns=[((0, 0, n), (0, 0, n), "fixed_indegree", 20, ("normal", 0.001, 0.1), 1.5)],
+                drive=[(0, counts, 40.0, 1.5)], T=T)
+
+
+@pytest.mark.parametrize("of", [3, 4, 5, 16, 17, 100, 511, 512])
+def test_spike_lists_of_one_length(of):
+    # lists that come with the counts, that one thread copies and that are looked up
+    _run(_volleys(1024, of, 15.0), {"targets_per_block": 512}, ("V_m",))
+
+
+def test_long_spike_lists_cost_what_many_spikes_cost():
+    # 1,000 spikes per slice in two lists, and 1,030 (in three), which are more than a chunk: a thread that
+    # copied a list of 500 entries made the smaller number the slower one (60 %)
+    import time
+
+    sims = [nb.build_gpu(_volleys(n, n // 2, 600.0), layout={"targets_per_block": 512}) for n in (1000, 1030)]
+    took = [[], []]
+    for i in range(10):
+        for (k, _, _), t in zip(sims, took):
+            if i == 0:
+                k.Prepare()
+            at = time.perf_counter()
+            k.Run(60.0)
+            t.append(time.perf_counter() - at)
+    us = [sorted(t[2:])[4] / 40 * 1e6 for t in took]
+    print("us per slice: %.1f (1,000 spikes), %.1f (1,030)" % tuple(us), flush=True)
+    assert us[0] < 1.15 * us[1]
+
+
 @pytest.mark.parametrize("model, fields", [("iaf_psc_exp", ("V_m", "I_syn_ex", "I_syn_in")),
                                            ("iaf_psc_alpha", ("V_m", "I_syn_ex", "I_syn_in")), ("iaf_psc_delta", ("V_m",))])
 @pytest.mark.parametrize("delay, slots", [(7.0, 0), (7.0, 20), (0.1, 0)])
