@@ -740,3 +740,20 @@ def test_iaf_psc_alpha_parameters():
         with pytest.raises(nestgpu.NESTError, match=msg):
             n.set(**bad)
     assert np.all(n.get("C_m") == 250.0)
+
+
+def test_every_model_set_has_its_slice_kernel_object():
+    # the objects follow the list of model sets, also one with a model more
+    import os
+    import re
+    import subprocess
+
+    pkg = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "nest-simulator_amd")
+    for extra in (0, 1):
+        parts = ["1<<M_IAF_PSC_DELTA", "1<<M_IAF_PSC_EXP", "1<<M_AEIF_COND_EXP", "1<<M_IAF_PSC_ALPHA"]
+        parts += ["1<<4"] * extra + ["ALL_MODELS"]
+        out = subprocess.run(["make", "-n", "-B", "-C", pkg] + (["PARTS=" + " ".join(parts)] if extra else []),
+                             check=True, capture_output=True, text=True).stdout
+        assert re.findall(r"'-DNG_PART=([^']*)'", out) == parts
+        link = [x for x in out.splitlines() if "-shared" in x][0]
+        assert re.findall(r"ng_slice_(\d+)\.o", link) == [str(i + 1) for i in range(len(parts))]
