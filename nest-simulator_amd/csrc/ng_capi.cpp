@@ -239,16 +239,13 @@ nestgpu_recorder_events( nestgpu_kernel* h, int64_t recorder_id, int64_t* sender
       h->k->recorder_events( recorder_id, s, st );
       if ( n )
         *n = static_cast< int64_t >( s.size() );
-      if ( senders )
+      const double ms = h->k->timebase().ms_per_tic * h->k->timebase().tics_per_step;
+      const int64_t m = std::min< int64_t >( cap, static_cast< int64_t >( s.size() ) );
+      for ( int64_t i = 0; i < m; ++i )
       {
-        const double ms = h->k->timebase().ms_per_tic * h->k->timebase().tics_per_step;
-        const int64_t m = std::min< int64_t >( cap, static_cast< int64_t >( s.size() ) );
-        for ( int64_t i = 0; i < m; ++i )
-        {
-          senders[ i ] = s[ i ];
-          if ( times )
-            times[ i ] = ms * static_cast< double >( st[ i ] );  // Time::step(stamp).get_ms()
-        }
+        senders[ i ] = s[ i ];
+        if ( times )
+          times[ i ] = ms * static_cast< double >( st[ i ] );  // Time::step(stamp).get_ms()
       }
     } );
 }
@@ -272,19 +269,16 @@ nestgpu_multimeter_events( nestgpu_kernel* h, int64_t multimeter_id, int64_t* se
       const size_t nf = h->k->multimeter_record_from( multimeter_id ).size();
       if ( n )
         *n = static_cast< int64_t >( s.size() );
-      if ( senders )
+      const double ms = h->k->timebase().ms_per_tic * h->k->timebase().tics_per_step;
+      const int64_t m = std::min< int64_t >( cap, static_cast< int64_t >( s.size() ) );
+      for ( int64_t i = 0; i < m; ++i )
       {
-        const double ms = h->k->timebase().ms_per_tic * h->k->timebase().tics_per_step;
-        const int64_t m = std::min< int64_t >( cap, static_cast< int64_t >( s.size() ) );
-        for ( int64_t i = 0; i < m; ++i )
-        {
-          senders[ i ] = s[ i ];
-          if ( times )
-            times[ i ] = ms * static_cast< double >( st[ i ] );
-          if ( values )
-            for ( size_t j = 0; j < nf; ++j )
-              values[ i * nf + j ] = v[ i * nf + j ];
-        }
+        senders[ i ] = s[ i ];
+        if ( times )
+          times[ i ] = ms * static_cast< double >( st[ i ] );
+        if ( values )
+          for ( size_t j = 0; j < nf; ++j )
+            values[ i * nf + j ] = v[ i * nf + j ];
       }
     } );
 }

@@ -1369,34 +1369,18 @@ Kernel::get_values( const std::vector< int64_t >& gids, const std::string& key, 
     const int field = M.state_field( key );
     if ( field >= 0 or key == "refractory_steps" )
     {
-      double v;
-      int32_t rr;
-      if ( live )
+      // fields of a live network are read above
+      const double vals[] = { s.v0, s.v1, s.v2, s.v3, s.v4 };
+      if ( field >= 0 )
+        out[ i ] = vals[ field ] + M.state_offset( p, field );
+      else if ( live )
       {
-        const uint32_t dev = static_cast< uint32_t >( gid_to_dev_[ gids[ i ] ] );
-        if ( field >= 0 )
-        {
-          if ( cache[ field ].empty() )
-            engine_->get_state( field, cache[ field ] );
-          v = cache[ field ][ dev ];
-        }
-        else
-        {
-          if ( rcache.empty() )
-            engine_->get_r( rcache );
-          rr = rcache[ dev ];
-        }
+        if ( rcache.empty() )
+          engine_->get_r( rcache );
+        out[ i ] = rcache[ gid_to_dev_[ gids[ i ] ] ];
       }
       else
-      {
-        const double vals[] = { s.v0, s.v1, s.v2, s.v3, s.v4 };
-        v = field >= 0 ? vals[ field ] : 0;
-        rr = s.r;
-      }
-      if ( field < 0 )
-        out[ i ] = rr;
-      else
-        out[ i ] = v + M.state_offset( p, field );
+        out[ i ] = s.r;
       continue;
     }
     double pv;
