@@ -21,10 +21,10 @@
 //
 // Determinism: NEST adds into one ring-buffer cell in the order (delivery batch, receive
 // order of the spike, position in the connector run). A workgroup takes events in that key
-// order in rounds of R; each round is bucketed by target (LDS counters give every event a
-// place in its target's bucket), every event finds its rank in the bucket ordered by
-// (cell, key), and the first event of each cell's run adds the run in key order. No result
-// depends on thread timing or atomics order.
+// order in rounds of R; each round is bucketed by target, and by slot where a block has few
+// targets (LDS counters give every event a place in its bucket), every event finds its rank in
+// the bucket ordered by (cell, key), and the first event of each cell's run adds the run in key
+// order. No result depends on thread timing or atomics order.
 // Built with -ffp-contract=off: every multiply and add rounds as in the reference.
 
 #include <hip/hip_runtime.h>
@@ -39,8 +39,9 @@ namespace nestgpu
 constexpr int IDX_BITS = 11;  // bucket key = slot-channel << 11 | round index: sorted keys group
                               // a bucket's events by cell, in key order within each cell
 
-// Tile shape per kernel variant. With its ring-buffer window, two window workgroups fit in the
-// 160 KB of LDS of a CU; global delivery runs two or three (global_waves).
+// Tile shape: chunks and rounds are the same in both variants. With its ring-buffer window, two
+// window workgroups fit in the 160 KB of LDS of a CU; global delivery runs two or three
+// (global_waves).
 template < bool WIN >
 struct Tile
 {
@@ -727,7 +728,9 @@ __global__ void __launch_bounds__( Tile< WIN >::BS,
   constexpr int RQ = Tile< WIN >::RQ;
   constexpr int R = Tile< WIN >::R;
   constexpr bool SINGLE = single_model< MASK >() >= 0;
-  constexpr bool EARLY = WIN;  // global delivery's larger rounds leave no registers for it
+  // loads ahead of the delivery: the global kernels held to 80 registers (global_waves) have none
+  // left for them; those at 128 were not measured with them
+  constexpr bool EARLY = WIN;
 
   // ---- which instance and block
   const uint32_t gb = n_nets > 1 ? blockIdx.x : xcd_block( blockIdx.x, gridDim.x );
@@ -1127,7 +1130,7 @@ __global__ void __launch_bounds__( Tile< WIN >::BS,
       for ( uint32_t e0 = 0; e0 < E; e0 += R, cur ^= 1 )
       {
         // stage: thread t holds events e0 + t*RQ .. + RQ - 1 (key order = round index) and
-        // takes an unordered place in its target's bucket
+        // takes an unordered place in its bucket (target and part of the slots)
         uint32_t key[ RQ ], loc[ RQ ], dst[ RQ ], ci[ RQ ], goff[ RQ ];
         double val[ RQ ], cv[ RQ ];
         bool lw[ RQ ];  // the event's cell is in the LDS window
@@ -1188,7 +1191,7 @@ __global__ void __launch_bounds__( Tile< WIN >::BS,
 #pragma unroll
         for ( int q = 0; q < RQ; ++q )
           cv[ q ] = cell_load( rb_rsrc, goff[ q ] );
-        // bucket starts: wave 0 scans the per-target counts, BS / 64 per lane; the others
+        // bucket starts: wave 0 scans the buckets' counts, BS / 64 per lane; the others
         // clear the counters of the next round
         if ( t < 64 )
         {

@@ -60,13 +60,6 @@ constexpr int N_DEVICE_MODELS = 4;
 constexpr int ALL_MODELS = ( 1 << N_DEVICE_MODELS ) - 1;
 static_assert( ALL_MODELS < MASK_STDP, "model bits must stay below the stdp bit" );
 
-// GLOBAL_WAVES: waves per SIMD of a model's global delivery kernel. That kernel serves networks
-// of more than 512 blocks, whose workgroups mostly wait for run table entries and ring cells; at
-// 6 (three workgroups per CU, 80 VGPRs) all blocks of up to 393,000 neurons are resident at once.
-// Measured per slice with rounds of 1,024 events, 4 against 6 waves (rounds of 2,048 at 4 waves
-// before): 300,000 iaf_psc_delta neurons 592 / 390 us (629), 450,000 - / 986 (1,035);
-// iaf_psc_alpha 300,000 - / 251 (385), 450,000 - / 592 (613); iaf_psc_exp, which spills 164
-// registers at 6, 300,000 195 / 174 (208), 450,000 297 / 353 (325).
 // the one model id of a launch mask with a single model bit, else -1
 template < int MASK >
 __device__ constexpr int
@@ -82,7 +75,7 @@ single_model()
 // input in flight; a body unrolled over LB lags was 5 KB of code fetched anew in every launch,
 // 890 cycles per lag against 540 (1,777 iaf_psc_exp, slices of ten steps, 16.5 -> 13.9 us with the
 // drive in waves of its own). Cells in HBM are read LU lags at a time, so that their loads
-// overlap. The words of bits are selected, not indexed: indexed, they lived in scratch memory, 24
+// overlap. The words of bits are selected, not indexed: indexed, they lived in scratch memory, 48
 // bytes per thread written in every launch and read back before the spike lists (20 ms passes of
 // 1,777 iaf_psc_exp 368 -> 349 us, 60 ms of 5,000 iaf_psc_delta 934 -> 859, 200 ms of 100,000
 // iaf_psc_exp 21.4 -> 21.0 ms). The words take registers during the update, so the global delivery
@@ -363,8 +356,9 @@ struct DeviceNode< M_AEIF_COND_EXP >
     // Every iteration is one attempted step of the quad's neuron, preceded by the exchange of
     // a finished neuron for the next one. More than AEIF_MAX_STEPS accepted steps within one
     // time step stop the neuron's lag and raise ERR_AEIF_STEPS, which fails the run (the
-    // oracle stops with the same limit); a rejected attempt shrinks h by a factor of at most
-    // 0.9 * 1.1^(-1/5) < 0.89 and is accepted once t + h rounds to t, so every quad finishes.
+    // oracle stops with the same limit). A rejected attempt shrinks h by a factor of at most
+    // 0.9 * 1.1^(-1/5) < 0.89 and is accepted once t + h rounds to t or, in a lag's first step
+    // (t = 0), once h underflows, after fewer than 6,400 attempts; so every quad finishes.
     // integrate: the loop with divisions by reciprocals (FAST) ends, for its wave, where a neuron's
     // state or an overflow rules them out (aeif_fast_state, aeif_finite), the one with plain
     // divisions after at least one attempt, once it is fit again.
@@ -621,7 +615,13 @@ struct DeviceNode< M_IAF_PSC_ALPHA >
 #define NG_WIDE( ID ) | ( DeviceNode< ( ID ) >::WIDE ? ( 1 << ( ID ) ) : 0 )
 constexpr int WIDE_MODELS = 0 NG_DEVICE_MODELS( NG_WIDE );
 #undef NG_WIDE
-// waves per SIMD of the global delivery kernel of a launch mask
+// Waves per SIMD of the global delivery kernel of a launch mask: GLOBAL_WAVES of its model. That
+// kernel serves networks of more than 512 blocks, whose workgroups mostly wait for run table
+// entries and ring cells; at 6 (three workgroups per CU, 80 VGPRs) all blocks of up to 393,000
+// neurons are resident at once. Measured per slice with rounds of 1,024 events, 4 against 6 waves
+// (rounds of 2,048 at 4 waves before): 300,000 iaf_psc_delta neurons 592 / 390 us (629), 450,000
+// - / 986 (1,035); iaf_psc_alpha 300,000 - / 251 (385), 450,000 - / 592 (613); iaf_psc_exp, which
+// spills 164 registers at 6, 300,000 195 / 174 (208), 450,000 297 / 353 (325).
 template < int MASK >
 __host__ __device__ constexpr int
 global_waves()

@@ -1,6 +1,6 @@
 """Hub targets: thousands of events to one target within one round of delivery.
 
-A round buckets up to 1024 (window) or 2048 (global) events by target and ranks each event in
+A round buckets up to 1024 events by target and ranks each event in
 its bucket by (cell, key); a hub target's bucket can hold the whole round. Three hubs receive
 every spike of 3,000 synchronously driven sources, so each volley brings 3,000 events per hub
 into one cell (equal delays) or a few cells (uniform delays), spread over several rounds. The
