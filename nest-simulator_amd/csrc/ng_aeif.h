@@ -77,9 +77,8 @@ struct AeifLane
 // Below, bits get lost: a conductance of 0.2 ms without input is less than 2^-1016 after 141 ms,
 // where ng_div misses the last bit of 1 to 9 % of the quotients. Overflow gives NaN, which the
 // end of the step shows (aeif_finite).
-// 6,000 neurons in slices of 15 steps take 3 % longer with it (310 -> 321 us); looking at each
-// dividend instead took 6 %, a branch at each division, or a second copy of the step for those
-// that turned out unfit, 9 %.
+// 6,000 neurons in slices of 15 steps take 4 % longer with it (306 -> 318 us); looking at each
+// dividend took 6 %, collecting their range or a branch at each division 9 %.
 __device__ __forceinline__ bool
 aeif_fast_state( const AeifLane& P, double y )
 {
@@ -140,11 +139,12 @@ aeif_rhs( const AeifLane& P, bool refractory, double y, double& I_spike )
   return aeif_dynamics< FAST >( P, refractory, V, I_spike, y );
 }
 
-// One attempted step of size h from component y with derivative k1: the lane's component at
-// its end, the error of the embedded 4th-order solution and the derivative at the end.
+// One attempted step of size h from component y, where the spike current is I_start: the lane's
+// component at its end, the error of the embedded 4th-order solution, and the derivative and the
+// spike current at the end.
 template < bool FAST >
 __device__ __forceinline__ double
-aeif_rkf45_step( const AeifLane& P, bool refr, double y, double h, double k1, double& yerr, double& yp, double& I_spike )
+aeif_step( const AeifLane& P, bool refr, double y, double h, double I_start, double& yerr, double& yp, double& I_end )
 {
   const double b21 = 1.0 / 4.0;
   const double b31 = 3.0 / 32.0, b32 = 9.0 / 32.0;
@@ -156,6 +156,7 @@ aeif_rkf45_step( const AeifLane& P, bool refr, double y, double h, double k1, do
                c5 = -1371249.0 / 7618050.0, c6 = 277020.0 / 7618050.0;
   const double ec1 = 1.0 / 360.0, ec3 = -128.0 / 4275.0, ec4 = -2197.0 / 75240.0, ec5 = 1.0 / 50.0, ec6 = 2.0 / 55.0;
   double I;
+  const double k1 = aeif_dynamics< FAST >( P, refr, aeif_V( P, refr, quad_bcast< 0 >( y ) ), I_start, y );
   const double k2 = aeif_rhs< FAST >( P, refr, y + b21 * h * k1, I );
   const double k3 = aeif_rhs< FAST >( P, refr, y + h * ( b31 * k1 + b32 * k2 ), I );
   const double k4 = aeif_rhs< FAST >( P, refr, y + h * ( b41 * k1 + b42 * k2 + b43 * k3 ), I );
@@ -163,7 +164,7 @@ aeif_rkf45_step( const AeifLane& P, bool refr, double y, double h, double k1, do
   const double k6 = aeif_rhs< FAST >( P, refr, y + h * ( b61 * k1 + b62 * k2 + b63 * k3 + b64 * k4 + b65 * k5 ), I );
   const double y1 = y + h * ( c1 * k1 + c3 * k3 + c4 * k4 + c5 * k5 + c6 * k6 );
   yerr = h * ( ec1 * k1 + ec3 * k3 + ec4 * k4 + ec5 * k5 + ec6 * k6 );
-  yp = aeif_rhs< FAST >( P, refr, y1, I_spike );
+  yp = aeif_rhs< FAST >( P, refr, y1, I_end );
   return y1;
 }
 

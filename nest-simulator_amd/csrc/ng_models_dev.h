@@ -352,173 +352,154 @@ struct DeviceNode< M_AEIF_COND_EXP >
         n = __hip_atomic_fetch_add( next, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP );
       local = at( quad_bcast< 0 >( n ) );
     };
-    bool have = false, done = false;
+    bool have = false;
     // Every iteration is one attempted step of the quad's neuron, preceded by the exchange of
     // a finished neuron for the next one. More than AEIF_MAX_STEPS accepted steps within one
     // time step stop the neuron's lag and raise ERR_AEIF_STEPS, which fails the run (the
     // oracle stops with the same limit). A rejected attempt shrinks h by a factor of at most
     // 0.9 * 1.1^(-1/5) < 0.89 and is accepted once t + h rounds to t or, in a lag's first step
     // (t = 0), once h underflows, after fewer than 6,400 attempts; so every quad finishes.
-    // integrate: the loop with divisions by reciprocals (FAST) ends, for its wave, where a neuron's
-    // state or an overflow rules them out (aeif_fast_state, aeif_finite), the one with plain
-    // divisions after at least one attempt, once it is fit again.
-    auto integrate = [ & ]( auto fast )
+    for ( ;; )
     {
-      constexpr bool FAST = decltype( fast )::value;
-      bool tried = false;
-      for ( ;; )
+      if ( lag >= ph.to )
       {
-        if ( lag >= ph.to )
+        if ( have )
         {
-          if ( have )
-          {
-            vc[ dev ] = y;
-            if ( c == 0 )
-              glob( d.v[ 4 ] )[ dev ] = h;
-            if ( c == 1 )
-              glob( d.r )[ dev ] = r;
-            if ( static_cast< uint32_t >( c ) < nw )
-              spk[ local * nw + c ] = bits;
+          vc[ dev ] = y;
+          if ( c == 0 )
+            glob( d.v[ 4 ] )[ dev ] = h;
+          if ( c == 1 )
+            glob( d.r )[ dev ] = r;
+          if ( static_cast< uint32_t >( c ) < nw )
+            spk[ local * nw + c ] = bits;
+          take();
+        }
+        if ( not SINGLE )
+          while ( local < nb and glob( d.model )[ dev0 + local ] != M_AEIF_COND_EXP )
             take();
-          }
-          if ( not SINGLE )
-            while ( local < nb and glob( d.model )[ dev0 + local ] != M_AEIF_COND_EXP )
-              take();
-          if ( local >= nb )
-          {
-            done = true;
-            return;
-          }
-          have = true;
-          dev = dev0 + local;
-          y = vc[ dev ];
-          h = glob( d.v[ 4 ] )[ dev ];
-          r = glob( d.r )[ dev ];
-          lag = ph.from;
-          in = channel ? C.get( lag, ch, local ) : 0.0;
-          const uint32_t pi = glob( d.pidx )[ dev ];
-          if ( d.mm_int > 0 )
-          {
-            mcol = glob( d.mm_col )[ dev ];
-            next_sample = mcol != NONE ? first_sample_lag( d, ph.origin, ph.from, ph.to ) : ph.to;
-          }
-          if ( pi != pset )
-          {
-            pset = pi;
-            gref< const ParamSet > ps = glob( d.psets )[ pi ];
-            A.V_peak = ps.p[ 0 ];
-            A.V_reset = ps.p[ 1 ];
-            A.Delta_T = ps.p[ 7 ];
-            A.V_th = ps.p[ 11 ];
-            A.I_e = ps.p[ 14 ];
-            A.tol = ps.p[ 15 ];
-            A.gD = ps.p[ 2 ] * ps.p[ 7 ];
-            A.E = ps.p[ c == 1 ? 4 : c == 2 ? 5 : 6 ];
-            A.m = c == 0 ? -ps.p[ 2 ] : ps.p[ 9 ];
-            A.zero_fits = channel or ( c == 3 and ps.p[ 9 ] == 0.0 );
-            A.den = ps.p[ c == 0 ? 3 : c == 1 ? 12 : c == 2 ? 13 : 8 ];
-            A.r_den = ng_recip( A.den );
-            A.r_Delta_T = ng_recip( A.Delta_T );
-            b_adapt = ps.p[ 10 ];
-            V_peak_eff = ps.p[ 16 ];
-            hstep = ps.p[ 17 ];
-            refractory_counts = ps.refractory_counts;
-            I_reset = aeif_spike_current< FAST >( A, aeif_V( A, false, A.V_reset ) );
-          }
-          tt = 0.0;
-          guard = 0;
-          bits = 0;
-          I_spk = aeif_spike_current< FAST >( A, aeif_V( A, false, quad_bcast< 0 >( y ) ) );
-        }
-        // the derivative at the step's start: its spike current is the one the last step ended
-        // with, or that of the reset potential (inputs change the conductances only)
-        const bool refr = r > 0;
-        const double dt = hstep - tt;
-        const bool final_step = h > dt;
-        const double h_old = final_step ? dt : h;
-        const double k1 = aeif_dynamics< FAST >( A, refr, aeif_V( A, refr, quad_bcast< 0 >( y ) ), I_spk, y );
-        // looked at behind k1, as the end of the step behind its control, which hides the latency
-        const bool unfit = __any( not aeif_fast_state( A, y ) );
-        if ( FAST ? unfit : tried and not unfit and not d.plain_div )
-          return;
-        tried = true;
-        double yerr, yp, I_end;
-        const double y1 = aeif_rkf45_step< FAST >( A, refr, y, h_old, k1, yerr, yp, I_end );
-        const double tn = final_step ? hstep : tt + h_old;
-        double h_new = h_old;
-        const int st = aeif_yp_hadjust( A.tol, yerr, yp, &h_new );
-        if ( FAST and __any( not aeif_finite( y1, yp ) ) )
-          return;
-        h = h_new;
-        if ( st < 0 )
+        if ( local >= nb )
+          break;
+        have = true;
+        dev = dev0 + local;
+        y = vc[ dev ];
+        h = glob( d.v[ 4 ] )[ dev ];
+        r = glob( d.r )[ dev ];
+        lag = ph.from;
+        in = channel ? C.get( lag, ch, local ) : 0.0;
+        const uint32_t pi = glob( d.pidx )[ dev ];
+        if ( d.mm_int > 0 )
         {
-          if ( fabs( h_new ) < fabs( h_old ) and tn + h_new != tn )
-            continue;  // again from the same state
-          h = h_old;
+          mcol = glob( d.mm_col )[ dev ];
+          next_sample = mcol != NONE ? first_sample_lag( d, ph.origin, ph.from, ph.to ) : ph.to;
         }
-        y = y1;
-        I_spk = I_end;
-        tt = tn;
-        ++guard;
-        const double V = quad_bcast< 0 >( y ), w = quad_bcast< 3 >( y );
-        if ( V < -1e3 or w < -1e6 or w > 1e6 )
+        if ( pi != pset )
         {
-          if ( c == 0 )
-            g_or( &d.counters[ 0 ], ERR_AEIF_INSTABILITY );
-          tt = hstep;
+          pset = pi;
+          gref< const ParamSet > ps = glob( d.psets )[ pi ];
+          A.V_peak = ps.p[ 0 ];
+          A.V_reset = ps.p[ 1 ];
+          A.Delta_T = ps.p[ 7 ];
+          A.V_th = ps.p[ 11 ];
+          A.I_e = ps.p[ 14 ];
+          A.tol = ps.p[ 15 ];
+          A.gD = ps.p[ 2 ] * ps.p[ 7 ];
+          A.E = ps.p[ c == 1 ? 4 : c == 2 ? 5 : 6 ];
+          A.m = c == 0 ? -ps.p[ 2 ] : ps.p[ 9 ];
+          A.zero_fits = channel or ( c == 3 and ps.p[ 9 ] == 0.0 );
+          A.den = ps.p[ c == 0 ? 3 : c == 1 ? 12 : c == 2 ? 13 : 8 ];
+          A.r_den = ng_recip( A.den );
+          A.r_Delta_T = ng_recip( A.Delta_T );
+          b_adapt = ps.p[ 10 ];
+          V_peak_eff = ps.p[ 16 ];
+          hstep = ps.p[ 17 ];
+          refractory_counts = ps.refractory_counts;
+          I_reset = aeif_spike_current< false >( A, aeif_V( A, false, A.V_reset ) );
         }
-        else if ( r > 0 )
+        tt = 0.0;
+        guard = 0;
+        bits = 0;
+        I_spk = aeif_spike_current< false >( A, aeif_V( A, false, quad_bcast< 0 >( y ) ) );
+      }
+      const bool refr = r > 0;
+      const double dt = hstep - tt;
+      const bool final_step = h > dt;
+      const double h_old = final_step ? dt : h;
+      // the spike current at the step's start is the one the last step ended with, or that of the
+      // reset potential (inputs change the conductances only)
+      double y1, yerr, yp, I_end;
+      bool plain = __any( d.plain_div or not aeif_fast_state( A, y ) );
+      if ( not plain )
+      {
+        y1 = aeif_step< true >( A, refr, y, h_old, I_spk, yerr, yp, I_end );
+        plain = __any( not aeif_finite( y1, yp ) );
+      }
+      if ( plain )
+        y1 = aeif_step< false >( A, refr, y, h_old, I_spk, yerr, yp, I_end );
+      const double tn = final_step ? hstep : tt + h_old;
+      double h_new = h_old;
+      const int st = aeif_yp_hadjust( A.tol, yerr, yp, &h_new );
+      h = h_new;
+      if ( st < 0 )
+      {
+        if ( fabs( h_new ) < fabs( h_old ) and tn + h_new != tn )
+          continue;  // again from the same state
+        h = h_old;
+      }
+      y = y1;
+      I_spk = I_end;
+      tt = tn;
+      ++guard;
+      const double V = quad_bcast< 0 >( y ), w = quad_bcast< 3 >( y );
+      if ( V < -1e3 or w < -1e6 or w > 1e6 )
+      {
+        if ( c == 0 )
+          g_or( &d.counters[ 0 ], ERR_AEIF_INSTABILITY );
+        tt = hstep;
+      }
+      else if ( r > 0 )
+      {
+        y = c == 0 ? A.V_reset : y;
+        I_spk = I_reset;
+      }
+      else if ( V >= V_peak_eff )
+      {
+        y = c == 0 ? A.V_reset : c == 3 ? y + b_adapt : y;
+        I_spk = I_reset;
+        r = refractory_counts > 0 ? refractory_counts + 1 : 0;
+        if ( ( lag >> 6 ) == c )
         {
-          y = c == 0 ? A.V_reset : y;
-          I_spk = I_reset;
-        }
-        else if ( V >= V_peak_eff )
-        {
-          y = c == 0 ? A.V_reset : c == 3 ? y + b_adapt : y;
-          I_spk = I_reset;
-          r = refractory_counts > 0 ? refractory_counts + 1 : 0;
-          if ( ( lag >> 6 ) == c )
-          {
-            const unsigned long long bit = 1ull << ( lag & 63 );
-            if ( bits & bit )
-              g_or( &d.counters[ 0 ], ERR_AEIF_DOUBLE_SPIKE );
-            bits |= bit;
-          }
-        }
-        if ( tt < hstep and guard >= AEIF_MAX_STEPS )
-        {
-          if ( c == 0 )
-            g_or( &d.counters[ 0 ], ERR_AEIF_STEPS );
-          tt = hstep;
-        }
-        if ( not( tt < hstep ) )
-        {
-          if ( r > 0 )
-            --r;
-          if ( channel )
-          {
-            y += in;
-            C.put( lag, ch, local, 0.0 );
-          }
-          if ( lag == next_sample )
-          {
-            store_sample_field( d, mcol, ph.origin + lag + 1, c, y );
-            next_sample += d.mm_int;
-          }
-          ++lag;
-          tt = 0.0;
-          guard = 0;
-          if ( channel and lag < ph.to )
-            in = C.get( lag, ch, local );  // arrives while the lag is integrated
+          const unsigned long long bit = 1ull << ( lag & 63 );
+          if ( bits & bit )
+            g_or( &d.counters[ 0 ], ERR_AEIF_DOUBLE_SPIKE );
+          bits |= bit;
         }
       }
-    };
-    while ( not done )
-    {
-      if ( not d.plain_div )
-        integrate( std::true_type {} );
-      if ( not done )
-        integrate( std::false_type {} );
+      if ( tt < hstep and guard >= AEIF_MAX_STEPS )
+      {
+        if ( c == 0 )
+          g_or( &d.counters[ 0 ], ERR_AEIF_STEPS );
+        tt = hstep;
+      }
+      if ( not( tt < hstep ) )
+      {
+        if ( r > 0 )
+          --r;
+        if ( channel )
+        {
+          y += in;
+          C.put( lag, ch, local, 0.0 );
+        }
+        if ( lag == next_sample )
+        {
+          store_sample_field( d, mcol, ph.origin + lag + 1, c, y );
+          next_sample += d.mm_int;
+        }
+        ++lag;
+        tt = 0.0;
+        guard = 0;
+        if ( channel and lag < ph.to )
+          in = C.get( lag, ch, local );  // arrives while the lag is integrated
+      }
     }
   }
   // aeif_cond_exp neurons are loaded and updated by update_block
